@@ -90,29 +90,31 @@ typedef struct {
    * increment conservatively (pp_chem_flatten / pp_chem_unflatten). */
   int clean_init_massfrac;
   /* Batched forms: persistent waves per compute unit (0: every wave that fits,
-   * 8 at the kernels' 2 waves per SIMD); a tuning parameter
-   * (python -m pelephysics_amd.autotune). */
+   * 8 at the kernels' 2 waves per SIMD) of the kernels the caller names
+   * (batched_cells_per_wave) and of the QSS mechanisms' one-cell-per-lane
+   * kernels; a tuning parameter (python -m pelephysics_amd.autotune). */
   int batched_waves_per_cu;
-  /* Batched forms: a wave factors the Newton matrices of its waiting lanes
-   * together once batched_lu_batch lanes (1..64) wait or a request has waited
-   * batched_lu_wait trips (0: 64 and 32); results do not depend on them. */
+  /* Batched forms: a wave factors the Newton matrices of its waiting cells
+   * together once batched_lu_batch cells (1..64) wait or a request has waited
+   * batched_lu_wait trips (0: the kernel's default; read where
+   * batched_waves_per_cu is); results do not depend on them. */
   int batched_lu_batch, batched_lu_wait;
-  /* Batched forms, box call: 0 (default) runs box -> flat, the 1-D kernel,
-   * flat -> box (same per-cell operations, faster kernel build); 1 runs the
-   * box kernel directly. */
+  /* Batched forms, box call: 0 or 1.  Both run box -> flat, the 1-D kernel,
+   * flat -> box; results do not depend on it. */
   int batched_box_direct;
-  /* The kernel build a launch uses.  Batched forms: held to 2 waves per SIMD
-   * (0 or 2, the default) or to 1 (more registers per lane, fewer spills;
-   * 1-D kernel only, so not with batched_box_direct = 1).  The plain adaptive
-   * BDF (PP_CHEM_BDF_ADAPTIVE): 0 (the compiler's choice), 2 or 4.  The
-   * parity integrators: 0. */
+  /* The kernel build a launch uses.  Batched forms: the one-cell-per-lane
+   * kernels of the QSS mechanisms held to 2 waves per SIMD (0 or 2, the
+   * default) or to 1 (more registers per lane, fewer spills; not with
+   * batched_box_direct = 1); the other mechanisms accept and do not read it.
+   * The plain adaptive BDF (PP_CHEM_BDF_ADAPTIVE): 0 (the compiler's choice),
+   * 2 or 4.  The parity integrators: 0. */
   int batched_waves_per_simd;
-  /* Batched forms, cells per 64-lane wavefront: 0 (default) integrates one
-   * cell per lane (64 per wave); 8, 4, 2 or 1 give each cell a group of 8, 16,
-   * 32 or 64 lanes that share its equations, reactions and LU rows, so its
-   * state stays in registers (table-driven mechanism kernels only; the values
-   * a mechanism supports depend on its size; box calls go through flat
-   * state). */
+  /* Batched forms, cells per 64-lane wavefront: 8, 4, 2 or 1 give each cell a
+   * group of 8, 16, 32 or 64 lanes that share its equations, reactions and
+   * Newton-matrix rows, so its state stays in registers (table-driven
+   * mechanism kernels only; the values a mechanism supports depend on its
+   * size); 0 (default): the library chooses by the mechanism's size and the
+   * number of cells (QSS mechanisms: one cell per lane). */
   int batched_cells_per_wave;
   /* PP_CHEM_BDF_ADAPTIVE and PP_CHEM_CVODE (0 elsewhere): order cap 1..5
    * (cvode.max_order; 0: 5), Newton iterations per step attempt

@@ -51,44 +51,6 @@ struct IO1D {
   }
 };
 
-// Cell input/output of the box (Array4) form, with the initial and final
-// temperature inversions of ReactorBDF.cpp:376-389,461-478.
-struct IOBox {
-  BoxArgs b;
-  PPC_DI void ijk(int c, int& i, int& j, int& k) const {
-    i = b.lo[0] + c % b.len[0];
-    j = b.lo[1] + (c / b.len[0]) % b.len[1];
-    k = b.lo[2] + c / (b.len[0] * b.len[1]);
-  }
-  template <class M>
-  PPC_DI void load(int c, double* y0, double* src, double& rhoe, double& rhoesrc, int reactor_type) const {
-    int i, j, k;
-    ijk(c, i, j, k);
-    double Y[M::NS], rinv;
-    for (int s = 0; s < M::NS; ++s) {
-      y0[s] = b.rY(i, j, k, s);
-      src[s] = b.rYsrc(i, j, k, s);
-    }
-    const double rho = rho_and_Y<M>(y0, Y, rinv);
-    rhoe = b.rE(i, j, k, 0);
-    rhoesrc = b.rEsrc(i, j, k, 0);
-    y0[M::NS] = T_from_energy_rt<M>(reactor_type, rhoe / rho, Y, b.T(i, j, k, 0));
-  }
-  template <class M>
-  PPC_DI void store(int c, const double* yv, double rhoe, double rhoesrc, double dt, int nsteps,
-                    int reactor_type) const {
-    int i, j, k;
-    ijk(c, i, j, k);
-    double Y[M::NS], rinv;
-    const double rho = rho_and_Y<M>(yv, Y, rinv);
-    for (int s = 0; s < M::NS; ++s) b.rY(i, j, k, s) = yv[s];
-    const double rE_new = rhoe + dt * rhoesrc;
-    b.rE(i, j, k, 0) = rE_new;
-    b.T(i, j, k, 0) = T_from_energy_rt<M>(reactor_type, rE_new / rho, Y, yv[M::NS]);
-    if (b.FC.p) b.FC(i, j, k, 0) = (double)nsteps;
-  }
-};
-
 enum : int { PH_F0 = 0, PH_F1 = 1, PH_NEWTON = 2 };
 
 // OCC: waves per SIMD the register allocation is held to.  At 2 (256 VGPRs)

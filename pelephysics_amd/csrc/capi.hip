@@ -167,8 +167,12 @@ struct pp_chem {
   pp_chem_config cfg;
   std::string mech_name;
   const MechLauncher* L = nullptr;
+  // the launcher with this mechanism's group kernels (group_bdf.h): L itself or
+  // its table-driven sibling; null when there are none
+  const MechLauncher* GL = nullptr;
   ppc::ReactParamsDev P{};
   int device = 0;
+  int ncu = 0;  // compute units
   // per-cell counters (device), grown on demand
   int cap = 0;
   int* d_cnt = nullptr;  // 6 * cap ints
@@ -348,28 +352,73 @@ hipError_t scratch_address(int device, unsigned char** out) {
   return hipSuccess;
 }
 
-// Per-lane workspace of mechanisms too large for private memory: one row of
-// doubles per lane and matrix element, for at most the resident waves per CU
-// of the kernel build (4 SIMDs x 2 waves for the 2-wave batched build, x 1
-// for the 1-wave batched build and the one-lane-per-cell kernels of the other
-// integrators) and at most cfg.workspace_bytes (default kWsMaxBytes).
 constexpr long long kWsMaxBytes = 32LL << 30;
 
+// Cells per wave of the group kernels where the caller leaves the choice
+// (batched_cells_per_wave = 0): a lane per equation, rounded up to 8, 16, 32 or
+// 64 lanes per cell, while that fills the chip no more than kGroupRounds times
+// over; half as many lanes, two equations in each, above it.  A wide group ends
+// a cell's trip sooner, which is what a call of few cells waits for; a narrow
+// one has less of its lanes idle in the exchanges and reductions, which is what
+// a call of many cells waits for.  Measured (one call of 1e-5 s at rtol 1e-10,
+// cells in index order, 32 / 16 lanes): drm19 2898 cells 5.9 / 8.2 ms, 262144
+// cells 95 / 79 ms.  Above 32 equations the inverse's two rows per lane leave
+// one wave per SIMD (dodecane_lu, 10000 cells: 17.5 ms at 64 lanes, 27.3 at 32).
+constexpr long long kGroupRounds = 8;
+
+int auto_cells_per_wave(const pp_chem* h, long long ncells) {
+  const int n = h->L->ns + 1;
+  int lanes = 64;
+  while (lanes > 8 && lanes / 2 >= n) lanes /= 2;
+  int cpw = 64 / lanes;
+  const long long waves = 8LL * std::max(h->ncu, 1);
+  if (n <= 32 && h->GL->group_ws_rows(2 * cpw) > 0 && ncells >= kGroupRounds * waves * 2 * cpw) cpw *= 2;
+  return cpw;
+}
+
+// Cells per wave of this call's group kernel; 0: one lane per cell.
+int cells_per_wave(const pp_chem* h, long long ncells) {
+  if (!is_batched(h->cfg.mode) || !h->GL) return 0;
+  return h->cfg.batched_cells_per_wave != 0 ? h->cfg.batched_cells_per_wave : auto_cells_per_wave(h, ncells);
+}
+
+// 64-lane blocks of workspace a call of ncells cells can use, and its rows per
+// lane: the Jacobians of the group kernels (group_bdf.h), per wave, and
+// the per-lane matrices of mechanisms too large for private memory
+// (lane_ws.h), for at most the resident waves per CU of the kernel build (4
+// SIMDs x 2 waves, x 1 for the 1-wave build and the one-lane-per-cell kernels
+// of the other integrators) and (by the caller) at most the bytes there are.
+long long workspace_blocks(const pp_chem* h, long long ncells, int cpw, long long& rows) {
+  rows = cpw ? h->GL->group_ws_rows(cpw) : h->L->ws_rows(kmode(h->cfg.mode));
+  if (rows == 0 || ncells == 0) return 0;
+  const long long per_cu =
+      (cpw || (is_batched(h->cfg.mode) && h->cfg.batched_waves_per_simd != 1)) ? 8 : 4;
+  const long long lanes_per_cell = cpw ? 64 / cpw : 1;
+  long long blocks = std::min<long long>((ncells * lanes_per_cell + 63) / 64, per_cu * std::max(h->ncu, 1));
+  if (h->max_blocks > 0) blocks = std::min<long long>(blocks, h->max_blocks);
+  return blocks;
+}
+
+// What the group kernel of cpw cells per wave takes from the configuration: the
+// LU service parameters only where the caller chose the kernel (they are
+// counted in lanes of the one-cell-per-lane kernels otherwise).
+void group_params(const pp_chem* h, int cpw, ppc::AdaptParamsDev& a) {
+  a.group = cpw;
+  const bool own = h->cfg.batched_cells_per_wave != 0;
+  if (cpw) {
+    a.lu_batch = own ? h->cfg.batched_lu_batch : 0;
+    a.lu_wait = own ? h->cfg.batched_lu_wait : 0;
+  }
+}
+
 int prepare_workspace(pp_chem* h, int ncells) {
+  const int cpw = cells_per_wave(h, ncells);
+  group_params(h, cpw, h->P.adapt);
   h->P.ws = nullptr;
   h->P.ws_lanes = 0;
-  const bool group = is_batched(h->cfg.mode) && h->cfg.batched_cells_per_wave != 0;
-  const long long rows = group ? h->L->group_ws_rows(h->cfg.batched_cells_per_wave) : h->L->ws_rows(kmode(h->cfg.mode));
-  if (rows == 0 || ncells == 0) return 0;
-  int ncu = 0;
-  HIPCHK(h, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, h->device));
-  const long long per_cu =
-      (is_batched(h->cfg.mode) && (group || h->cfg.batched_waves_per_simd != 1)) ? 8 : 4;
-  // blocks of 64 lanes that can hold a cell each: one cell per lane, or per
-  // group of 64 / batched_cells_per_wave lanes
-  const long long lanes_per_cell = group ? 64 / h->cfg.batched_cells_per_wave : 1;
-  long long blocks = std::min<long long>(((long long)ncells * lanes_per_cell + 63) / 64, per_cu * std::max(ncu, 1));
-  if (h->max_blocks > 0) blocks = std::min<long long>(blocks, h->max_blocks);
+  long long rows = 0;
+  long long blocks = workspace_blocks(h, ncells, cpw, rows);
+  if (blocks == 0) return 0;
   const long long cap = h->cfg.workspace_bytes > 0 ? h->cfg.workspace_bytes : kWsMaxBytes;
   const long long lane_bytes = 64 * rows * (long long)sizeof(double);  // one 64-lane block
   if (lane_bytes > cap) return fail(h, PP_CHEM_EINVAL, "workspace_bytes below one 64-cell block");
@@ -416,7 +465,7 @@ hipError_t enqueue_1d(pp_chem* h, double* y, double* ysrc, double* rX, double* r
   hipError_t e;
   if (is_batched(h->cfg.mode)) {
     const ppc::QueueArgs q = prepare_queue(h, ncells, key, s);
-    e = h->L->batched_1d(h->cfg.mode, h->P, y, ysrc, rX, rXsrc, dt, q, counters(h), s);
+    e = (h->GL ? h->GL : h->L)->batched_1d(h->cfg.mode, h->P, y, ysrc, rX, rXsrc, dt, q, counters(h), s);
   } else {
     e = h->L->react_1d(kmode(h->cfg.mode), h->P, y, ysrc, rX, rXsrc, dt, ncells, counters(h), h->cfg.block_size, s);
   }
@@ -653,12 +702,18 @@ int pp_chem_create(const pp_chem_config* cfg, pp_chem** out) {
     h->P.erk = {h->d_erk, s, T->q, T->p, T->fsal, cfg->erk_controller};
     h->cfg.erk_method = T->code;
   }
-  hipError_t e = hipGetDevice(&h->device);
-  if (e == hipSuccess && cfg->batched_waves_per_cu > 0) {
-    int ncu = 0;
-    e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, h->device);
-    h->max_blocks = cfg->batched_waves_per_cu * ncu;  // one 64-lane wave per block
+  if (!manifold) {
+    const MechLauncher* T = find_mech((h->mech_name + "_table").c_str());
+    if (!T) T = L;
+    for (int cpw = 1; cpw <= 8; cpw *= 2)
+      if (T->group_ws_rows(cpw) > 0) h->GL = T;
   }
+  hipError_t e = hipGetDevice(&h->device);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&h->ncu, hipDeviceAttributeMultiprocessorCount, h->device);
+  // persistent-grid bound of the kernels it was chosen for: the
+  // one-lane-per-cell ones, or the group size the caller names
+  if (cfg->batched_waves_per_cu > 0 && (!h->GL || cfg->batched_cells_per_wave != 0))
+    h->max_blocks = cfg->batched_waves_per_cu * h->ncu;  // 64-lane waves
   if (e == hipSuccess) e = hipMalloc(&h->d_red, sizeof(unsigned long long) * 9);
   if (e == hipSuccess) e = hipMalloc(&h->d_queue, sizeof(int) * (1 + 2 * NBINS));
   if (e == hipSuccess) e = hipMalloc(&h->d_fail, sizeof(int));
@@ -821,9 +876,9 @@ int pp_chem_num_species(const pp_chem* h) { return h ? h->L->ns : PP_CHEM_EINVAL
 int pp_chem_num_reactions(const pp_chem* h) { return h ? h->L->nr : PP_CHEM_EINVAL; }
 long long pp_chem_workspace_rows(const pp_chem* h) {
   if (!h) return PP_CHEM_EINVAL;
-  if (is_batched(h->cfg.mode) && h->cfg.batched_cells_per_wave != 0)
-    return h->L->group_ws_rows(h->cfg.batched_cells_per_wave);
-  return h->L->ws_rows(kmode(h->cfg.mode));
+  // group kernels whose cells per wave depend on the call: of a large call
+  const int cpw = cells_per_wave(h, 1LL << 40);
+  return cpw ? h->GL->group_ws_rows(cpw) : h->L->ws_rows(kmode(h->cfg.mode));
 }
 
 int pp_chem_adjoint_1d(pp_chem* h, double* y, const double* rX, int ncells, int nmacro, double dt,
@@ -885,11 +940,11 @@ int pp_chem_react_box(pp_chem* h, const int lo[3], const int hi[3], const pp_arr
   HIPCHK(h, hipEventRecord(h->ev0, s));
   if (ncells > 0) {
     hipError_t e;
-    if (is_batched(h->cfg.mode) && !h->cfg.batched_box_direct) {
-      // flat state, the 1-D kernel, back to the box: the same operations per
-      // cell as the box kernel (T from e / rho with the box T as guess;
-      // rE + dt rEsrc; T from the new energy with the integrated T as guess;
-      // FC = steps), and the 1-D kernel is the faster build of the two
+    if (is_batched(h->cfg.mode)) {
+      // flat state, the 1-D kernel, back to the box: the operations of
+      // ReactorBDF.cpp:376-389,461-478 (T from e / rho with the box T as
+      // guess; rE + dt rEsrc; T from the new energy with the integrated T as
+      // guess; FC = steps)
       const int ns = h->L->ns;
       const size_t nc = (size_t)ncells, need = nc * (size_t)(2 * ns + 3);
       if (need > h->stage_cap) {
@@ -910,16 +965,14 @@ int pp_chem_react_box(pp_chem* h, const int lo[3], const int hi[3], const pp_arr
       e = h->L->flatten(fa, 0, s);
       if (e == hipSuccess) {
         const ppc::QueueArgs q = prepare_queue(h, ncells, rY->p, s);
-        e = h->L->batched_1d(h->cfg.mode, h->P, fa.y, fa.ysrc, fa.e, fa.esrc, *dt_react, q, counters(h), s);
+        e = (h->GL ? h->GL : h->L)
+                ->batched_1d(h->cfg.mode, h->P, fa.y, fa.ysrc, fa.e, fa.esrc, *dt_react, q, counters(h), s);
       }
       if (e == hipSuccess) {
         fa.dt = 0.0;  // the 1-D kernel has already advanced e by dt * rEsrc
         fa.fc32 = counters(h).nsteps;
         e = h->L->flatten(fa, 1, s);
       }
-    } else if (is_batched(h->cfg.mode)) {
-      const ppc::QueueArgs q = prepare_queue(h, ncells, rY->p, s);
-      e = h->L->batched_box(h->cfg.mode, h->P, b, *dt_react, q, counters(h), s);
     } else {
       e = h->L->react_box(kmode(h->cfg.mode), h->P, b, *dt_react, ncells, counters(h), h->cfg.block_size, s);
     }
@@ -1003,16 +1056,11 @@ int pp_chem_react_1d_noalloc(pp_chem* h, double* y, double* ysrc, double* rX, do
   ppc::ReactParamsDev P = h->P;
   P.ws = nullptr;
   P.ws_lanes = 0;
-  const bool group = is_batched(h->cfg.mode) && h->cfg.batched_cells_per_wave != 0;
-  const long long rows = group ? h->L->group_ws_rows(h->cfg.batched_cells_per_wave) : h->L->ws_rows(kmode(h->cfg.mode));
-  if (rows > 0 && ncells > 0) {
-    int ncu = 0;
-    HIPCHK(h, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, h->device));
-    const long long per_cu =
-        (is_batched(h->cfg.mode) && (group || h->cfg.batched_waves_per_simd != 1)) ? 8 : 4;
-    const long long lanes_per_cell = group ? 64 / h->cfg.batched_cells_per_wave : 1;
-    long long blocks = std::min<long long>(((long long)ncells * lanes_per_cell + 63) / 64, per_cu * std::max(ncu, 1));
-    if (h->max_blocks > 0) blocks = std::min<long long>(blocks, h->max_blocks);
+  const int cpw = cells_per_wave(h, ncells);
+  group_params(h, cpw, P.adapt);
+  long long rows = 0;
+  long long blocks = workspace_blocks(h, ncells, cpw, rows);
+  if (blocks > 0) {
     blocks = std::min<long long>(blocks, (long long)(ws_bytes / (64 * rows * sizeof(double))));
     if (blocks < 1) return fail(h, PP_CHEM_EINVAL, "the device scratch holds no 64-lane block of this workspace");
     P.ws = reinterpret_cast<double*>(ws);
@@ -1027,7 +1075,7 @@ int pp_chem_react_1d_noalloc(pp_chem* h, double* y, double* ysrc, double* rX, do
     if (is_batched(h->cfg.mode)) {
       hipLaunchKernelGGL(zero_ints, dim3(1), dim3(64), 0, s, counter, 1);
       const ppc::QueueArgs q{nullptr, counter, ncells, h->max_blocks};  // cells in index order
-      e = h->L->batched_1d(h->cfg.mode, P, y, ysrc, rX, rXsrc, *dt_react, q, st, s);
+      e = (h->GL ? h->GL : h->L)->batched_1d(h->cfg.mode, P, y, ysrc, rX, rXsrc, *dt_react, q, st, s);
     } else {
       e = h->L->react_1d(kmode(h->cfg.mode), P, y, ysrc, rX, rXsrc, *dt_react, ncells, st, h->cfg.block_size, s);
     }

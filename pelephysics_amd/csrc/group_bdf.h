@@ -1,40 +1,47 @@
 // Batched adaptive BDF with a group of G lanes per cell (64 / G cells per
 // wavefront, G = 8, 16, 32 or 64).
 //
-// The lane-per-cell batched kernel (batched.h) keeps a whole cell's
-// integrator state in one lane: ~12 KB for drm19, which the register file
-// cannot hold, so it lives in private (scratch) memory and every access waits
-// on the memory system.  Here the equations of a cell are spread over the G
-// lanes of its group, so the state fits the registers:
-//
 // * lane g of a group holds equations i = e*G + g for slots e < EPL =
 //   ceil(NEQ / G): its entries of the BDF difference array, the iterate, the
-//   error weights and rows i of the Newton-matrix LU factors;
+//   error weights and rows i of the inverted Newton matrix, all in registers;
+// * the mechanism's packed tables (tab/<name>.h, struct Packed) are copied to
+//   LDS once per block; the four waves of a block share them and never wait
+//   for each other afterwards;
 // * right-hand side: each lane evaluates the NASA7 polynomials and
 //   exponentials of its species, concentrations and exponentials go to a small
-//   per-group LDS area, reactions j = r*G + g are spread over the lanes and
-//   write their net rates of progress to LDS, and each lane sums its species'
-//   production rates over the compressed species -> reaction table; mixture
-//   sums (density, energy, the temperature Newton iteration) are group
+//   per-group LDS area, reactions j = g, g + G, ... are spread over the lanes
+//   and write their net rates of progress to LDS, the chunks of 8 terms that
+//   the species' stoichiometric rows are cut into are spread over the lanes
+//   again, and each lane adds up its species' chunks; mixture sums are group
 //   reductions;
-// * Jacobian (rare: about one per cell and call): the same reaction split,
-//   accumulated with FP64 atomics into a per-group matrix in the device
-//   workspace, then each lane takes its rows (molecular-weight scaling of
-//   ReactorBDF.cpp:67-82) and keeps them in the workspace in LU_T for the
-//   Newton-matrix refreshes;
+// * Jacobian (rare: about one per cell and call): all 64 lanes of the wave
+//   work on one group's cell at a time, accumulating with FP64 atomics into an
+//   n x n area (LDS when it fits, else the device workspace), then store the
+//   group's rows (molecular-weight scaling of ReactorBDF.cpp:67-82) in LU_T in
+//   the workspace for the Newton-matrix refreshes;
 // * Newton matrix: inverted in LU_T by row-per-lane Gauss-Jordan exchange
-//   steps with partial pivoting (the pivot a group arg-max, the pivot row
-//   through LDS, rows never move), so that each Newton iteration's solve is
-//   one dot product per row: no sequential triangular sweeps.
+//   steps with partial pivoting (the pivot row through LDS, rows never move,
+//   the columns rotate through the registers so that the step loop is not
+//   unrolled), so that each Newton iteration's solve is one dot product per
+//   row: no sequential triangular sweeps.
+//
+// What bounds it: the latency of a trip (one right-hand side and one Newton
+// iteration for every group of the wave) at 1 or 2 waves per SIMD: about 27000
+// cycles for drm19 at 32 lanes, a third of them the falloff reactions.  Tables
+// read from device memory by lane and unrolled factorisation steps made it
+// 105000.  Measured (one MI355X, box or 1-D call of 1e-5 s at rtol 1e-10, state
+// restored before each call), against one cell per lane: drm19 64^3 cells 222 ->
+// 70 ms, 2898 cells 95 -> 5.9 ms; dodecane_lu 10000 cells 1558 -> 13.6 ms;
+// heptane_lu_88sk 2048 cells, 1e-6 s at rtol 1e-8, 1169 -> 11.0 ms.
 //
 // Every group reduction returns the bitwise-identical value in all lanes of
 // the group (pairs are always added in commuted order on both partners), so
-// the integrator's control flow is uniform within a group: the group's lanes
-// are always active together, which the lane exchanges require.  Different
-// groups of a wave follow their own cells; as in batched.h every trip of the
+// the integrator's control flow is uniform within a group.  Different groups
+// of a wave follow their own cells; as in batched.h every trip of the
 // persistent loop evaluates one right-hand side for every group that is not
-// waiting for a factorisation, and the groups' Jacobian / LU requests are
-// served together once enough of them wait.
+// waiting for a factorisation, and the groups' LU requests are served together
+// once enough of them wait.  A cell's arithmetic does not depend on which
+// groups share its wave, so results do not depend on the queue's order.
 //
 // The step / order / Newton logic is that of batched_kernel (batched.h), the
 // NDF family of SciPy's BDF integrator; every loop over a cell's work is
@@ -47,6 +54,7 @@
 #include "reactors.h"
 #include "wave.h"
 #include "batched.h"
+#include "pack.h"
 
 namespace ppc {
 
@@ -55,6 +63,35 @@ template <int G>
 struct Grp {
   static_assert(G == 8 || G == 16 || G == 32 || G == 64, "groups of 8, 16, 32 or 64 lanes");
   PPC_DI static int lane() { return (int)__lane_id() & (G - 1); }
+  // v of the partner row(s): the two results hold, in every lane, the value of
+  // this lane's 16-lane row (32-lane half) pair, the same pair on both sides
+  template <bool HALF>
+  PPC_DI static void pair32(unsigned v, unsigned& a, unsigned& b) {
+    if constexpr (HALF) {
+      const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+      a = r[0];
+      b = r[1];
+    } else {
+      const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+      a = r[0];
+      b = r[1];
+    }
+  }
+  template <bool HALF>
+  PPC_DI static void pair(double v, double& a, double& b) {
+    unsigned al, bl, ah, bh;
+    pair32<HALF>(wave::lo32(v), al, bl);
+    pair32<HALF>(wave::hi32(v), ah, bh);
+    a = wave::from32(ah, al);
+    b = wave::from32(bh, bl);
+  }
+  template <bool HALF>
+  PPC_DI static void pair(float v, float& a, float& b) {
+    unsigned x, y;
+    pair32<HALF>(__float_as_uint(v), x, y);
+    a = __uint_as_float(x);
+    b = __uint_as_float(y);
+  }
   // all-reduce sum / max over the group, bitwise identical in every lane
   template <typename T>
   PPC_DI static T sum(T v) {
@@ -62,8 +99,15 @@ struct Grp {
     v += wave::dpp<wave::DPP_XOR2>(v);
     v += wave::dpp<wave::DPP_HALF_MIRROR>(v);
     if (G >= 16) v += wave::dpp<wave::DPP_MIRROR>(v);
-    if (G >= 32) v += __shfl_xor(v, 16, 64);
-    if (G >= 64) v += __shfl_xor(v, 32, 64);
+    T a, b;
+    if (G >= 32) {
+      pair<false>(v, a, b);
+      v = a + b;
+    }
+    if (G >= 64) {
+      pair<true>(v, a, b);
+      v = a + b;
+    }
     return v;
   }
   template <typename T>
@@ -72,18 +116,26 @@ struct Grp {
     v = fmax(v, wave::dpp<wave::DPP_XOR2>(v));
     v = fmax(v, wave::dpp<wave::DPP_HALF_MIRROR>(v));
     if (G >= 16) v = fmax(v, wave::dpp<wave::DPP_MIRROR>(v));
-    if (G >= 32) v = fmax(v, __shfl_xor(v, 16, 64));
-    if (G >= 64) v = fmax(v, __shfl_xor(v, 32, 64));
-    return v;
-  }
-  PPC_DI static unsigned long long umax(unsigned long long v) {
-#pragma unroll
-    for (int m = 1; m < G; m <<= 1) {
-      const unsigned long long o = __shfl_xor(v, m, G);
-      v = o > v ? o : v;
+    T a, b;
+    if (G >= 32) {
+      pair<false>(v, a, b);
+      v = fmax(a, b);
+    }
+    if (G >= 64) {
+      pair<true>(v, a, b);
+      v = fmax(a, b);
     }
     return v;
   }
+  // this group's bits of a ballot
+  PPC_DI static unsigned long long bits(unsigned long long b) {
+    if constexpr (G == 64) {
+      return b;
+    } else {
+      return (b >> (__lane_id() & ~(unsigned)(G - 1))) & ((1ULL << G) - 1);
+    }
+  }
+  PPC_DI static bool any(bool p) { return bits(__ballot(p)) != 0; }
   // value of lane src (0 <= src < G) of the group
   template <typename T>
   PPC_DI static T bcast(T v, int src) {
@@ -91,233 +143,303 @@ struct Grp {
   }
 };
 
-// Orders this lane's LDS accesses around an exchange with the other lanes of
-// its group (all in the same wavefront).
-PPC_DI void group_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+// Orders this lane's LDS accesses around an exchange with other lanes of its
+// wavefront: a wave's LDS operations execute in order, so only the compiler
+// has to be held back.
+PPC_DI void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-// Loads and stores of the per-group Jacobian accumulator in the workspace,
-// which the group's lanes update with device-scope atomics.
+// Loads and stores of the Jacobian accumulator in the workspace, which the
+// wave's lanes update with device-scope atomics.
 PPC_DI double ws_load(const double* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 PPC_DI void ws_store(double* p, double v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// The block's copy of a mechanism's packed tables.
+template <class T>
+PPC_DI typename T::Packed& lds_pack() {
+  __shared__ typename T::Packed p;
+  return p;
+}
+
+// The table accessors TabMech::jac_reaction reads, in packed reaction order.
+template <class T>
+struct PackTab : T {
+  PPC_DI static int sp(int k) { return k == T::NX ? -1 : k; }
+  PPC_DI static double rxA_(int j) { return lds_pack<T>().rx[j].A; }
+  PPC_DI static double rxB_(int j) { return lds_pack<T>().rx[j].b; }
+  PPC_DI static double rxE_(int j) { return lds_pack<T>().rx[j].E; }
+  PPC_DI static int rxR_(int i) { return sp(lds_pack<T>().rx[i / 3].r[i % 3]); }
+  PPC_DI static int rxP_(int i) { return sp(lds_pack<T>().rx[i / 3].p[i % 3]); }
+  PPC_DI static int rxDelta_(int j) { return lds_pack<T>().rx[j].delta; }
+  PPC_DI static int rxRev_(int j) { return lds_pack<T>().rx[j].flags & 1; }
+  PPC_DI static int rxNet_(int i) {
+    return T::rxNet_(T::MAXNET * (int)lds_pack<T>().perm[i / T::MAXNET] + i % T::MAXNET);
+  }
+  PPC_DI static double rxNu_(int i) {
+    return T::rxNu_(T::MAXNET * (int)lds_pack<T>().perm[i / T::MAXNET] + i % T::MAXNET);
+  }
+  PPC_DI static int rxEff0_(int j) { return lds_pack<T>().eff[j - T::N_EL].e0; }
+  PPC_DI static int rxEffN_(int j) { return lds_pack<T>().eff[j - T::N_EL].n; }
+  PPC_DI static int effK_(int i) { return lds_pack<T>().effK[i]; }
+  PPC_DI static double effV_(int i) { return lds_pack<T>().effV[i]; }
+  PPC_DI static double foA_(int f) { return lds_pack<T>().fo[f].A; }
+  PPC_DI static double foB_(int f) { return lds_pack<T>().fo[f].b; }
+  PPC_DI static double foE_(int f) { return lds_pack<T>().fo[f].E; }
+  PPC_DI static double troe_(int i) {
+    const auto& f = lds_pack<T>().fo[i / 4];
+    return i % 4 == 0 ? f.tA : (i % 4 == 1 ? f.t3 : (i % 4 == 2 ? f.t1 : f.t2));
+  }
+  PPC_DI static int troeT2_(int f) { return lds_pack<T>().fo[f].has2 != 0.0; }
+};
 
 // ------------------------------------------- the mechanism on a group --
 template <class T, int G>
 struct GroupChem {
-  using TM = TabMech<T>;
+  using TM = TabMech<PackTab<T>>;
+  using PK = typename T::Packed;
   using Gr = Grp<G>;
-  static constexpr int NS = T::NS, NR = T::NR, n = T::NEQ;
-  static constexpr int EPL = (n + G - 1) / G;   // equation slots per lane
-  static constexpr int SPL = (NS + G - 1) / G;  // species slots per lane
-  static constexpr int RPL = (NR + G - 1) / G;  // reaction slots per lane
+  static constexpr int NS = T::NS, NR = T::NR, n = T::NEQ, NX = T::NX, NCH = T::NCH;
+  static constexpr int NG = 64 / G;
+  static constexpr int EPL = (n + G - 1) / G;    // equation slots per lane
+  static constexpr int SPL = (NS + G - 1) / G;   // species slots per lane
   static constexpr int TL = NS % G, TS = NS / G;  // lane and slot of the temperature equation
+  static constexpr int NP = (n + 1) & ~1;        // vectors of n, 16-byte aligned
 
-  // per-group LDS: RHS exchange, Jacobian species data, the pivot row of
-  // the Newton-matrix inversion and two vectors for its column scaling and
-  // solves
-  struct Shared {
-    double c[NS], a[NS], b[NS], q[NR];
-    double g[NS], h[NS], wd[NS];
-    double v[n], w[n], prow[n];
-  };
+  // A group's LDS area (doubles): concentrations with exp(-g/RT) and
+  // c exp(g/RT) of every species, an unused place's ones after them (later
+  // the chunk sums), then the rates of progress with a zero after them (later
+  // the vectors of the Newton solve).  Its size is 4 modulo 8 doubles, so that
+  // the groups' broadcasts fall into different banks.
+  static constexpr int cmax(int a, int b) { return a > b ? a : b; }
+  static constexpr int S_CA = 0, S_B = 2 * (NX + 1);
+  static constexpr int S_Q = (cmax(3 * (NX + 1), NCH) + 1) & ~1;
+  static constexpr int S_RAW = S_Q + cmax(NR + 1, 3 * NP);
+  static constexpr int AREA = ((S_RAW + 3) / 8) * 8 + 4;
+  // The wave's Jacobian area overlays its groups' areas: 5 species vectors and,
+  // where n is small enough, the n x n accumulator.
+  static constexpr bool JLDS = n <= 32;
+  static constexpr int J_AT = (5 * NP + 1) & ~1;
+  static constexpr int WAREA = (cmax(NG * AREA, J_AT + (JLDS ? n * n : 0)) + 3) & ~3;
 
-  // Per-lane constants of the lane's species, set once per kernel: when a
-  // lane holds one species (SPL == 1) its NASA7 coefficients and range
-  // midpoint (no table loads in the hot loop); for every slot, imw_k times
-  // h_k/RT and cp_k/R (or e_k/RT, cv_k/R) at the bounds 90 K and 4000 K of
-  // the temperature inversion.
-  static constexpr int NC = SPL == 1 ? 1 : 0;
-  struct Cache {
-    double lo[NC > 0 ? NC : 1][7], hi[NC > 0 ? NC : 1][7], tmid[NC > 0 ? NC : 1];
-    double hb[2][SPL], cb[2][SPL];
-  };
-  PPC_DI static void init_cache(Cache& cc, const int g, const bool enth) {
+  PPC_DI static void coefs(const PK& pk, const int k, const double Tv, double (&a)[7], double& imw) {
+    const double* s = pk.sp[k].lo;
+    const double* c = Tv < s[7] ? s : s + 8;
 #pragma unroll
-    for (int e = 0; e < NC; ++e) {
-      const int k = (e * G + g < NS) ? e * G + g : 0;
-#pragma unroll
-      for (int i = 0; i < 7; ++i) {
-        cc.lo[e][i] = T::nasaLo_(7 * k + i);
-        cc.hi[e][i] = T::nasaHi_(7 * k + i);
-      }
-      cc.tmid[e] = T::tmid_(k);
-    }
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const double Tb = b == 0 ? 90.0 : 4000.0;
-#pragma unroll
-      for (int e = 0; e < SPL; ++e) {
-        const int k = e * G + g;
-        cc.hb[b][e] = cc.cb[b][e] = 0.0;
-        if (k < NS) {
-          double a[7];
-          TM::nasa(k, Tb, a);
-          const double hp = TM::h_poly(a, Tb, 1.0 / Tb), cp = TM::cp_poly(a, Tb);
-          cc.hb[b][e] = T::imw_(k) * (enth ? hp : hp - 1.0);
-          cc.cb[b][e] = T::imw_(k) * (enth ? cp : cp - 1.0);
-        }
-      }
-    }
-  }
-  // NASA7 coefficients of slot e (species k) for temperature Tv
-  PPC_DI static void nasa(const Cache& cc, const int e, const int k, const double Tv, double* a) {
-    if constexpr (NC > 0) {
-      const bool lo = Tv < cc.tmid[0];
-#pragma unroll
-      for (int i = 0; i < 7; ++i) a[i] = lo ? cc.lo[0][i] : cc.hi[0][i];
-    } else {
-      TM::nasa(k, Tv, a);
-    }
+    for (int i = 0; i < 7; ++i) a[i] = c[i];
+    imw = s[15];
   }
 
-  // mixture h (erg/g) and cp (erg/g/K), or e and cv, at Tv (Fuego.H CKHBMS/CKCPBS)
-  template <bool ENTH>
-  PPC_DI static void mix(const Cache& cc, const int g, const double (&Y)[SPL], const double Tv, double& hm,
-                         double& cm) {
+  // sum y h/RT imw and sum y cp/R imw (or e, cv) of the group's cell at Tv
+  PPC_DI static void heat(const PK& pk, const int g, const bool eform, const double (&y)[EPL], const double Tv,
+                          double& hs, double& cs, double (&hk)[SPL]) {
     const double invT = 1.0 / Tv;
-    double hs = 0.0, cs = 0.0;
+    double h = 0.0, c = 0.0;
 #pragma unroll
     for (int e = 0; e < SPL; ++e) {
       const int k = e * G + g;
+      hk[e] = 0.0;
       if (k < NS) {
-        double a[7];
-        nasa(cc, e, k, Tv, a);
+        double a[7], imw;
+        coefs(pk, k, Tv, a, imw);
         double hp = TM::h_poly(a, Tv, invT), cp = TM::cp_poly(a, Tv);
-        if (!ENTH) {
+        if (eform) {
           hp -= 1.0;
           cp -= 1.0;
         }
-        const double yw = Y[e] * T::imw_(k);
-        hs += yw * hp;
-        cs += yw * cp;
+        const double yw = y[e] * imw;
+        h += yw * hp;
+        c += yw * cp;
+        hk[e] = hp;
       }
     }
-    hm = Gr::sum(hs) * (RU * Tv);
-    cm = Gr::sum(cs) * RU;
-  }
-
-  // mixture h (or e) at bound b (0: 90 K, 1: 4000 K) from the cached species
-  // values; with cp too only when the caller extrapolates
-  PPC_DI static double mix_bound(const Cache& cc, const int b, const double (&Y)[SPL], const bool want_c,
-                                 double& cm) {
-    double hs = 0.0, cs = 0.0;
-#pragma unroll
-    for (int e = 0; e < SPL; ++e) {
-      hs += Y[e] * cc.hb[b][e];
-      cs += Y[e] * cc.cb[b][e];
-    }
-    cm = want_c ? Gr::sum(cs) * RU : 0.0;
-    return Gr::sum(hs) * (RU * (b == 0 ? 90.0 : 4000.0));
+    hs = Gr::sum(h);
+    cs = Gr::sum(c);
   }
 
   // GET_T_GIVEN_HY / GET_T_GIVEN_EY (Mechanisms/drm19/mechanism.H:2789-2890)
-  // with group sums: Newton on T, |dT| clamped to 100 K, stop at |dT| < 1e-6,
-  // at most 200 iterations, linear extrapolation outside [90, 4000] K.  (The
-  // cache was built for the same energy form.)
-  template <bool ENTH>
-  PPC_DI static double T_from_energy(const Cache& cc, const int g, const double hv, const double (&Y)[SPL],
-                                     const double tguess) {
+  // of the cell's energy per volume E: Newton on T, |dT| clamped to 100 K, stop
+  // at |dT| < 1e-6, at most 200 iterations, linear extrapolation outside [90,
+  // 4000] K.  The integrated temperature is nearly always within 1e-6 K, so
+  // the energies at the bounds are formed only when the first iteration has
+  // not ended there.  Also the heat sums and species energies at the result.
+  PPC_DI static double T_from_energy(const PK& pk, const int g, const bool eform, const double E,
+                                     const double (&y)[EPL], double Tv, double& cs, double (&hk)[SPL]) {
     const double tmin = 90.0, tmax = 4000.0;
-    double cmin, cmax;
-    const double hmin = mix_bound(cc, 0, Y, false, cmin), hmax = mix_bound(cc, 1, Y, false, cmax);
-    if (hv < hmin) {
-      mix_bound(cc, 0, Y, true, cmin);
-      return tmin - (hmin - hv) / cmin;
-    }
-    if (hv > hmax) {
-      mix_bound(cc, 1, Y, true, cmax);
-      return tmax - (hmax - hv) / cmax;
-    }
-    double t1 = tguess;
-    if (t1 < tmin || t1 > tmax) t1 = tmin + (tmax - tmin) / (hmax - hmin) * (hv - hmin);
-    for (int i = 0; i < 200; ++i) {
-      double h1, c1;
-      mix<ENTH>(cc, g, Y, t1, h1, c1);
-      double dt = (hv - h1) / c1;
-      if (dt > 100.0) {
-        dt = 100.0;
-      } else if (dt < -100.0) {
-        dt = -100.0;
-      } else if (fabs(dt) < 1.0e-6) {
-        break;
+    // 0: at the guess; 1, 2: at the bounds; 3: Newton; 4: at the final T
+    int what = 0, it = 0;
+    double Tq = Tv, dt = 0.0, rinv = 0.0, hmin = 0.0, cmin = 0.0;
+#pragma unroll 1
+    for (;;) {
+      double hs;
+      heat(pk, g, eform, y, Tq, hs, cs, hk);
+      if (what == 4) break;
+      if (what == 0 || what == 3) {
+        dt = (E - hs * (RU * Tq)) / (cs * RU);
+        if (fabs(dt) < 1.0e-6 && (what == 3 || (Tv >= tmin && Tv <= tmax))) break;
+        if (what == 0) {
+          double rs = 0.0;
+#pragma unroll
+          for (int e = 0; e < SPL; ++e)
+            if (e * G + g < NS) rs += y[e];
+          rinv = 1.0 / Gr::sum(rs);
+          what = 1;
+          Tq = tmin;
+          continue;
+        }
+      } else if (what == 1) {
+        hmin = hs * (RU * tmin * rinv);
+        cmin = cs * (RU * rinv);
+        what = 2;
+        Tq = tmax;
+        continue;
+      } else {
+        const double hv = E * rinv, hmax = hs * (RU * tmax * rinv), cmax = cs * (RU * rinv);
+        if (hv < hmin || hv > hmax) {
+          Tv = hv < hmin ? tmin - (hmin - hv) / cmin : tmax - (hmax - hv) / cmax;
+          what = 4;
+          Tq = Tv;
+          continue;
+        }
+        what = 3;
+        if (Tv < tmin || Tv > tmax) {
+          Tv = tmin + (tmax - tmin) / (hmax - hmin) * (hv - hmin);
+          Tq = Tv;
+          continue;
+        }
       }
-      t1 += dt;
+      Tv += dt > 100.0 ? 100.0 : (dt < -100.0 ? -100.0 : dt);
+      Tq = Tv;
+      // 200 iterations, or NaN (as every further iterate would be)
+      if (++it == 200 || !(dt == dt)) what = 4;
     }
-    return t1;
+    return Tv;
   }
 
-  // net rates of progress of this lane's reactions into sh.q, from sh.c/a/b
-  PPC_DI static void progress(Shared& sh, const int g, const double mixture, const double Tv, const double invT,
-                              const double logT) {
-    const double refC = 101325.0 / 8.31446 * invT, refCinv = 1.0 / refC;
-#pragma unroll 1
-    for (int r = 0; r < RPL; ++r) {
-      const int j = r * G + g;
-      if (j < NR) {
-        double q;
-        if (j < T::N_EL) {
-          q = TM::template rate<0>(j, 0, sh.c, sh.a, sh.b, mixture, Tv, invT, logT, refC, refCinv);
-        } else if (j < T::N_EL + T::N_TB) {
-          q = TM::template rate<1>(j, 0, sh.c, sh.a, sh.b, mixture, Tv, invT, logT, refC, refCinv);
-        } else if (j < T::N_EL + T::N_TB + T::N_TROE) {
-          q = TM::template rate<2>(j, j - T::N_EL - T::N_TB, sh.c, sh.a, sh.b, mixture, Tv, invT, logT, refC,
-                                   refCinv);
+  PPC_DI static double refc_pow(const int d, const double refC, const double refCinv) {
+    double r = d > 0 ? refC : (d < 0 ? refCinv : 1.0);
+    const double b = r;
+    for (int i = d < 0 ? -d : d; i > 1; --i) r *= b;
+    return r;
+  }
+
+  // net rate of progress of reaction j (packed order) of KIND (0 elementary, 1
+  // three-body, 2 Troe, 3 Lindemann falloff) from the group's LDS area
+  template <int KIND>
+  PPC_DI static double rate(const PK& pk, const double* ca, const double* b, const int j, const double mixture,
+                            const double Tv, const double invT, const double logT, const double refC,
+                            const double refCinv) {
+    const tab::PackRx rx = pk.rx[j];
+    const double kf0 = rx.A * exp(rx.b * logT - rx.E * invT);
+    double kf = kf0;
+    if constexpr (KIND >= 1) {
+      double alpha = mixture;
+      const tab::PackEff ef = pk.eff[j - T::N_EL];
+#pragma unroll 4
+      for (int i = 0; i < ef.n; ++i) alpha += pk.effV[ef.e0 + i] * ca[2 * pk.effK[ef.e0 + i]];
+      if constexpr (KIND == 1) {
+        kf *= alpha;
+      } else {
+        const tab::PackFo f = pk.fo[j - T::N_EL - T::N_TB];
+        const double k0 = f.A * exp(f.b * logT - f.E * invT);
+        const double redP = alpha / kf0 * k0;
+        const double F = redP / (1.0 + redP);
+        if constexpr (KIND == 2) {
+          double Fcent = (1.0 - f.tA) * exp(-Tv / f.t3) + f.tA * exp(-Tv / f.t1);
+          if (f.has2 != 0.0) Fcent += exp(-f.t2 * invT);
+          const double logFcent = log10(Fcent);
+          const double logPred = log10(redP);
+          const double tc = -0.4 - 0.67 * logFcent;
+          const double tn = 0.75 - 1.27 * logFcent;
+          const double tr = (tc + logPred) / (tn - 0.14 * (tc + logPred));
+          kf *= F * exp(LN10 * logFcent / (1.0 + tr * tr));
         } else {
-          q = TM::template rate<3>(j, j - T::N_EL - T::N_TB, sh.c, sh.a, sh.b, mixture, Tv, invT, logT, refC,
-                                   refCinv);
+          kf *= F;
         }
-        sh.q[j] = q;
       }
     }
+    const int r0 = rx.r[0], r1 = rx.r[1], r2 = rx.r[2];
+    const double c0 = ca[2 * r0], a0 = ca[2 * r0 + 1], c1 = ca[2 * r1], a1 = ca[2 * r1 + 1];
+    double qf = kf * c0 * c1;
+    double a2 = 1.0;
+    if (r2 != NX) {
+      qf *= ca[2 * r2];
+      a2 = ca[2 * r2 + 1];
+    }
+    double qr = 0.0;
+    if (rx.flags & 1) {
+      const int p2 = rx.p[2];
+      qr = kf * refc_pow(rx.delta, refC, refCinv) * a0 * b[rx.p[0]] * a1 * a2 * b[rx.p[1]];
+      if (p2 != NX) qr *= b[p2];
+    }
+    return qf - qr;
   }
 
   // fKernelSpec (Source/Reactions/ReactorUtils.H:358-415) for the group's
   // cell: y (this lane's equation slots), f = ydot of the same slots.
-  PPC_DI static void rhs(Shared& sh, const Cache& cc, const int g, const int reactor_type, const double dt_save,
+  PPC_DI static void rhs(const PK& pk, double* sh, const int g, const bool eform, const double dt_save,
                          const double (&y)[EPL], const double (&src)[SPL], const double rhoe_init,
                          const double rhoesrc_ext, double (&f)[EPL]) {
-    double rsum = 0.0;
-#pragma unroll
-    for (int e = 0; e < SPL; ++e)
-      if (e * G + g < NS) rsum += y[e];
-    const double rho = Gr::sum(rsum);
-    const double rinv = 1.0 / rho;
-    double Y[SPL];
-#pragma unroll
-    for (int e = 0; e < SPL; ++e) Y[e] = (e * G + g < NS) ? y[e] * rinv : 0.0;
-    const double nrg = (rhoe_init + rhoesrc_ext * dt_save) * rinv;
-    double Tv = Gr::bcast(y[TS], TL);
-    const bool eform = reactor_type == E_REACTOR;
-    Tv = eform ? T_from_energy<false>(cc, g, nrg, Y, Tv) : T_from_energy<true>(cc, g, nrg, Y, Tv);
+    double hk[SPL], cs;
+    const double Tv = T_from_energy(pk, g, eform, rhoe_init + rhoesrc_ext * dt_save, y, Gr::bcast(y[TS], TL), cs, hk);
     const double invT = 1.0 / Tv, logT = log(Tv), RT = RU * Tv;
-    double ek[SPL], csum = 0.0, msum = 0.0;
+    double* ca = sh + S_CA;
+    double* b = sh + S_B;
+    double* q = sh + S_Q;
+    double msum = 0.0;
+    if (g == 0) {
+      ca[2 * NX] = 1.0;
+      ca[2 * NX + 1] = 1.0;
+      b[NX] = 1.0;
+      q[NR] = 0.0;
+    }
 #pragma unroll
     for (int e = 0; e < SPL; ++e) {
       const int k = e * G + g;
-      ek[e] = 0.0;
       if (k < NS) {
-        double a[7];
-        nasa(cc, e, k, Tv, a);
-        const double hp = TM::h_poly(a, Tv, invT), cp = TM::cp_poly(a, Tv);
-        const double imw = T::imw_(k);
-        ek[e] = (eform ? hp - 1.0 : hp) * RT * imw;  // CKUMS / CKHMS
-        csum += Y[e] * imw * (eform ? cp - 1.0 : cp);
-        const double sc = (rho * Y[e] * imw) * 1.0e6;  // CKYTCR, SI
+        double a[7], imw;
+        coefs(pk, k, Tv, a, imw);
+        hk[e] *= RT * imw;  // CKUMS / CKHMS
+        const double sc = (y[e] * imw) * 1.0e6;  // CKYTCR, SI
         const double eg = exp(TM::g_poly(a, Tv, invT, logT));
-        sh.c[k] = sc;
-        sh.a[k] = 1.0 / eg;
-        sh.b[k] = sc * eg;
+        ca[2 * k] = sc;
+        ca[2 * k + 1] = 1.0 / eg;
+        b[k] = sc * eg;
         msum += sc;
       }
     }
-    const double cmix = Gr::sum(csum) * RU;
     const double mixture = Gr::sum(msum);
-    group_sync();
-    progress(sh, g, mixture, Tv, invT, logT);
-    group_sync();
+    const double refC = 101325.0 / 8.31446 * invT, refCinv = 1.0 / refC;
+    wave_sync();
+#pragma unroll 1
+    for (int j = g; j < T::N_EL; j += G) q[j] = rate<0>(pk, ca, b, j, mixture, Tv, invT, logT, refC, refCinv);
+    if constexpr (T::N_TB > 0) {
+#pragma unroll 1
+      for (int j = T::N_EL + g; j < T::N_EL + T::N_TB; j += G)
+        q[j] = rate<1>(pk, ca, b, j, mixture, Tv, invT, logT, refC, refCinv);
+    }
+    if constexpr (T::N_TROE > 0) {
+#pragma unroll 1
+      for (int j = T::N_EL + T::N_TB + g; j < NR - T::N_LIND; j += G)
+        q[j] = rate<2>(pk, ca, b, j, mixture, Tv, invT, logT, refC, refCinv);
+    }
+    if constexpr (T::N_LIND > 0) {
+#pragma unroll 1
+      for (int j = NR - T::N_LIND + g; j < NR; j += G)
+        q[j] = rate<3>(pk, ca, b, j, mixture, Tv, invT, logT, refC, refCinv);
+    }
+    wave_sync();
+    double* part = sh;
+#pragma unroll 1
+    for (int v = g; v < NCH; v += G) {
+      const tab::PackCh ch = pk.ch[v];
+      double w = 0.0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) w += (double)((int)(ch.e[i] >> 12) - 8) * q[ch.e[i] & 0xfff];
+      part[v] = w;
+    }
+    wave_sync();
     double esum = 0.0;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) f[e] = 0.0;
@@ -326,44 +448,59 @@ struct GroupChem {
       const int k = e * G + g;
       if (k < NS) {
         double w = 0.0;
-        const int e1 = T::spPtr_(k + 1);
-#pragma unroll 1
-        for (int s = T::spPtr_(k); s < e1; ++s) w += T::spNu_(s) * sh.q[T::spRx_(s)];
-        const double v = w * 1.0e-6 * T::mw_(k) + src[e];  // RTY2WDOT (CKWC units) + source
-        f[e] = v;
-        esum += v * ek[e];
+        const int v1 = pk.spCh[k + 1];
+#pragma unroll 2
+        for (int v = pk.spCh[k]; v < v1; ++v) w += part[v];
+        const double s = w * 1.0e-6 * pk.mw[k] + src[e];  // RTY2WDOT (CKWC units) + source
+        f[e] = s;
+        esum += s * hk[e];
       }
     }
-    group_sync();
+    wave_sync();
     const double srcT = rhoesrc_ext - Gr::sum(esum);
-    if (g == TL) f[TS] = srcT * (rinv / cmix);
+    if (g == TL) f[TS] = srcT / (cs * RU);
   }
 
-  // The BDF Jacobian d f_i / d y_j at y (bdf_jacobian in chem_cell.h with
-  // s = 1): accumulated in the group's n x n FP64 area Jw of the workspace
-  // (column-major, aJacobian / DWDOT layout), then row i = e*G + g written
-  // to Jrow(e, j) in JT.
-  template <int CONSP, typename JT, class JR>
-  PPC_DI static void jacobian(Shared& sh, const Cache& cc, const int g, double* Jw, const double (&y)[EPL],
-                              JR Jrow) {
-    const double Tv = Gr::bcast(y[TS], TL);
+  // The BDF Jacobian d f_i / d y_j (bdf_jacobian in chem_cell.h with s = 1) of
+  // one cell by the whole wave: y in wa[0..n) of the wave's area, accumulated
+  // column-major (aJacobian / DWDOT layout) in J, then element (i, j) stored at
+  // out[(e*n + j)*G + g] for i = e*G + g.  J is in LDS or, for the larger
+  // mechanisms, in the workspace.
+  template <int CONSP, typename JT>
+  PPC_DI static void jacobian(const PK& pk, double* wa, double* J, JT* out) {
+    constexpr int W = (NS + 63) / 64;
+    const int l = (int)__lane_id();
+    const double* y = wa;
+    double *c = wa + NP, *gk = wa + 2 * NP, *hh = wa + 3 * NP, *wd = wa + 4 * NP;
+    const auto ld = [&](int i) { return JLDS ? J[i] : ws_load(J + i); };
+    const auto st = [&](int i, double v) {
+      if (JLDS)
+        J[i] = v;
+      else
+        ws_store(J + i, v);
+    };
+    const auto jsync = [&]() {
+      if (!JLDS) __threadfence();
+      wave_sync();
+    };
+    const double Tv = y[NS];
     const double invT = 1.0 / Tv, invT2 = invT * invT, logT = log(Tv);
     const double refC = 101325.0 / 8.31446 * invT, refCinv = 1.0 / refC;
-    double cR[SPL], dcR[SPL], eh[SPL], sc[SPL];
+    double cR[W], dcR[W], eh[W], sc[W];
     double msum = 0.0;
 #pragma unroll
-    for (int e = 0; e < SPL; ++e) {
-      const int k = e * G + g;
+    for (int e = 0; e < W; ++e) {
+      const int k = e * 64 + l;
       cR[e] = dcR[e] = eh[e] = sc[e] = 0.0;
       if (k < NS) {
-        double a[7];
-        nasa(cc, e, k, Tv, a);
+        double a[7], imw;
+        coefs(pk, k, Tv, a, imw);
         const double hRT = TM::h_poly(a, Tv, invT), cpR = TM::cp_poly(a, Tv);
-        sc[e] = y[e] * T::imw_(k) * 1.0e6;  // CKYTCR + DWDOT (x1e6)
-        sh.c[k] = sc[e];
-        sh.g[k] = TM::g_poly(a, Tv, invT, logT);
-        sh.h[k] = hRT;
-        sh.wd[k] = 0.0;
+        sc[e] = y[k] * imw * 1.0e6;  // CKYTCR + DWDOT (x1e6)
+        c[k] = sc[e];
+        gk[k] = TM::g_poly(a, Tv, invT, logT);
+        hh[k] = hRT;
+        wd[k] = 0.0;
         cR[e] = (CONSP == 1) ? cpR : cpR - 1.0;
         eh[e] = (CONSP == 1) ? hRT : hRT - 1.0;
         dcR[e] = TM::dcp_poly(a, Tv);
@@ -371,79 +508,69 @@ struct GroupChem {
       }
     }
 #pragma unroll 1
-    for (int i = g; i < n * n; i += G) ws_store(Jw + i, 0.0);
-    const double mixture = Gr::sum(msum);
-    __threadfence();
-    group_sync();
+    for (int i = l; i < n * n; i += 64) st(i, 0.0);
+    const double mixture = wave::sum(msum);
+    jsync();
 #pragma unroll 1
-    for (int r = 0; r < RPL; ++r) {
-      const int j = r * G + g;
-      if (j < NR)
-        TM::template jac_reaction<CONSP>(
-            j, sh.c, sh.g, sh.h, mixture, Tv, invT, invT2, logT, refC, refCinv,
-            [&](int idx, double v) { unsafeAtomicAdd(Jw + idx, v); },
-            [&](int m, double v) { atomicAdd(&sh.wd[m], v); });
-    }
-    __threadfence();
-    group_sync();
+    for (int j = l; j < NR; j += 64)
+      TM::template jac_reaction<CONSP>(
+          j, c, gk, hh, mixture, Tv, invT, invT2, logT, refC, refCinv,
+          [&](int idx, double v) {
+            if (JLDS)
+              __hip_atomic_fetch_add(J + idx, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            else
+              unsafeAtomicAdd(J + idx, v);
+          },
+          [&](int m, double v) {
+            __hip_atomic_fetch_add(wd + m, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          });
+    jsync();
     // temperature row (aJacobian, Mechanisms/drm19/mechanism.H:15317-15352)
     double s_cm = 0.0, s_dcm = 0.0, s_eh = 0.0, s_deh = 0.0;
 #pragma unroll
-    for (int e = 0; e < SPL; ++e) {
-      const int k = e * G + g;
+    for (int e = 0; e < W; ++e) {
+      const int k = e * 64 + l;
       if (k < NS) {
-        const double wdk = sh.wd[k];
+        const double wdk = wd[k];
         s_cm += cR[e] * sc[e];
         s_dcm += dcR[e] * sc[e];
         s_eh += eh[e] * wdk;
-        s_deh += invT * (cR[e] - eh[e]) * wdk + eh[e] * ws_load(Jw + NS * n + k);
+        s_deh += invT * (cR[e] - eh[e]) * wdk + eh[e] * ld(NS * n + k);
       }
     }
-    const double cmix = Gr::sum(s_cm), dcmixdT = Gr::sum(s_dcm);
-    const double ehmix = Gr::sum(s_eh), dehmixdT = Gr::sum(s_deh);
+    const double cmix = wave::sum(s_cm), dcmixdT = wave::sum(s_dcm);
+    const double ehmix = wave::sum(s_eh), dehmixdT = wave::sum(s_deh);
     const double cmixinv = 1.0 / cmix;
     const double tmp1 = ehmix * cmixinv, tmp3 = cmixinv * Tv, tmp2 = tmp1 * tmp3;
-    double trow[SPL];
+    double trow[W];
 #pragma unroll
-    for (int e = 0; e < SPL; ++e) {
-      const int k = e * G + g;
+    for (int e = 0; e < W; ++e) {
+      const int k = e * 64 + l;
       trow[e] = 0.0;
       if (k < NS) {
         double d = 0.0;
-#pragma unroll 1
-        for (int mm = 0; mm < NS; ++mm) d += ((CONSP == 1) ? sh.h[mm] : sh.h[mm] - 1.0) * ws_load(Jw + k * n + mm);
+#pragma unroll 8
+        for (int mm = 0; mm < NS; ++mm) d += ((CONSP == 1) ? hh[mm] : hh[mm] - 1.0) * ld(k * n + mm);
         trow[e] = tmp2 * cR[e] - tmp3 * d;
       }
     }
-    __threadfence();
-    group_sync();
+    jsync();
 #pragma unroll
-    for (int e = 0; e < SPL; ++e)
-      if (e * G + g < NS) ws_store(Jw + (e * G + g) * n + NS, trow[e]);
-    if (g == 0) ws_store(Jw + n * n - 1, -tmp1 + tmp2 * dcmixdT - tmp3 * dehmixdT);
-    __threadfence();
-    group_sync();
-    // DWDOT scaling (T column x1e-6, T row x1e6) and the transpose with
-    // molecular-weight scaling: row i, column j = d f_i / d y_j
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      const int i = e * G + g;
-      if (i < n) {
-        const bool spi = i < NS;
-        const double wi = spi ? T::mw_(i) : 1.0;
-#pragma unroll 1
-        for (int jj = 0; jj < n; ++jj) {
-          double a;
-          if (jj < NS) {
-            const double Jv = spi ? ws_load(Jw + jj * n + i) : ws_load(Jw + jj * n + NS) * 1.0e6;
-            a = Jv * wi * T::imw_(jj);
-          } else {
-            const double Jv = spi ? ws_load(Jw + NS * n + i) * 1.0e-6 : ws_load(Jw + n * n - 1);
-            a = Jv * wi;
-          }
-          Jrow(e, jj) = (JT)a;
-        }
-      }
+    for (int e = 0; e < W; ++e)
+      if (e * 64 + l < NS) st((e * 64 + l) * n + NS, trow[e]);
+    if (l == 0) st(n * n - 1, -tmp1 + tmp2 * dcmixdT - tmp3 * dehmixdT);
+    jsync();
+    // DWDOT scaling (T column x1e-6, T row x1e6) and the molecular-weight
+    // scaling: row i, column j = d f_i / d y_j
+#pragma unroll 4
+    for (int t = l; t < n * n; t += 64) {
+      const int j = t / n, i = t - j * n;
+      double v = ld(t);
+      v *= i < NS ? pk.mw[i] : 1.0;
+      v *= j < NS ? pk.sp[j].imw : 1.0;
+      if (i == NS && j < NS) v *= 1.0e6;
+      if (j == NS && i < NS) v *= 1.0e-6;
+      out[((i / G) * n + j) * G + i % G] = (JT)v;
     }
   }
 };
@@ -452,60 +579,71 @@ struct GroupChem {
 // Gauss-Jordan exchange steps on the row-distributed n x n matrix a (lane g
 // holds rows i = e*G + g, e < EPL) with partial pivoting: step k pivots on the
 // largest |a(i, k)| among the rows not yet used (the choice LU with partial
-// pivoting makes), lowest row on ties; rows never move.  The pivot row goes
-// through the group's LDS (prow).  Exchange on (r, k): a(r, k) <- 1 / a(r, k),
+// pivoting makes); rows never move.  The pivot row goes through the group's
+// LDS (prow).  Exchange on (r, k): a(r, k) <- 1 / a(r, k),
 // a(r, j) <- -a(r, j) / a(r, k), a(i, k) <- a(i, k) / a(r, k) and
 // a(i, j) <- a(i, j) - a(i, k) a(r, j) / a(r, k) for the other rows.  After the
 // n steps (kstep[e] = the step at which row i was the pivot) A x = b is
-// solved by x_{kstep(i)} = sum_j a(i, j) b_{p_j}, p_j the pivot row of step j:
-// one dot product per row instead of two sequential triangular sweeps.
+// solved by x_{kstep(i)} = sum_j a(i, j) b_{p_j}, p_j the pivot row of step j.
+//
+// Every step's column is a[.][0]: the update of column j + 1 is written to
+// place j and the exchanged column to place n - 1, so after n steps the
+// columns are back in order, register indices are constants and the step loop
+// is a loop: unrolled over n it is n^2 instructions per row slot (heptane,
+// n = 89: ~0.4 MB of code) that miss the instruction cache at every step
+// (heptane_lu_88sk, 2048 cells, one call of 1e-6 s at rtol 1e-8: 134 ms, 90%
+// of it in this function, against 14.1 ms).
 template <int n, int G, int EPL, typename LT>
-PPC_DI void group_inv_factor(LT (&a)[EPL][n], int (&kstep)[EPL], double* prow, const int g) {
+PPC_DI void group_inv_factor(LT (&a)[EPL][n], int (&kstep)[EPL], LT* prow, const int g) {
   using Gr = Grp<G>;
 #pragma unroll
   for (int e = 0; e < EPL; ++e) kstep[e] = (e * G + g < n) ? -1 : n;
-  group_sync();
-#pragma unroll
+#pragma unroll 1
   for (int k = 0; k < n; ++k) {
-    unsigned long long key = 0;
+    LT best = LT(-1);
+    int be = 0;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
-      if (kstep[e] < 0) {
-        const float m = (float)fabs(a[e][k]);
-        const unsigned long long kk =
-            ((unsigned long long)__float_as_uint(m) << 32) | (unsigned long long)(0xffffffffu - (unsigned)(e * G + g));
-        key = kk > key ? kk : key;
+      LT m = fabs(a[e][0]);
+      m = m == m ? m : LT(INFINITY);
+      if (kstep[e] < 0 && m > best) {
+        best = m;
+        be = e;
       }
     }
-    key = Gr::umax(key);
-    const int p = (int)(0xffffffffu - (unsigned)(key & 0xffffffffu));
-    const int pl = p % G, ps = p / G;
+    const LT mx = Gr::max(best);
+    const int pl = __ffsll((long long)Gr::bits(__ballot(best == mx))) - 1;
+    wave_sync();
     if (g == pl) {
 #pragma unroll
       for (int j = 0; j < n; ++j) {
         LT v = a[0][j];
 #pragma unroll
-        for (int e = 1; e < EPL; ++e) v = (ps == e) ? a[e][j] : v;
-        prow[j] = (double)v;
+        for (int e = 1; e < EPL; ++e) v = (be == e) ? a[e][j] : v;
+        prow[j] = v;
       }
     }
-    group_sync();
-    const LT prs = LT(1) / (LT)prow[k];
+    wave_sync();
+    const LT prs = LT(1) / prow[0];
+    bool isp[EPL];
+    LT f[EPL];
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
-      const bool isp = e * G + g == p;
-      kstep[e] = isp ? k : kstep[e];
-      const LT f = a[e][k] * prs;
-#pragma unroll
-      for (int j = 0; j < n; ++j) {
-        if (j == k) continue;
-        const LT r = (LT)prow[j];
-        a[e][j] = isp ? -r * prs : a[e][j] - f * r;
-      }
-      a[e][k] = isp ? prs : f;
+      isp[e] = g == pl && be == e;
+      kstep[e] = isp[e] ? k : kstep[e];
+      f[e] = isp[e] ? prs : a[e][0] * prs;
     }
-    group_sync();
+#pragma unroll
+    for (int j = 1; j < n; ++j) {
+      if (j % 16 == 0) asm volatile("" ::: "memory");  // keeps few of the row's values in flight
+      const LT r = prow[j];
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) a[e][j - 1] = (isp[e] ? LT(0) : a[e][j]) - f[e] * r;
+    }
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) a[e][n - 1] = f[e];
   }
+  wave_sync();
 }
 
 // x (this lane's equation slots) = A^-1 b (this lane's rows) from the
@@ -517,23 +655,28 @@ PPC_DI void group_inv_solve(const LT (&a)[EPL][n], const int (&kstep)[EPL], doub
 #pragma unroll
   for (int e = 0; e < EPL; ++e)
     if (e * G + g < n) v[kstep[e]] = b[e];  // v_j = b_{p_j}
-  group_sync();
-  double acc[EPL];
+  wave_sync();
+  double acc[EPL], acc2[EPL];
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) acc[e] = 0.0;
+  for (int e = 0; e < EPL; ++e) acc[e] = acc2[e] = 0.0;
 #pragma unroll
   for (int j = 0; j < n; ++j) {
     const double vj = v[j];
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) acc[e] += (double)a[e][j] * vj;
+    for (int e = 0; e < EPL; ++e) {
+      if (j % 2 == 0)
+        acc[e] += (double)a[e][j] * vj;
+      else
+        acc2[e] += (double)a[e][j] * vj;
+    }
   }
 #pragma unroll
   for (int e = 0; e < EPL; ++e)
-    if (e * G + g < n) w[kstep[e]] = acc[e];  // x_{kstep(i)}
-  group_sync();
+    if (e * G + g < n) w[kstep[e]] = acc[e] + acc2[e];  // x_{kstep(i)}
+  wave_sync();
 #pragma unroll
   for (int e = 0; e < EPL; ++e) x[e] = (e * G + g < n) ? w[e * G + g] : 0.0;
-  group_sync();
+  wave_sync();
 }
 
 // D[0..order][e] <- (R U)^T D[0..order][e] for a step-size ratio `factor`
@@ -543,6 +686,7 @@ PPC_DI void group_inv_solve(const LT (&a)[EPL][n], const int (&kstep)[EPL], doub
 // held.
 template <int EPL>
 PPC_DI void group_change_D(double (&D)[AMAXORD + 3][EPL], const int order, const double factor) {
+  constexpr double inv[AMAXORD + 1] = {0.0, 1.0, 0.5, 1.0 / 3.0, 0.25, 0.2};
   double w[AMAXORD + 1][EPL];
 #pragma unroll
   for (int k = 0; k <= AMAXORD; ++k) {
@@ -551,7 +695,7 @@ PPC_DI void group_change_D(double (&D)[AMAXORD + 3][EPL], const int order, const
     for (int e = 0; e < EPL; ++e) w[k][e] = D[0][e];
 #pragma unroll
     for (int kp = 1; kp <= AMAXORD; ++kp) {
-      r *= (k == 0) ? 0.0 : (kp - 1 - factor * k) / (double)kp;
+      r *= (k == 0) ? 0.0 : (kp - 1 - factor * k) * inv[kp];
 #pragma unroll
       for (int e = 0; e < EPL; ++e)
         if (kp <= order) w[k][e] += r * D[kp][e];
@@ -565,10 +709,10 @@ PPC_DI void group_change_D(double (&D)[AMAXORD + 3][EPL], const int order, const
     for (int e = 0; e < EPL; ++e) s[e] = w[0][e];
 #pragma unroll
     for (int k = 1; k <= AMAXORD; ++k) {
-      u *= (i == 0) ? 0.0 : (k - 1 - i) / (double)k;
+      u *= (i == 0) ? 0.0 : (k - 1 - i) * inv[k];  // zero for k > i: only terms k <= i <= order remain
 #pragma unroll
       for (int e = 0; e < EPL; ++e)
-        if (k <= order) s[e] += u * w[k][e];
+        if (k <= i) s[e] += u * w[k][e];
     }
 #pragma unroll
     for (int e = 0; e < EPL; ++e)
@@ -576,61 +720,113 @@ PPC_DI void group_change_D(double (&D)[AMAXORD + 3][EPL], const int order, const
   }
 }
 
-// Doubles of device workspace per group: the FP64 Jacobian accumulator and
-// the group's Jacobian rows in JT.
+// A vector of the lane's equation slots kept in LDS: of the integrator's vectors
+// the four that a trip reads and writes only a few times, so that the others
+// and the inverse's rows stay in registers.
+template <int EPL>
+struct LaneVec {
+  double* p;
+  PPC_DI double& operator[](int e) const { return p[64 * e]; }
+};
+
+// 10 x the distance from t (>= 0) to the next double
+PPC_DI double ten_ulps(const double t) {
+  return 10.0 * (__longlong_as_double(__double_as_longlong(t) + 1) - t);
+}
+
+// Waves per block: they share one copy of the tables.
+constexpr int GROUP_WAVES = 4;
+
+// Doubles of device workspace per wave: the Jacobian accumulator of the larger
+// mechanisms and the groups' Jacobian rows in JT.
 template <int n, int G, typename JT>
 constexpr long long group_ws_doubles() {
   constexpr long long epl = (n + G - 1) / G;
-  return (long long)n * n + (epl * n * G * (long long)sizeof(JT) + 7) / 8;
+  return (long long)((n * n + 1) & ~1) + (64 / G) * ((epl * n * G * (long long)sizeof(JT) + 15) / 16 * 2);
 }
 
 // Persistent kernel: each group of G lanes integrates cells from the queue
-// until it is empty.  ws: (gridDim.x * 64 / G) group areas of
-// group_ws_doubles<NEQ, G, LU_T>() doubles.
+// until it is empty.  P.ws holds group_ws_doubles<NEQ, G, LU_T>() doubles for
+// each of P.ws_lanes / 64 waves; waves beyond that leave at once.
 template <class T, typename LU_T, int G, int OCC>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(OCC, 8)))
+__global__ void __launch_bounds__(64 * GROUP_WAVES) __attribute__((amdgpu_waves_per_eu(OCC, 8)))
 group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st) {
   using C = GroupChem<T, G>;
   using Gr = Grp<G>;
-  constexpr int n = C::n, NS = C::NS, EPL = C::EPL, SPL = C::SPL, NG = 64 / G;
-  __shared__ typename C::Shared shg[NG];
+  using PK = typename T::Packed;
+  constexpr int n = C::n, NS = C::NS, EPL = C::EPL, SPL = C::SPL, NP = C::NP;
+  __shared__ __attribute__((aligned(16))) double lds[GROUP_WAVES * C::WAREA];
+  __shared__ double lvec[GROUP_WAVES * 4 * 64 * EPL];
+  PK& pk = lds_pack<T>();
+  {
+    const int4* from = reinterpret_cast<const int4*>(&T::pack());
+    int4* to = reinterpret_cast<int4*>(&pk);
+    static_assert(sizeof(PK) % 16 == 0, "packed tables in 16-byte words");
+    for (int i = threadIdx.x; i < (int)(sizeof(PK) / 16); i += 64 * GROUP_WAVES) to[i] = from[i];
+    __syncthreads();
+  }
+  const int wv = (int)(threadIdx.x >> 6);
+  const long long wid = (long long)blockIdx.x * GROUP_WAVES + wv;
+  if (wid >= P.ws_lanes / 64) return;  // the workspace holds no more waves
   const int g = Gr::lane();
   const int gi = (int)__lane_id() / G;
-  typename C::Shared& sh = shg[gi];
-  typename C::Cache cc;
-  C::init_cache(cc, g, P.reactor_type != E_REACTOR);
-  const long long gid = (long long)blockIdx.x * NG + gi;
-  double* Jw = P.ws + gid * group_ws_doubles<n, G, LU_T>();
-  // this lane's Jacobian rows: element (e, j) at jrow[(e * n + j) * G]
-  LU_T* const jrow = reinterpret_cast<LU_T*>(Jw + (long long)n * n) + g;
-  auto Jrow = [&](int e, int j) -> LU_T& { return jrow[(e * n + j) * G]; };
+  double* const wa = lds + wv * C::WAREA;
+  double* const lv = lvec + wv * (4 * 64 * EPL) + (threadIdx.x & 63);
+  double* const sh = wa + gi * C::AREA;
+  double* const sv = sh + C::S_Q;
+  double* const sw = sv + NP;
+  LU_T* const prow = reinterpret_cast<LU_T*>(sw + NP);
+  constexpr long long GROWS = (long long)EPL * n * G;
+  constexpr long long GSTRIDE = (GROWS * (long long)sizeof(LU_T) + 15) / 16 * 16 / (long long)sizeof(LU_T);
+  double* const Jw = C::JLDS ? wa + C::J_AT : P.ws + wid * group_ws_doubles<n, G, LU_T>();
+  // the groups' Jacobian rows: element (e, j) of lane g at [(e * n + j) * G + g]
+  LU_T* const rows = reinterpret_cast<LU_T*>(P.ws + wid * group_ws_doubles<n, G, LU_T>() + ((n * n + 1) & ~1));
+  const LU_T* const jrow = rows + gi * GSTRIDE + g;
 
   const AdaptParamsDev& ap = P.adapt;
+  const bool eform = P.reactor_type == E_REACTOR;
   const double rtol = ap.rtol, atol = ap.atol;
   const double newton_tol = fmax(10 * 2.220446049250313e-16 / rtol, fmin(0.03, sqrt(rtol)));
   const double t_bound = dt;
   const long long rhs_cap = rhs_budget(ap.max_steps);
-  const int lu_batch = ap.lu_batch > 0 ? (ap.lu_batch < NG ? ap.lu_batch : NG) : NG;
-  const int lu_wait = ap.lu_wait > 0 ? ap.lu_wait : 32;
+  // LU service: half of the wave's groups waiting, or as many trips.  A
+  // factorisation for one group costs the whole wave the same, but a waiting
+  // group idles (drm19, 262144 cells, 16 lanes per cell: 87 ms serving each
+  // request at once, 79 ms at 2 groups or 2 trips, 83 ms at 4).
+  constexpr int HALF = C::NG > 1 ? C::NG / 2 : 1;
+  const int lu_batch = ap.lu_batch > 0 ? ap.lu_batch : HALF;
+  const int lu_wait = ap.lu_wait > 0 ? ap.lu_wait : HALF;
 
   // this lane's equation slots (rows i = e*G + g); `valid` marks real equations
   bool valid[EPL];
 #pragma unroll
   for (int e = 0; e < EPL; ++e) valid[e] = e * G + g < n;
   double D[AMAXORD + 3][EPL];
-  double yv[EPL], f[EPL], d[EPL], ypred[EPL], psi[EPL], scl[EPL], lus[EPL], yjac[EPL], src[SPL];
+  double yv[EPL];
+  const LaneVec<EPL> d{lv}, ypred{lv + 64 * EPL}, psi{lv + 128 * EPL}, lus{lv + 192 * EPL};
   LU_T LU[EPL][n];  // the exchanged (inverted) Newton matrix, this lane's rows
   int kstep[EPL];
   double rhoe = 0, rhoesrc = 0;
   double t = 0, t_new = 0, h_abs = 0, c = 0, dy_norm_old = -1, h0 = 0;
   int order = 1, n_equal = 0, k_newton = 0, phase = PH_F0;
-  bool lu_valid = false, current_jac = false, need_jac = false, need_lu = false;
+  int need_jac = 0;  // 1: at the initial state D[0], 2: at the predictor
+  bool lu_valid = false, current_jac = false, need_lu = false;
   int nsteps = 0, nrhs = 0, njac = 0, nlu = 0, nnewton = 0, nrej = 0, status = 0, wait = 0;
-  int cell = 0, cid = 0;
+  int cid = 0;
   bool active = false;
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) {
+    kstep[e] = 0;
+    yv[e] = 0.0;
+    ypred[e] = 0.0;
+#pragma unroll
+    for (int j = 0; j < n; ++j) LU[e][j] = LU_T(0);
+#pragma unroll
+    for (int k = 0; k < AMAXORD + 3; ++k) D[k][e] = 0.0;
+  }
 
-  // root-mean-square norm over the cell's n equations
-  auto rms = [&](const double (&x)[EPL], const double (&s)[EPL]) {
+  // sum over the cell's equations of (x / s)^2, root of its mean
+  auto sq = [&](const double (&x)[EPL], const double (&s)[EPL]) {
     double acc = 0.0;
 #pragma unroll
     for (int e = 0; e < EPL; ++e)
@@ -638,13 +834,14 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
         const double v = x[e] / s[e];
         acc += v * v;
       }
-    return sqrt(Gr::sum(acc) / n);
+    return acc;
   };
+  auto rms = [&](const double (&x)[EPL], const double (&s)[EPL]) { return sqrt(Gr::sum(sq(x, s)) / n); };
 
   auto next_cell = [&]() {
     int cl = 0;
     if (g == 0) cl = atomicAdd(q.counter, 1);
-    cell = Gr::bcast(cl, 0);
+    const int cell = Gr::bcast(cl, 0);
     active = cell < q.ncells;
     if (!active) return;
     cid = q.order ? q.order[cell] : cell;
@@ -655,13 +852,10 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
       yv[e] = D[0][e];
 #pragma unroll
       for (int k = 1; k < AMAXORD + 3; ++k) D[k][e] = 0.0;
-      f[e] = d[e] = ypred[e] = psi[e] = 0.0;
-      scl[e] = lus[e] = 1.0;
-    }
-#pragma unroll
-    for (int e = 0; e < SPL; ++e) {
-      const int k = e * G + g;
-      src[e] = k < NS ? io.ysrc[(long long)cid * NS + k] : 0.0;
+      d[e] = 0.0;
+      ypred[e] = 0.0;
+      psi[e] = 0.0;
+      lus[e] = 1.0;
     }
     rhoe = io.rX[cid];
     rhoesrc = io.rXsrc[cid];
@@ -669,8 +863,8 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
     phase = PH_F0;
     order = 1;
     n_equal = 0;
-    lu_valid = false;
-    need_jac = need_lu = false;
+    lu_valid = need_lu = false;
+    need_jac = 0;
     wait = 0;
     nsteps = nrhs = njac = nlu = nnewton = nrej = status = 0;
   };
@@ -695,311 +889,314 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
 
   next_cell();
 
-  // S^-1 (I - c J) S in LU_T with S the current error weights, factored
+  // S^-1 (I - c J) S in LU_T with S the error weights at the predictor, inverted
   auto factor = [&]() {
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
-      lus[e] = scl[e];
-      if (valid[e]) sh.v[e * G + g] = lus[e];
+      const double w = atol + rtol * fabs(ypred[e]);
+      lus[e] = w;
+      if (valid[e]) sv[e * G + g] = w;
     }
-    group_sync();
+    wave_sync();
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
+      asm volatile("" ::: "memory");  // one slot's loads at a time
       const double si = 1.0 / lus[e];
       const int i = e * G + g;
 #pragma unroll
       for (int j = 0; j < n; ++j) {
-        const double jf = valid[e] ? (double)Jrow(e, j) : 0.0;
+        const double jf = valid[e] ? (double)jrow[(e * n + j) * G] : 0.0;
         const double m = (i == j ? 1.0 : 0.0) - c * jf;
-        LU[e][j] = valid[e] ? (LU_T)(si * m * sh.v[j]) : LU_T(0);
+        LU[e][j] = valid[e] ? (LU_T)(si * m * sv[j]) : LU_T(0);
       }
     }
-    group_inv_factor<n, G, EPL, LU_T>(LU, kstep, sh.prow, g);
+    group_inv_factor<n, G, EPL, LU_T>(LU, kstep, prow, g);
     nlu++;
     lu_valid = true;
   };
 
-  auto jacobian = [&](const double (&yj)[EPL]) {
-    if (P.reactor_type == H_REACTOR)
-      C::template jacobian<1, LU_T>(sh, cc, g, Jw, yj, Jrow);
-    else
-      C::template jacobian<0, LU_T>(sh, cc, g, Jw, yj, Jrow);
-    __threadfence();
-    group_sync();
-    njac++;
-  };
-
-  auto request_jacobian = [&](const double (&yj)[EPL]) {
+  // the loop runs until every group of the wave has drained the queue: all 64
+  // lanes take part in the Jacobians
+  while (__ballot(active)) {
+    // ---- Jacobian requests, one cell at a time by the whole wave
+    unsigned long long jreq = __ballot(active && need_jac != 0 && g == 0);
+    while (__builtin_expect(jreq != 0, 0)) {
+      const int lead = __ffsll((long long)jreq) - 1, s = lead / G;
+      jreq &= jreq - 1;
+      wave_sync();
+      if (gi == s) {
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) yjac[e] = yj[e];
-    need_jac = true;
-  };
-
-  auto begin_attempt = [&]() -> bool {
-    const double min_step = 10 * fabs(nextafter(t, INFINITY) - t);
-    if (!(h_abs >= min_step)) {  // also ends a cell whose step size is NaN
-      status = -3;
-      return false;
-    }
-    t_new = t + h_abs;
-    if (t_new - t_bound > 0) {
-      t_new = t_bound;
-      group_change_D<EPL>(D, order, fabs(t_new - t) / h_abs);
-      n_equal = 0;
-      lu_valid = false;
-    }
-    const double h = t_new - t;
-    h_abs = fabs(h);
-    const double inv_alpha = 1.0 / ndf_alpha(order);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      double sum = 0.0, ps = 0.0;
-#pragma unroll
-      for (int kk = 0; kk <= AMAXORD; ++kk)
-        if (kk <= order) sum += D[kk][e];
-#pragma unroll
-      for (int kk = 1; kk <= AMAXORD; ++kk)
-        if (kk <= order) ps += D[kk][e] * bdf_gamma(kk);
-      ypred[e] = sum;
-      scl[e] = atol + rtol * fabs(sum);
-      psi[e] = ps * inv_alpha;
-      yv[e] = sum;
-      d[e] = 0.0;
-    }
-    c = h * inv_alpha;
-    if (!lu_valid) need_lu = true;
-    dy_norm_old = -1.0;
-    k_newton = 0;
-    phase = PH_NEWTON;
-    return true;
-  };
-
-  auto begin_step = [&]() -> bool {
-    if (nsteps >= ap.max_steps) {
-      status = -2;
-      return false;
-    }
-    const double min_step = 10 * fabs(nextafter(t, INFINITY) - t);
-    if (h_abs < min_step) {
-      group_change_D<EPL>(D, order, min_step / h_abs);
-      h_abs = min_step;
-      n_equal = 0;
-    }
-    current_jac = false;
-    return begin_attempt();
-  };
-
-  while (active) {
-    // ---- Jacobian / LU requests, served for the waiting groups together
-    const unsigned long long lead = __ballot(g == 0);
-    const unsigned long long waiting = __ballot(g == 0 && need_lu);
-    if (waiting) {
-      const bool stale = __ballot(g == 0 && need_lu && wait >= lu_wait) != 0;
-      if (__popcll(waiting) >= lu_batch || waiting == lead || stale) {
-        if (need_jac) {
-          jacobian(yjac);
-          need_jac = false;
-        }
-        if (need_lu) {
-          factor();
-          need_lu = false;
-          wait = 0;
-        }
+        for (int e = 0; e < EPL; ++e)
+          if (valid[e]) wa[e * G + g] = need_jac == 1 ? D[0][e] : ypred[e];
+      }
+      wave_sync();
+      if (eform)
+        C::template jacobian<0, LU_T>(pk, wa, Jw, rows + s * GSTRIDE);
+      else
+        C::template jacobian<1, LU_T>(pk, wa, Jw, rows + s * GSTRIDE);
+      __threadfence_block();
+      wave_sync();
+      if (gi == s) {
+        need_jac = 0;
+        njac++;
       }
     }
+    // ---- LU requests, served for the waiting groups together
+    const unsigned long long lead = __ballot(active && g == 0);
+    const unsigned long long waiting = __ballot(active && g == 0 && need_lu);
+    if (waiting) {
+      const bool stale = __ballot(active && need_lu && wait >= lu_wait) != 0;
+      if ((__popcll(waiting) >= lu_batch || waiting == lead || stale) && active && need_lu) {
+        factor();
+        need_lu = false;
+        wait = 0;
+      }
+    }
+    if (!active) continue;
     if (need_lu) {  // not served yet: no RHS, no Newton iteration this trip
       ++wait;
       continue;
     }
+    // what this trip leaves to do: a step attempt (of a new step or a repeated
+    // one) after scaling D by a step-size ratio, or the end of the cell
+    bool attempt = false, new_step = false, finish = false;
+    double fac = 1.0;
     if (nrhs >= rhs_cap) {  // out of budget: the cell fails with the step-limit status
       status = -2;
-      finish_cell();
-      continue;
-    }
-    // ---- the one RHS evaluation of this trip
-    const double t_eval = (phase == PH_F0) ? 0.0 : (phase == PH_F1 ? h0 : t_new);
-    C::rhs(sh, cc, g, P.reactor_type, t_eval, yv, src, rhoe, rhoesrc, f);
-    nrhs++;
-    bool ok = true;
-    if (phase == PH_F0) {
-      // f0 = f(y0): initial step size (Hairer, Norsett & Wanner I, II.4)
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) {
-        D[1][e] = f[e];  // f0 kept in D[1] until h is known
-        scl[e] = atol + fabs(D[0][e]) * rtol;
-      }
-      if (ap.first_step > 0) {
-        h_abs = ap.first_step;
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) {
-          D[1][e] *= h_abs;
-          yv[e] = D[0][e];
-        }
-        request_jacobian(yv);
-        ok = begin_step();
-      } else {
-        const double d0 = rms(D[0], scl), d1 = rms(f, scl);
-        h0 = (d0 < 1e-5 || d1 < 1e-5) ? 1e-6 : 0.01 * d0 / d1;
-        h0 = fmin(h0, t_bound);
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) yv[e] = D[0][e] + h0 * f[e];
-        phase = PH_F1;
-      }
-    } else if (phase == PH_F1) {
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) d[e] = f[e] - D[1][e];
-      const double d1 = rms(D[1], scl);
-      const double d2 = rms(d, scl) / h0;
-      const double h1 = (d1 <= 1e-15 && d2 <= 1e-15) ? fmax(1e-6, h0 * 1e-3) : sqrt(0.01 / fmax(d1, d2));
-      h_abs = fmin(fmin(100 * h0, h1), t_bound);
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) {
-        D[1][e] *= h_abs;
-        yv[e] = D[0][e];
-      }
-      request_jacobian(yv);
-      ok = begin_step();
+      finish = true;
     } else {
-      // one modified-Newton iteration with f = f(t_new, yv)
-      nnewton++;
-      double bad = 0.0;
+      // ---- the one RHS evaluation of this trip
+      const double t_eval = (phase == PH_F0) ? 0.0 : (phase == PH_F1 ? h0 : t_new);
+      double f[EPL], src[SPL];
 #pragma unroll
-      for (int e = 0; e < EPL; ++e)
-        if (valid[e] && !isfinite(f[e])) bad = 1.0;
-      const bool finite = Gr::max(bad) == 0.0;
-      bool failed = !finite, converged = false;
-      const int n_iter = k_newton + 1;
-      if (finite) {
-        double b[EPL], dy[EPL];
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) b[e] = valid[e] ? (c * f[e] - psi[e] - d[e]) / lus[e] : 0.0;
-        group_inv_solve<n, G, EPL, LU_T>(LU, kstep, sh.v, sh.w, g, b, dy);
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) dy[e] *= lus[e];
-        const double dy_norm = rms(dy, scl);
-        const double rate = dy_norm_old < 0 ? -1.0 : dy_norm / dy_norm_old;
-        if (rate >= 0 && (rate >= 1 || pow(rate, 4 - k_newton) / (1 - rate) * dy_norm > newton_tol)) {
-          failed = true;
-        } else {
-#pragma unroll
-          for (int e = 0; e < EPL; ++e) {
-            yv[e] += dy[e];
-            d[e] += dy[e];
-          }
-          if (dy_norm == 0 || (rate >= 0 && rate / (1 - rate) * dy_norm < newton_tol)) {
-            converged = true;
-          } else {
-            dy_norm_old = dy_norm;
-            k_newton++;
-            if (k_newton == 4) failed = true;
-          }
-        }
+      for (int e = 0; e < SPL; ++e) {
+        const int k = e * G + g;
+        src[e] = k < NS ? io.ysrc[(long long)cid * NS + k] : 0.0;
       }
-      if (failed) {
-        if (!current_jac) {
-          // refresh the Jacobian at the predictor and retry the same step
-          request_jacobian(ypred);
-          current_jac = true;
-          need_lu = true;
+      C::rhs(pk, sh, g, eform, t_eval, yv, src, rhoe, rhoesrc, f);
+      nrhs++;
+      double scl[EPL];
+      if (__builtin_expect(phase != PH_NEWTON, 0)) {
+        // initial step size (Hairer, Norsett & Wanner I, II.4)
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) scl[e] = atol + fabs(D[0][e]) * rtol;
+        if (phase == PH_F0) {
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) D[1][e] = f[e];  // f0 kept in D[1] until h is known
+          if (ap.first_step > 0) {
+            h_abs = ap.first_step;
+            attempt = true;
+          } else {
+            const double d0 = rms(D[0], scl), d1 = rms(f, scl);
+            h0 = (d0 < 1e-5 || d1 < 1e-5) ? 1e-6 : 0.01 * d0 / d1;
+            h0 = fmin(h0, t_bound);
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) yv[e] = D[0][e] + h0 * f[e];
+            phase = PH_F1;
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) f[e] -= D[1][e];
+          const double d1 = rms(D[1], scl);
+          const double d2 = rms(f, scl) / h0;
+          const double h1 = (d1 <= 1e-15 && d2 <= 1e-15) ? fmax(1e-6, h0 * 1e-3) : sqrt(0.01 / fmax(d1, d2));
+          h_abs = fmin(fmin(100 * h0, h1), t_bound);
+          attempt = true;
+        }
+        if (attempt) {
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) D[1][e] *= h_abs;
+          need_jac = 1;
+          new_step = true;
+        }
+      } else {
+        // one modified-Newton iteration with f = f(t_new, yv)
+        nnewton++;
+        bool bad = false;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) bad = bad || (valid[e] && !isfinite(f[e]));
+        const bool finite = !Gr::any(bad);
+        bool failed = !finite, converged = false;
+        const int n_iter = k_newton + 1;
+        if (finite) {
+          double b[EPL], dy[EPL];
 #pragma unroll
           for (int e = 0; e < EPL; ++e) {
-            yv[e] = ypred[e];
-            d[e] = 0.0;
+            b[e] = valid[e] ? (c * f[e] - psi[e] - d[e]) / lus[e] : 0.0;
+            scl[e] = atol + rtol * fabs(ypred[e]);
           }
-          dy_norm_old = -1.0;
-          k_newton = 0;
-        } else {
-          h_abs *= 0.5;
-          group_change_D<EPL>(D, order, 0.5);
-          n_equal = 0;
-          lu_valid = false;
-          nrej++;
-          ok = begin_attempt();
-        }
-      } else if (converged) {
-        const double safety = 0.9 * 9.0 / (double)(8 + n_iter);
-        double err[EPL];
+          group_inv_solve<n, G, EPL, LU_T>(LU, kstep, sv, sw, g, b, dy);
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) {
-          scl[e] = atol + rtol * fabs(yv[e]);
-          err[e] = ndf_econst(order) * d[e];
-        }
-        const double error_norm = rms(err, scl);
-        if (error_norm > 1) {
-          const double fac = fmax(0.2, safety * pow(error_norm, -1.0 / (order + 1)));
-          h_abs *= fac;
-          group_change_D<EPL>(D, order, fac);
-          n_equal = 0;
-          nrej++;
-          ok = begin_attempt();
-        } else {
-          // accept: D[order+2] = d - D[order+1]; D[order+1] = d; D[k] += D[k+1], k = order..0
-          nsteps++;
-          n_equal++;
-          t = t_new;
+          for (int e = 0; e < EPL; ++e) dy[e] *= lus[e];
+          const double dy_norm = rms(dy, scl);
+          const double rate = dy_norm_old < 0 ? -1.0 : dy_norm / dy_norm_old;
+          double left = rate;  // rate^(4 - k_newton)
+          for (int i = k_newton; i < 3; ++i) left *= rate;
+          if (rate >= 0 && (rate >= 1 || left / (1 - rate) * dy_norm > newton_tol)) {
+            failed = true;
+          } else {
 #pragma unroll
-          for (int e = 0; e < EPL; ++e) {
-#pragma unroll
-            for (int kk = AMAXORD + 2; kk >= 1; --kk) {
-              if (kk == order + 2) D[kk][e] = d[e] - D[kk - 1][e];
-              if (kk == order + 1) D[kk][e] = d[e];
+            for (int e = 0; e < EPL; ++e) {
+              yv[e] += dy[e];
+              d[e] += dy[e];
             }
-#pragma unroll
-            for (int kk = AMAXORD; kk >= 0; --kk)
-              if (kk <= order) D[kk][e] += D[kk + 1][e];
+            if (dy_norm == 0 || (rate >= 0 && rate / (1 - rate) * dy_norm < newton_tol)) {
+              converged = true;
+            } else {
+              dy_norm_old = dy_norm;
+              k_newton++;
+              if (k_newton == 4) failed = true;
+            }
           }
-          if (n_equal >= order + 1) {
-            double em = INFINITY, ep = INFINITY;
-            if (order > 1) {
+        }
+        if (failed) {
+          if (!current_jac) {
+            // refresh the Jacobian at the predictor and retry the same step
+            need_jac = 2;
+            current_jac = true;
+            need_lu = true;
 #pragma unroll
-              for (int e = 0; e < EPL; ++e) {
-                double v = 0.0;
-#pragma unroll
-                for (int kk = 0; kk <= AMAXORD; ++kk)
-                  if (kk == order) v = D[kk][e];
-                err[e] = ndf_econst(order - 1) * v;
-              }
-              em = rms(err, scl);
+            for (int e = 0; e < EPL; ++e) {
+              yv[e] = ypred[e];
+              d[e] = 0.0;
             }
-            if (order < AMAXORD) {
-#pragma unroll
-              for (int e = 0; e < EPL; ++e) {
-                double v = 0.0;
-#pragma unroll
-                for (int kk = 0; kk < AMAXORD + 3; ++kk)
-                  if (kk == order + 2) v = D[kk][e];
-                err[e] = ndf_econst(order + 1) * v;
-              }
-              ep = rms(err, scl);
-            }
-            const double norms[3] = {em, error_norm, ep};
-            double best = -1.0;
-            int delta = 0;
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-              const double fct = (norms[i] == 0.0) ? INFINITY : pow(norms[i], -1.0 / (order + i));
-              if (fct > best) {
-                best = fct;
-                delta = i - 1;
-              }
-            }
-            order += delta;
-            const double fac = fmin(10.0, safety * best);
-            h_abs *= fac;
-            group_change_D<EPL>(D, order, fac);
+            dy_norm_old = -1.0;
+            k_newton = 0;
+          } else {
+            fac = 0.5;
+            h_abs *= 0.5;
             n_equal = 0;
             lu_valid = false;
+            nrej++;
+            attempt = true;
           }
-          if (t < t_bound) {
-            ok = begin_step();
+        } else if (converged) {
+          const double safety = 0.9 * 9.0 / (double)(8 + n_iter);
+          double err[EPL];
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) {
+            scl[e] = atol + rtol * fabs(yv[e]);
+            err[e] = ndf_econst(order) * d[e];
+          }
+          const double error_norm = rms(err, scl);
+          attempt = true;
+          if (error_norm > 1) {
+            fac = fmax(0.2, safety * exp(-log(error_norm) / (order + 1)));
+            h_abs *= fac;
+            n_equal = 0;
+            nrej++;
           } else {
-            finish_cell();
-            continue;
+            // accept: D[order+2] = d - D[order+1]; D[order+1] = d; D[k] += D[k+1], k = order..0
+            nsteps++;
+            n_equal++;
+            t = t_new;
+            new_step = true;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) {
+#pragma unroll
+              for (int kk = AMAXORD + 2; kk >= 1; --kk) {
+                if (kk == order + 2) D[kk][e] = d[e] - D[kk - 1][e];
+                if (kk == order + 1) D[kk][e] = d[e];
+              }
+#pragma unroll
+              for (int kk = AMAXORD; kk >= 0; --kk)
+                if (kk <= order) D[kk][e] += D[kk + 1][e];
+            }
+            if (n_equal >= order + 1) {
+              double err2[EPL];
+              const double cm = order > 1 ? ndf_econst(order - 1) : 0.0;
+              const double cp = order < AMAXORD ? ndf_econst(order + 1) : 0.0;
+#pragma unroll
+              for (int e = 0; e < EPL; ++e) {
+                double vm = 0.0, vp = 0.0;
+#pragma unroll
+                for (int kk = 0; kk < AMAXORD + 3; ++kk) {
+                  if (kk == order) vm = D[kk][e];
+                  if (kk == order + 2) vp = D[kk][e];
+                }
+                err[e] = cm * vm;
+                err2[e] = cp * vp;
+              }
+              const double sm = Gr::sum(sq(err, scl)), sp = Gr::sum(sq(err2, scl));
+              const double norms[3] = {order > 1 ? sqrt(sm / n) : INFINITY, error_norm,
+                                       order < AMAXORD ? sqrt(sp / n) : INFINITY};
+              double best = -1.0;
+              int delta = 0;
+#pragma unroll
+              for (int i = 0; i < 3; ++i) {
+                const double fct = (norms[i] == 0.0) ? INFINITY : exp(-log(norms[i]) / (order + i));
+                if (fct > best) {
+                  best = fct;
+                  delta = i - 1;
+                }
+              }
+              order += delta;
+              fac = fmin(10.0, safety * best);
+              h_abs *= fac;
+              n_equal = 0;
+              lu_valid = false;
+            }
+            if (!(t < t_bound)) {
+              attempt = false;
+              finish = true;
+              // D[0] is the result whatever the next step size would be
+              fac = 1.0;
+            }
           }
         }
       }
     }
-    if (!ok) finish_cell();  // failed cell: store with the negative status
+    if (attempt) {
+      const double min_step = ten_ulps(t);
+      if (new_step) {
+        if (nsteps >= ap.max_steps) {
+          status = -2;
+          finish = true;
+        } else if (h_abs < min_step) {
+          fac *= min_step / h_abs;
+          h_abs = min_step;
+          n_equal = 0;
+        }
+        current_jac = false;
+      }
+      if (!finish && !(h_abs >= min_step)) {  // also ends a cell whose step size is NaN
+        status = -3;
+        finish = true;
+      }
+      if (!finish) {
+        t_new = t + h_abs;
+        if (t_new - t_bound > 0) {
+          t_new = t_bound;
+          fac *= fabs(t_new - t) / h_abs;
+          n_equal = 0;
+          lu_valid = false;
+        }
+        const double h = t_new - t;
+        h_abs = fabs(h);
+        if (fac != 1.0) group_change_D<EPL>(D, order, fac);
+        const double inv_alpha = 1.0 / ndf_alpha(order);
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) {
+          double sum = 0.0, ps = 0.0;
+#pragma unroll
+          for (int kk = 0; kk <= AMAXORD; ++kk)
+            if (kk <= order) {
+              sum += D[kk][e];
+              if (kk > 0) ps += D[kk][e] * bdf_gamma(kk);
+            }
+          ypred[e] = sum;
+          psi[e] = ps * inv_alpha;
+          yv[e] = sum;
+          d[e] = 0.0;
+        }
+        c = h * inv_alpha;
+        if (!lu_valid) need_lu = true;
+        dy_norm_old = -1.0;
+        k_newton = 0;
+        phase = PH_NEWTON;
+      }
+    }
+    if (__builtin_expect(finish, 0)) finish_cell();
   }
 }
 

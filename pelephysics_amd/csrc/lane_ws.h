@@ -97,11 +97,11 @@ constexpr bool group_ok() {
   return has_table<M>::value && !has_qss<M>::value && M::NEQ <= 3 * G && G <= 2 * M::NEQ;
 }
 
-// Device workspace of one group: the n x n FP64 Jacobian accumulator and its
-// rows (at most FP64)
+// Device workspace of one wave of the group kernel (doubles, at most): an n x n
+// FP64 Jacobian accumulator and the Jacobian rows of its 64 / G groups.
 template <int n, int G>
-constexpr long long group_ws_doubles_max() {
-  return (long long)n * n + (long long)((n + G - 1) / G) * n * G;
+constexpr long long group_wave_doubles() {
+  return (long long)n * n + 1 + (64 / G) * ((long long)((n + G - 1) / G) * n * G + 1);
 }
 
 // Workspace rows per lane (doubles, 64-lane blocks as lane_ws) of the group
@@ -110,10 +110,10 @@ template <class M>
 long long group_ws_rows(int cells_per_wave) {
   constexpr int n = M::NEQ;
   switch (cells_per_wave) {
-    case 8: return group_ok<M, 8>() ? (8 * group_ws_doubles_max<n, 8>() + 63) / 64 : 0;
-    case 4: return group_ok<M, 16>() ? (4 * group_ws_doubles_max<n, 16>() + 63) / 64 : 0;
-    case 2: return group_ok<M, 32>() ? (2 * group_ws_doubles_max<n, 32>() + 63) / 64 : 0;
-    case 1: return group_ok<M, 64>() ? (group_ws_doubles_max<n, 64>() + 63) / 64 : 0;
+    case 8: return group_ok<M, 8>() ? (group_wave_doubles<n, 8>() + 63) / 64 : 0;
+    case 4: return group_ok<M, 16>() ? (group_wave_doubles<n, 16>() + 63) / 64 : 0;
+    case 2: return group_ok<M, 32>() ? (group_wave_doubles<n, 32>() + 63) / 64 : 0;
+    case 1: return group_ok<M, 64>() ? (group_wave_doubles<n, 64>() + 63) / 64 : 0;
     default: return 0;
   }
 }

@@ -21,8 +21,6 @@ struct MechLauncher {
   // batched (persistent, work-queue) forms; grid = number of 64-lane blocks
   hipError_t (*batched_1d)(int mode, const ReactParamsDev& P, double* y, const double* ysrc, double* rX,
                            const double* rXsrc, double dt, QueueArgs q, CellStats st, hipStream_t s);
-  hipError_t (*batched_box)(int mode, const ReactParamsDev& P, const BoxArgs& b, double dt, QueueArgs q,
-                            CellStats st, hipStream_t s);
   // discrete adjoint of the fixed-step BDF (table-driven mechanisms only)
   hipError_t (*adjoint_1d)(const ReactParamsDev& P, const AdjointArgs& a, hipStream_t s);
   // workspace rows per lane a mode needs (lane_ws.h); 0: none
@@ -57,23 +55,11 @@ hipError_t launch_box_mode(const ReactParamsDev& P, const BoxArgs& b, double dt,
 template <class M, int MODE>
 hipError_t batched_1d_mode(const ReactParamsDev& P, double* y, const double* ysrc, double* rX, const double* rXsrc,
                            double dt, QueueArgs q, CellStats st, hipStream_t s);
-template <class M, int MODE>
-hipError_t batched_box_mode(const ReactParamsDev& P, const BoxArgs& b, double dt, QueueArgs q, CellStats st,
-                            hipStream_t s);
-
 template <class M>
 hipError_t launch_batched_1d(int mode, const ReactParamsDev& P, double* y, const double* ysrc, double* rX,
                              const double* rXsrc, double dt, QueueArgs q, CellStats st, hipStream_t s) {
   if (mode == MODE_BATCHED_MIXED) return batched_1d_mode<M, MODE_BATCHED_MIXED>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
   if (mode == MODE_BATCHED_FP64) return batched_1d_mode<M, MODE_BATCHED_FP64>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
-  return hipErrorInvalidValue;
-}
-
-template <class M>
-hipError_t launch_batched_box(int mode, const ReactParamsDev& P, const BoxArgs& b, double dt, QueueArgs q,
-                              CellStats st, hipStream_t s) {
-  if (mode == MODE_BATCHED_MIXED) return batched_box_mode<M, MODE_BATCHED_MIXED>(P, b, dt, q, st, s);
-  if (mode == MODE_BATCHED_FP64) return batched_box_mode<M, MODE_BATCHED_FP64>(P, b, dt, q, st, s);
   return hipErrorInvalidValue;
 }
 
@@ -110,7 +96,7 @@ hipError_t launch_box(int mode, const ReactParamsDev& P, const BoxArgs& b, doubl
     static const MechLauncher L = {#NAME, TYPE::NS, TYPE::NR,                                  \
                                    1,                                                          \
                                    &launch_1d<TYPE>, &launch_box<TYPE>,                        \
-                                   &launch_batched_1d<TYPE>, &launch_batched_box<TYPE>,        \
+                                   &launch_batched_1d<TYPE>,                                   \
                                    &launch_adjoint<TYPE>, &integrator_ws_rows<TYPE>,           \
                                    &group_ws_rows<TYPE>,                                       \
                                    &launch_flatten<TYPE>, &launch_mech_eval<TYPE>};            \

@@ -67,16 +67,16 @@ hipError_t launch_box_mode(const ReactParamsDev& P, const BoxArgs& b, double dt,
   return hipGetLastError();
 }
 
-// Persistent launch: as many 64-lane blocks as can be resident at once (never
-// more than `lanes` / 64 needs); lanes or waves take cells from the queue.
+// Persistent launch: as many blocks as can be resident at once (never more than
+// `lanes` needs); lanes or waves take cells from the queue.
 template <class K>
-int resident_blocks(K kernel, long long lanes) {
+int resident_blocks(K kernel, long long lanes, int block = 64) {
   int dev = 0, ncu = 0, per_cu = 0;
   if (hipGetDevice(&dev) != hipSuccess) return -1;
   if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return -1;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, 0) != hipSuccess) return -1;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, 0) != hipSuccess) return -1;
   if (per_cu < 1) per_cu = 1;
-  const long long need = (lanes + 63) / 64;
+  const long long need = (lanes + block - 1) / block;
   const long long blocks = (long long)ncu * per_cu;
   return (int)(blocks < need ? blocks : need);
 }
@@ -97,22 +97,24 @@ int batched_grid(K kernel, const ReactParamsDev& P, const QueueArgs& q) {
 }
 
 // The group kernel (group_bdf.h) with G lanes per cell: a persistent grid of
-// every resident block, at most q.max_blocks and at most the blocks the
-// workspace holds (group_ws_rows rows of 64 lanes per block).
+// every resident block of GROUP_WAVES waves, at most q.max_blocks waves and the
+// waves the workspace holds (group_ws_rows rows of 64 lanes per wave).
 template <class T, typename LU_T, int G>
 hipError_t launch_group(const ReactParamsDev& P, double* y, const double* ysrc, double* rX, const double* rXsrc,
                         double dt, QueueArgs q, CellStats st, hipStream_t s) {
-  static_assert(group_ws_doubles<T::NEQ, G, LU_T>() <= group_ws_doubles_max<T::NEQ, G>(), "workspace layout");
-  // registers of the LU rows: above ~100 VGPRs hold the build to one wave per SIMD
+  static_assert(group_ws_doubles<T::NEQ, G, LU_T>() <= group_wave_doubles<T::NEQ, G>(), "workspace layout");
+  // registers of the inverse's rows: above ~100 VGPRs hold the build to one wave per SIMD
   constexpr int lu_vgprs = (int)(((T::NEQ + G - 1) / G) * T::NEQ * sizeof(LU_T) / 4);
   auto k = group_bdf_kernel<T, LU_T, G, (lu_vgprs > 100 ? 1 : 2)>;
-  int grid = resident_blocks(k, (long long)q.ncells * G);
+  int grid = resident_blocks(k, (long long)q.ncells * G, 64 * GROUP_WAVES);
   if (grid < 0) return hipErrorInvalidDevice;
-  if (q.max_blocks > 0 && q.max_blocks < grid) grid = q.max_blocks;
   if (!P.ws || P.ws_lanes < 64 || P.ws_lanes % 64 != 0) return hipErrorInvalidValue;
-  if (P.ws_lanes / 64 < grid) grid = (int)(P.ws_lanes / 64);
+  long long waves = P.ws_lanes / 64;
+  if (q.max_blocks > 0 && q.max_blocks < waves) waves = q.max_blocks;
+  const int most = (int)((waves + GROUP_WAVES - 1) / GROUP_WAVES);
+  if (most < grid) grid = most;
   IO1D io{y, ysrc, rX, rXsrc};
-  hipLaunchKernelGGL(k, dim3(grid), dim3(64), 0, s, P, io, dt, q, st);
+  hipLaunchKernelGGL(k, dim3(grid), dim3(64 * GROUP_WAVES), 0, s, P, io, dt, q, st);
   return hipGetLastError();
 }
 
@@ -145,31 +147,19 @@ template <class M, int MODE>
 hipError_t batched_1d_mode(const ReactParamsDev& P, double* y, const double* ysrc, double* rX, const double* rXsrc,
                            double dt, QueueArgs q, CellStats st, hipStream_t s) {
   using LU_T = typename std::conditional<MODE == MODE_BATCHED_MIXED, float, double>::type;
-  if (P.adapt.group > 0) return batched_group<M, LU_T>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
-  {
+  if constexpr (!has_qss<M>::value) {
+    // a group of lanes per cell at every size (group_bdf.h): one cell per lane
+    // measured 3.2 times as long on 64^3 drm19 cells and 16 to 115 times on
+    // calls that do not fill the chip (figures there)
+    return batched_group<M, LU_T>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
+  } else {
     auto k = P.adapt.lane_occ == 1 ? batched_kernel<M, LU_T, IO1D, 1> : batched_kernel<M, LU_T, IO1D, 2>;
     const int grid = batched_grid<M, MODE>(k, P, q);
     if (grid < 0) return grid == -2 ? hipErrorInvalidValue : hipErrorInvalidDevice;
     IO1D io{y, ysrc, rX, rXsrc};
     hipLaunchKernelGGL(k, dim3(grid), dim3(64), 0, s, P, io, dt, q, st);
+    return hipGetLastError();
   }
-  return hipGetLastError();
-}
-
-template <class M, int MODE>
-hipError_t batched_box_mode(const ReactParamsDev& P, const BoxArgs& b, double dt, QueueArgs q, CellStats st,
-                            hipStream_t s) {
-  using LU_T = typename std::conditional<MODE == MODE_BATCHED_MIXED, float, double>::type;
-  {
-    // built at 2 waves per SIMD only: the 1-wave build of the table-driven
-    // drm19 box kernel returned failed cells, so 1-wave runs take the flat route
-    auto k = batched_kernel<M, LU_T, IOBox, 2>;
-    const int grid = batched_grid<M, MODE>(k, P, q);
-    if (grid < 0) return grid == -2 ? hipErrorInvalidValue : hipErrorInvalidDevice;
-    IOBox io{b};
-    hipLaunchKernelGGL(k, dim3(grid), dim3(64), 0, s, P, io, dt, q, st);
-  }
-  return hipGetLastError();
 }
 
 template <class M>
@@ -264,7 +254,5 @@ hipError_t launch_mech_eval(int what, const double* sc, const double* T, int nce
   namespace ppc {                                                                                      \
   template hipError_t batched_1d_mode<TYPE, MODE>(const ReactParamsDev&, double*, const double*,  \
                                                         double*, const double*, double, QueueArgs,      \
-                                                        CellStats, hipStream_t);                       \
-  template hipError_t batched_box_mode<TYPE, MODE>(const ReactParamsDev&, const BoxArgs&, double,  \
-                                                         QueueArgs, CellStats, hipStream_t);           \
+                                                        CellStats, hipStream_t);  \
   }

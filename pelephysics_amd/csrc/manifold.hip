@@ -29,9 +29,6 @@ hipError_t no_batched_1d(int, const ReactParamsDev&, double*, const double*, dou
                          QueueArgs, CellStats, hipStream_t) {
   return hipErrorInvalidValue;
 }
-hipError_t no_batched_box(int, const ReactParamsDev&, const BoxArgs&, double, QueueArgs, CellStats, hipStream_t) {
-  return hipErrorInvalidValue;
-}
 hipError_t no_adjoint(const ReactParamsDev&, const AdjointArgs&, hipStream_t) { return hipErrorNotSupported; }
 long long no_ws(int) { return 0; }
 long long no_group(int) { return 0; }
@@ -41,7 +38,7 @@ hipError_t no_eval(int, const double*, const double*, int, double*, hipStream_t)
 template <int D>
 const MechLauncher* man_launcher() {
   static const MechLauncher L = {"Manifold", D + 1, 0, 0, &man_1d<D>, &man_box<D>, &no_batched_1d,
-                                 &no_batched_box, &no_adjoint, &no_ws, &no_group, &no_flatten, &no_eval};
+                                 &no_adjoint, &no_ws, &no_group, &no_flatten, &no_eval};
   return &L;
 }
 

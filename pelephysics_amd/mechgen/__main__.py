@@ -1,12 +1,13 @@
 """Regenerate mechanism tables and HIP headers from the reference YAML files.
 
-    python -m pelephysics_amd.mechgen [--ref /root/reference] [mech ...]
+    python -m pelephysics_amd.mechgen [--ref /root/reference] [--tables] [mech ...]
 
 Writes ``pelephysics_amd/mechanisms/<mech>.json`` (normalised parameter
 tables, read by the oracle and the tests) and
 ``pelephysics_amd/csrc/mech/<mech>.h`` (unrolled device code, small
 mechanisms only) and
-``pelephysics_amd/csrc/tab/<mech>.h`` (constant-memory tables).
+``pelephysics_amd/csrc/tab/<mech>.h`` (constant-memory tables); with --tables only the
+last, from the committed JSON.
 """
 import argparse
 import os
@@ -48,6 +49,14 @@ def generate(mechs, ref="/root/reference"):
     return out
 
 
+def retable(mechs):
+    """Write csrc/tab/<mech>.h again from the committed mechanism data."""
+    for name in mechs:
+        with open(os.path.join(PKG, "csrc", "tab", f"{name}.h"), "w") as f:
+            f.write(emit_tables(load(name), f"Mechanisms/{name}/{source(name)}"))
+    return list(mechs)
+
+
 def load(name: str) -> Mechanism:
     with open(os.path.join(PKG, "mechanisms", f"{name}.json")) as f:
         return Mechanism.from_json(f.read())
@@ -56,6 +65,7 @@ def load(name: str) -> Mechanism:
 if __name__ == "__main__":
     ap = argparse.ArgumentParser()
     ap.add_argument("--ref", default="/root/reference")
+    ap.add_argument("--tables", action="store_true")
     ap.add_argument("mechs", nargs="*", default=DEFAULT_MECHS)
     a = ap.parse_args()
-    print(generate(a.mechs, a.ref))
+    print(retable(a.mechs) if a.tables else generate(a.mechs, a.ref))

@@ -24,6 +24,18 @@ no per-reaction branching.  For every reaction:
   reactions in table order), for kernels that form each species' production
   rate in its own lane.
 
+``kPack`` is a second, compact copy of what one right-hand side reads, laid out
+for the group kernels (group_bdf.h), which copy it to LDS as it stands: per
+species the NASA7 coefficients of both ranges, per reaction 32 bytes (rate,
+species as bytes with NX for an unused place, refC power, flags), the third
+bodies and falloff parameters, and the net stoichiometry by species cut into
+chunks of 8 terms (``ch``: reaction in 12 bits, coefficient + 8 in 4 bits, an
+unused place is reaction NR with coefficient 0; ``spCh``: first chunk of each
+species), so that the lanes of a group share the long rows.  Its reaction
+order is the table order with the reversible elementary reactions first
+(``perm``: position in the tables above), so that a wave's lanes agree on
+whether there is a reverse rate.
+
 QSS mechanisms (``NQ`` > 0) index their quasi-steady-state species NS..NS+NQ-1
 in ``rxR``/``rxP`` and the thermo tables; ``rxNet`` and ``spPtr`` keep the
 transported species only.  Their extra tables:
@@ -140,6 +152,79 @@ def qss_elimination(m: Mechanism):
     return terms, slot, init, lu, fs, bs
 
 
+CHUNK = 8
+
+
+def emit_pack(w, m: Mechanism, R: List[Reaction], n_el: int) -> None:
+    """The Packed struct and its values (see the module's docstring); R is in
+    table order, its first n_el reactions elementary."""
+    ns, nx, nr = m.n_species, m.n_species + m.n_qss, len(R)
+    if nx > 254 or nr > 4095:
+        raise ValueError("mechanism too large for the packed tables")
+
+    def shape(j):
+        r = R[j]
+        return (0 if r.reversible else 1, sum(r.reactants.values()) > 2, sum(r.products.values()) > 2, j)
+
+    perm = sorted(range(n_el), key=shape) + list(range(n_el, nr))
+    rx, rx_eff, effk, effv = [], [], [], []
+    for j in perm:
+        r = R[j]
+        rr = [nx if k < 0 else k for k in _expand(r.reactants)]
+        pp = [nx if k < 0 else k for k in (_expand(r.products) if r.reversible else [-1] * MAXR)]
+        d = int(round(r.delta_order()))
+        if r.reversible and abs(d) > 100:
+            raise ValueError("reaction order out of range")
+        flags = (1 if r.reversible else 0) + (2 if r.fwd_removed else 0)
+        rx.append(f"{{{_f(r.rate.A)}, {_f(r.rate.b)}, {_f(r.rate.EaR)}, "
+                  f"{{{', '.join(map(str, rr))}}}, {{{', '.join(map(str, pp))}}}, {d if r.reversible else 0}, {flags}}}")
+    for r in R[n_el:]:
+        e = [(k, v - 1.0) for k, v in sorted(r.efficiencies.items()) if v != 1.0]
+        rx_eff.append(f"{{{len(effk)}, {len(e)}}}")
+        effk += [str(k) for k, _ in e]
+        effv += [_f(v) for _, v in e]
+    fo = []
+    for r in R:
+        if r.kind != "falloff":
+            continue
+        t = list(r.troe or []) + [0.0] * 4
+        fo.append("{" + ", ".join(_f(x) for x in (r.low.A, r.low.b, r.low.EaR, t[0], t[1], t[2], t[3],
+                                                  1.0 if r.troe and len(r.troe) == 4 else 0.0)) + "}")
+    sp = [f"{{{{{', '.join(_f(x) for x in s.low)}}}, {_f(s.tmid)}, {{{', '.join(_f(x) for x in s.high)}}}, {_f(s.imw)}}}"
+          for s in m.all_species]
+    pos = {j: i for i, j in enumerate(perm)}
+    chunks, first = [], [0]
+    for k in range(ns):
+        terms = []
+        for j, r in enumerate(R):
+            v = r.net_stoich().get(k, 0.0)
+            if v:
+                if v != int(v) or not -8 <= v <= 7:
+                    raise ValueError("net coefficient out of range")
+                terms.append((pos[j], int(v)))
+        terms.sort()
+        for i in range(0, len(terms), CHUNK):
+            c = terms[i:i + CHUNK] + [(nr, 0)] * (CHUNK - len(terms[i:i + CHUNK]))
+            chunks.append("{" + ", ".join(str(((v + 8) << 12) | j) for j, v in c) + "}")
+        first.append(len(chunks))
+    rows = [("PackSp", "sp", sp), ("PackRx", "rx", rx), ("PackFo", "fo", fo or ["{}"]),
+            ("PackCh", "ch", chunks), ("double", "mw", [_f(s.mw) for s in m.species]),
+            ("double", "effV", effv or ["0.0"]), ("PackEff", "eff", rx_eff or ["{0, 0}"]),
+            ("unsigned short", "spCh", list(map(str, first))), ("unsigned short", "perm", list(map(str, perm))),
+            ("unsigned char", "effK", effk or ["0"])]
+    w("struct alignas(16) Packed {")
+    for t, nm, v in rows:
+        w(f"  {t} {nm}[{len(v)}];")
+    w("};")
+    w("")
+    w("static __constant__ Packed kPack = {")
+    for _, nm, v in rows:
+        w(f"    /* {nm} */ {{{', '.join(v)}}},")
+    w("};")
+    w("")
+    w(f"constexpr int kChunks = {len(chunks)};")
+
+
 def emit(m: Mechanism, source: str) -> str:
     order = ordered(m)
     R = [m.reactions[j] for j in order]
@@ -153,7 +238,7 @@ def emit(m: Mechanism, source: str) -> str:
     w = L.append
     w(f"// Generated by pelephysics_amd.mechgen.emit_tables from {source}. Do not edit.")
     w("#pragma once")
-    w('#include "../ppc_common.h"')
+    w('#include "../pack.h"')
     w("")
     w("namespace ppc {")
     w("namespace tab {")
@@ -283,6 +368,8 @@ def emit(m: Mechanism, source: str) -> str:
         qss_counts = {"NQR": len(qrx), "NSLOT": len(slot), "NLU": len(lu), "NFS": len(fs)}
     tab.emit(w, "Tables")
     w("")
+    emit_pack(w, m, R, n_el)
+    w("")
     w("}  // namespace")
     w("")
     w(f"struct {m.name} {{")
@@ -293,6 +380,9 @@ def emit(m: Mechanism, source: str) -> str:
     w("  static constexpr int " + ", ".join(f"{k} = {v}" for k, v in qss_counts.items()) + ";")
     w(f"  static constexpr int N_EL = {n_el}, N_TB = {n_tb}, N_TROE = {n_troe}, N_LIND = {n_lind};")
     w(f"  static constexpr int MAXR = {MAXR}, MAXNET = {MAXNET};")
+    w(f"  static constexpr int NCH = {m.name}_t::kChunks;")
+    w(f"  using Packed = {m.name}_t::Packed;")
+    w(f"  PPC_DI static const Packed& pack() {{ return {m.name}_t::kPack; }}")
     for nm in ("nasaLo", "nasaHi", "tmid", "mw", "imw", "rxA", "rxB", "rxE", "rxNu", "effV", "foA",
                "foB", "foE", "troe", "spNu"):
         w(f"  PPC_DI static double {nm}_(int i) {{ return {m.name}_t::kTab.{nm}[i]; }}")
