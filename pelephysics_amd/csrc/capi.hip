@@ -320,16 +320,19 @@ int finish_with(pp_chem* h, int ncells, hipStream_t s, float kernel_ms, const pp
 }
 
 bool is_batched(int mode) { return mode == ppc::MODE_BATCHED_MIXED || mode == ppc::MODE_BATCHED_FP64; }
-// Kernels of a mode: ReactorCvode runs the plain FP64 adaptive BDF with its options.
+// Kernels of a mode: ReactorCvode runs the plain FP64 adaptive BDF with its
+// options (QSS mechanisms; the others its group form, gmode).
 int kmode(int mode) {
   return mode == PP_CHEM_CVODE ? ppc::MODE_ADAPTIVE : (mode == PP_CHEM_ARKODE ? ppc::MODE_ERK : mode);
 }
 
 // ---- device scratch of pp_chem_react_1d_noalloc: one array per GPU, held
 // until the process ends.  Layout: [0, 256) queue counter, [256, 512) the
-// statistics reduction, then the per-cell step counts, then the integrator
-// workspace.
-constexpr size_t kScratchBytes = 64ull << 20;
+// statistics reduction, then the per-cell step counts (up to kScratchCells
+// bytes from the start), then the integrator workspace, which finds at least
+// kScratchWs bytes whatever the number of cells.
+constexpr size_t kScratchCells = 64ull << 20, kScratchWs = 64ull << 20;
+constexpr size_t kScratchBytes = kScratchCells + kScratchWs;
 constexpr size_t kScratchCounts = 512;
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
@@ -376,9 +379,15 @@ int auto_cells_per_wave(const pp_chem* h, long long ncells) {
   return cpw;
 }
 
+// The handle's calls run on the work queue: the batched forms, and ReactorCvode
+// where there are group kernels.
+bool on_queue(const pp_chem* h) { return is_batched(h->cfg.mode) || (h->cfg.mode == PP_CHEM_CVODE && h->GL); }
+// Batched kernels of the handle's mode.
+int gmode(const pp_chem* h) { return h->cfg.mode == PP_CHEM_CVODE ? ppc::MODE_GROUP_CVODE : h->cfg.mode; }
+
 // Cells per wave of this call's group kernel; 0: one lane per cell.
 int cells_per_wave(const pp_chem* h, long long ncells) {
-  if (!is_batched(h->cfg.mode) || !h->GL) return 0;
+  if (!on_queue(h) || !h->GL) return 0;
   return h->cfg.batched_cells_per_wave != 0 ? h->cfg.batched_cells_per_wave : auto_cells_per_wave(h, ncells);
 }
 
@@ -463,9 +472,9 @@ ppc::QueueArgs prepare_queue(pp_chem* h, int ncells, const void* key, hipStream_
 hipError_t enqueue_1d(pp_chem* h, double* y, double* ysrc, double* rX, double* rXsrc, double dt, int ncells,
                       const void* key, hipStream_t s, bool count_fail = false) {
   hipError_t e;
-  if (is_batched(h->cfg.mode)) {
+  if (on_queue(h)) {
     const ppc::QueueArgs q = prepare_queue(h, ncells, key, s);
-    e = (h->GL ? h->GL : h->L)->batched_1d(h->cfg.mode, h->P, y, ysrc, rX, rXsrc, dt, q, counters(h), s);
+    e = (h->GL ? h->GL : h->L)->batched_1d(gmode(h), h->P, y, ysrc, rX, rXsrc, dt, q, counters(h), s);
   } else {
     e = h->L->react_1d(kmode(h->cfg.mode), h->P, y, ysrc, rX, rXsrc, dt, ncells, counters(h), h->cfg.block_size, s);
   }
@@ -940,7 +949,7 @@ int pp_chem_react_box(pp_chem* h, const int lo[3], const int hi[3], const pp_arr
   HIPCHK(h, hipEventRecord(h->ev0, s));
   if (ncells > 0) {
     hipError_t e;
-    if (is_batched(h->cfg.mode)) {
+    if (on_queue(h)) {
       // flat state, the 1-D kernel, back to the box: the operations of
       // ReactorBDF.cpp:376-389,461-478 (T from e / rho with the box T as
       // guess; rE + dt rEsrc; T from the new energy with the integrated T as
@@ -966,11 +975,12 @@ int pp_chem_react_box(pp_chem* h, const int lo[3], const int hi[3], const pp_arr
       if (e == hipSuccess) {
         const ppc::QueueArgs q = prepare_queue(h, ncells, rY->p, s);
         e = (h->GL ? h->GL : h->L)
-                ->batched_1d(h->cfg.mode, h->P, fa.y, fa.ysrc, fa.e, fa.esrc, *dt_react, q, counters(h), s);
+                ->batched_1d(gmode(h), h->P, fa.y, fa.ysrc, fa.e, fa.esrc, *dt_react, q, counters(h), s);
       }
       if (e == hipSuccess) {
         fa.dt = 0.0;  // the 1-D kernel has already advanced e by dt * rEsrc
-        fa.fc32 = counters(h).nsteps;
+        fa.fc32 = h->P.adapt.fc_rhs ? counters(h).nrhs : counters(h).nsteps;
+        fa.status = h->P.adapt.fc_rhs ? counters(h).nsteps : nullptr;
         e = h->L->flatten(fa, 1, s);
       }
     } else {
@@ -1042,10 +1052,10 @@ int pp_chem_react_1d_noalloc(pp_chem* h, double* y, double* ysrc, double* rX, do
   if (ncells > 0 && (!y || !ysrc || !rX || !rXsrc)) return fail(h, PP_CHEM_EINVAL, "null array");
   if (!h->scratch) return fail(h, PP_CHEM_EHIP, "device scratch of pp_chem_react_1d_noalloc unavailable");
   const size_t counts = ((size_t)ncells * sizeof(int) + 255) & ~(size_t)255;
-  if (kScratchCounts + counts > kScratchBytes)
+  if (kScratchCounts + counts > kScratchCells)
     return fail(h, PP_CHEM_EINVAL,
                 "ncells = " + std::to_string(ncells) + " exceeds the device scratch of pp_chem_react_1d_noalloc (" +
-                    std::to_string((kScratchBytes - kScratchCounts) / sizeof(int)) + " cells at most)");
+                    std::to_string((kScratchCells - kScratchCounts) / sizeof(int)) + " cells at most)");
   int* counter = reinterpret_cast<int*>(h->scratch);
   unsigned long long* red = reinterpret_cast<unsigned long long*>(h->scratch + 256);
   int* nsteps = reinterpret_cast<int*>(h->scratch + kScratchCounts);
@@ -1072,10 +1082,10 @@ int pp_chem_react_1d_noalloc(pp_chem* h, double* y, double* ysrc, double* rX, do
   HIPCHK(h, hipEventRecord(h->ev0, s));
   if (ncells > 0) {
     hipError_t e;
-    if (is_batched(h->cfg.mode)) {
+    if (on_queue(h)) {
       hipLaunchKernelGGL(zero_ints, dim3(1), dim3(64), 0, s, counter, 1);
       const ppc::QueueArgs q{nullptr, counter, ncells, h->max_blocks};  // cells in index order
-      e = (h->GL ? h->GL : h->L)->batched_1d(h->cfg.mode, P, y, ysrc, rX, rXsrc, *dt_react, q, st, s);
+      e = (h->GL ? h->GL : h->L)->batched_1d(gmode(h), P, y, ysrc, rX, rXsrc, *dt_react, q, st, s);
     } else {
       e = h->L->react_1d(kmode(h->cfg.mode), P, y, ysrc, rX, rXsrc, *dt_react, ncells, st, h->cfg.block_size, s);
     }
@@ -1160,7 +1170,7 @@ int pp_chem_react_1d_chained(pp_chem* h, double* y, double* ysrc, double* rX, do
   hipLaunchKernelGGL(zero_ints, dim3(1), dim3(64), 0, s, h->d_fail, 1);
   HIPCHK(h, hipGetLastError());
   int done = 0;
-  if (ncells > 0 && is_batched(h->cfg.mode) &&
+  if (ncells > 0 && on_queue(h) &&
       !(h->hist_valid && h->hist_ncells == ncells && h->hist_key == y)) {
     // the first call sets the cost history the captured calls order by
     const hipError_t e = enqueue_1d(h, y, ysrc, rX, rXsrc, dt, ncells, y, s, true);

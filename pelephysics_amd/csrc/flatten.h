@@ -79,7 +79,10 @@ __global__ void __launch_bounds__(256) unflatten_kernel(FlatArgs a) {
     const double e = a.e[c] + a.dt * b.rEsrc(i, j, k, 0);
     b.rE(i, j, k, 0) = e;
     b.T(i, j, k, 0) = T_from_energy_rt<M>(a.reactor_type, a.divide ? e / rho : e * rinv, Y, yc[NS]);
-    if (b.FC.p) b.FC(i, j, k, 0) = a.fc ? (double)a.fc[c] : (double)a.fc32[c];
+    if (b.FC.p) {
+      const bool failed = !a.fc && a.status && a.status[c] < 0;
+      b.FC(i, j, k, 0) = a.fc ? (double)a.fc[c] : (double)(failed ? a.status[c] : a.fc32[c]);
+    }
   }
 }
 

@@ -748,7 +748,11 @@ constexpr long long group_ws_doubles() {
 // Persistent kernel: each group of G lanes integrates cells from the queue
 // until it is empty.  P.ws holds group_ws_doubles<NEQ, G, LU_T>() doubles for
 // each of P.ws_lanes / 64 waves; waves beyond that leave at once.
-template <class T, typename LU_T, int G, int OCC>
+//
+// CV: ReactorCvode's options (AdaptParamsDev), as adaptive_cell takes them: the
+// order cap, the Newton iterations per attempt, the Jacobian's largest age and
+// per-component absolute tolerances.
+template <class T, typename LU_T, int G, int OCC, bool CV>
 __global__ void __launch_bounds__(64 * GROUP_WAVES) __attribute__((amdgpu_waves_per_eu(OCC, 8)))
 group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st) {
   using C = GroupChem<T, G>;
@@ -789,6 +793,8 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
   const double newton_tol = fmax(10 * 2.220446049250313e-16 / rtol, fmin(0.03, sqrt(rtol)));
   const double t_bound = dt;
   const long long rhs_cap = rhs_budget(ap.max_steps);
+  const int maxord = CV && ap.max_order > 0 && ap.max_order < AMAXORD ? ap.max_order : AMAXORD;
+  const int nmax = CV && ap.newton_maxiter > 0 ? ap.newton_maxiter : 4;
   // LU service: half of the wave's groups waiting, or as many trips.  A
   // factorisation for one group costs the whole wave the same, but a waiting
   // group idles (drm19, 262144 cells, 16 lanes per cell: 87 ms serving each
@@ -801,6 +807,12 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
   bool valid[EPL];
 #pragma unroll
   for (int e = 0; e < EPL; ++e) valid[e] = e * G + g < n;
+  double atv[CV ? EPL : 1];
+#pragma unroll
+  for (int e = 0; e < (CV ? EPL : 1); ++e) atv[e] = CV && ap.atolv && valid[e] ? ap.atolv[e * G + g] : atol;
+  // error weight of slot e at the value y
+  auto weight = [&](int e, double y) { return atv[CV ? e : 0] + rtol * fabs(y); };
+  int jac_step = 0;  // accepted steps at the last Jacobian
   double D[AMAXORD + 3][EPL];
   double yv[EPL];
   const LaneVec<EPL> d{lv}, ypred{lv + 64 * EPL}, psi{lv + 128 * EPL}, lus{lv + 192 * EPL};
@@ -865,6 +877,7 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
     n_equal = 0;
     lu_valid = need_lu = false;
     need_jac = 0;
+    jac_step = 0;
     wait = 0;
     nsteps = nrhs = njac = nlu = nnewton = nrej = status = 0;
   };
@@ -893,7 +906,7 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
   auto factor = [&]() {
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
-      const double w = atol + rtol * fabs(ypred[e]);
+      const double w = weight(e, ypred[e]);
       lus[e] = w;
       if (valid[e]) sv[e * G + g] = w;
     }
@@ -979,7 +992,7 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
       if (__builtin_expect(phase != PH_NEWTON, 0)) {
         // initial step size (Hairer, Norsett & Wanner I, II.4)
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) scl[e] = atol + fabs(D[0][e]) * rtol;
+        for (int e = 0; e < EPL; ++e) scl[e] = weight(e, D[0][e]);
         if (phase == PH_F0) {
 #pragma unroll
           for (int e = 0; e < EPL; ++e) D[1][e] = f[e];  // f0 kept in D[1] until h is known
@@ -1023,15 +1036,15 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
 #pragma unroll
           for (int e = 0; e < EPL; ++e) {
             b[e] = valid[e] ? (c * f[e] - psi[e] - d[e]) / lus[e] : 0.0;
-            scl[e] = atol + rtol * fabs(ypred[e]);
+            scl[e] = weight(e, ypred[e]);
           }
           group_inv_solve<n, G, EPL, LU_T>(LU, kstep, sv, sw, g, b, dy);
 #pragma unroll
           for (int e = 0; e < EPL; ++e) dy[e] *= lus[e];
           const double dy_norm = rms(dy, scl);
           const double rate = dy_norm_old < 0 ? -1.0 : dy_norm / dy_norm_old;
-          double left = rate;  // rate^(4 - k_newton)
-          for (int i = k_newton; i < 3; ++i) left *= rate;
+          double left = rate;  // rate^(nmax - k_newton)
+          for (int i = k_newton; i < nmax - 1; ++i) left *= rate;
           if (rate >= 0 && (rate >= 1 || left / (1 - rate) * dy_norm > newton_tol)) {
             failed = true;
           } else {
@@ -1045,7 +1058,7 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
             } else {
               dy_norm_old = dy_norm;
               k_newton++;
-              if (k_newton == 4) failed = true;
+              if (k_newton == nmax) failed = true;
             }
           }
         }
@@ -1054,6 +1067,7 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
             // refresh the Jacobian at the predictor and retry the same step
             need_jac = 2;
             current_jac = true;
+            jac_step = nsteps;
             need_lu = true;
 #pragma unroll
             for (int e = 0; e < EPL; ++e) {
@@ -1071,11 +1085,11 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
             attempt = true;
           }
         } else if (converged) {
-          const double safety = 0.9 * 9.0 / (double)(8 + n_iter);
+          const double safety = 0.9 * (2 * nmax + 1) / (double)(2 * nmax + n_iter);
           double err[EPL];
 #pragma unroll
           for (int e = 0; e < EPL; ++e) {
-            scl[e] = atol + rtol * fabs(yv[e]);
+            scl[e] = weight(e, yv[e]);
             err[e] = ndf_econst(order) * d[e];
           }
           const double error_norm = rms(err, scl);
@@ -1105,7 +1119,7 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
             if (n_equal >= order + 1) {
               double err2[EPL];
               const double cm = order > 1 ? ndf_econst(order - 1) : 0.0;
-              const double cp = order < AMAXORD ? ndf_econst(order + 1) : 0.0;
+              const double cp = order < maxord ? ndf_econst(order + 1) : 0.0;
 #pragma unroll
               for (int e = 0; e < EPL; ++e) {
                 double vm = 0.0, vp = 0.0;
@@ -1119,7 +1133,7 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
               }
               const double sm = Gr::sum(sq(err, scl)), sp = Gr::sum(sq(err2, scl));
               const double norms[3] = {order > 1 ? sqrt(sm / n) : INFINITY, error_norm,
-                                       order < AMAXORD ? sqrt(sp / n) : INFINITY};
+                                       order < maxord ? sqrt(sp / n) : INFINITY};
               double best = -1.0;
               int delta = 0;
 #pragma unroll
@@ -1190,6 +1204,13 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
           d[e] = 0.0;
         }
         c = h * inv_alpha;
+        // a Jacobian older than jac_age steps is re-evaluated at the prediction
+        if (CV && ap.jac_age > 0 && !current_jac && nsteps - jac_step >= ap.jac_age) {
+          need_jac = 2;
+          current_jac = true;
+          jac_step = nsteps;
+          lu_valid = false;
+        }
         if (!lu_valid) need_lu = true;
         dy_norm_old = -1.0;
         k_newton = 0;

@@ -60,6 +60,7 @@ hipError_t launch_batched_1d(int mode, const ReactParamsDev& P, double* y, const
                              const double* rXsrc, double dt, QueueArgs q, CellStats st, hipStream_t s) {
   if (mode == MODE_BATCHED_MIXED) return batched_1d_mode<M, MODE_BATCHED_MIXED>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
   if (mode == MODE_BATCHED_FP64) return batched_1d_mode<M, MODE_BATCHED_FP64>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
+  if (mode == MODE_GROUP_CVODE) return batched_1d_mode<M, MODE_GROUP_CVODE>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
   return hipErrorInvalidValue;
 }
 

@@ -99,13 +99,13 @@ int batched_grid(K kernel, const ReactParamsDev& P, const QueueArgs& q) {
 // The group kernel (group_bdf.h) with G lanes per cell: a persistent grid of
 // every resident block of GROUP_WAVES waves, at most q.max_blocks waves and the
 // waves the workspace holds (group_ws_rows rows of 64 lanes per wave).
-template <class T, typename LU_T, int G>
+template <class T, typename LU_T, int G, bool CV>
 hipError_t launch_group(const ReactParamsDev& P, double* y, const double* ysrc, double* rX, const double* rXsrc,
                         double dt, QueueArgs q, CellStats st, hipStream_t s) {
   static_assert(group_ws_doubles<T::NEQ, G, LU_T>() <= group_wave_doubles<T::NEQ, G>(), "workspace layout");
   // registers of the inverse's rows: above ~100 VGPRs hold the build to one wave per SIMD
   constexpr int lu_vgprs = (int)(((T::NEQ + G - 1) / G) * T::NEQ * sizeof(LU_T) / 4);
-  auto k = group_bdf_kernel<T, LU_T, G, (lu_vgprs > 100 ? 1 : 2)>;
+  auto k = group_bdf_kernel<T, LU_T, G, (lu_vgprs > 100 ? 1 : 2), CV>;
   int grid = resident_blocks(k, (long long)q.ncells * G, 64 * GROUP_WAVES);
   if (grid < 0) return hipErrorInvalidDevice;
   if (!P.ws || P.ws_lanes < 64 || P.ws_lanes % 64 != 0) return hipErrorInvalidValue;
@@ -118,23 +118,23 @@ hipError_t launch_group(const ReactParamsDev& P, double* y, const double* ysrc, 
   return hipGetLastError();
 }
 
-template <class M, typename LU_T>
+template <class M, typename LU_T, bool CV>
 hipError_t batched_group(const ReactParamsDev& P, double* y, const double* ysrc, double* rX, const double* rXsrc,
                          double dt, QueueArgs q, CellStats st, hipStream_t s) {
   using Tab = typename wave_tables<M>::type;
   if constexpr (!std::is_void<Tab>::value) {
     switch (P.adapt.group) {
       case 8:
-        if constexpr (group_ok<M, 8>()) return launch_group<Tab, LU_T, 8>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
+        if constexpr (group_ok<M, 8>()) return launch_group<Tab, LU_T, 8, CV>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
         break;
       case 4:
-        if constexpr (group_ok<M, 16>()) return launch_group<Tab, LU_T, 16>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
+        if constexpr (group_ok<M, 16>()) return launch_group<Tab, LU_T, 16, CV>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
         break;
       case 2:
-        if constexpr (group_ok<M, 32>()) return launch_group<Tab, LU_T, 32>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
+        if constexpr (group_ok<M, 32>()) return launch_group<Tab, LU_T, 32, CV>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
         break;
       case 1:
-        if constexpr (group_ok<M, 64>()) return launch_group<Tab, LU_T, 64>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
+        if constexpr (group_ok<M, 64>()) return launch_group<Tab, LU_T, 64, CV>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
         break;
       default:
         break;
@@ -147,11 +147,14 @@ template <class M, int MODE>
 hipError_t batched_1d_mode(const ReactParamsDev& P, double* y, const double* ysrc, double* rX, const double* rXsrc,
                            double dt, QueueArgs q, CellStats st, hipStream_t s) {
   using LU_T = typename std::conditional<MODE == MODE_BATCHED_MIXED, float, double>::type;
+  constexpr bool CV = MODE == MODE_GROUP_CVODE;
   if constexpr (!has_qss<M>::value) {
     // a group of lanes per cell at every size (group_bdf.h): one cell per lane
     // measured 3.2 times as long on 64^3 drm19 cells and 16 to 115 times on
     // calls that do not fill the chip (figures there)
-    return batched_group<M, LU_T>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
+    return batched_group<M, LU_T, CV>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
+  } else if constexpr (CV) {
+    return hipErrorInvalidValue;
   } else {
     auto k = P.adapt.lane_occ == 1 ? batched_kernel<M, LU_T, IO1D, 1> : batched_kernel<M, LU_T, IO1D, 2>;
     const int grid = batched_grid<M, MODE>(k, P, q);

@@ -7,9 +7,10 @@ namespace ppc {
 
 // integrators: 0 ReactorBDF parity, 1 ReactorRK64 parity, 2 adaptive BDF (plain,
 // one lane per cell, FP64), 3 batched adaptive BDF with FP32 LU, 4 batched
-// adaptive BDF with FP64 LU, 6 ReactorArkode's explicit Runge-Kutta
+// adaptive BDF with FP64 LU, 6 explicit Runge-Kutta
+// (ReactorArkode), 7 ReactorCvode's options on the batched adaptive BDF with FP64 LU
 enum : int { MODE_BDF = 0, MODE_RK64 = 1, MODE_ADAPTIVE = 2, MODE_BATCHED_MIXED = 3, MODE_BATCHED_FP64 = 4,
-             MODE_ERK = 6 };
+             MODE_ERK = 6, MODE_GROUP_CVODE = 7 };
 
 // ------------------------------------------------------------------ I/O --
 struct A4 {  // amrex::Array4 layout
@@ -53,6 +54,7 @@ struct FlatArgs {
   double* esrc;          // ncells (flatten only)
   const long long* fc;   // ncells step counts written to FC (unflatten only)
   const int* fc32;       // the same as int counts, used when fc is null
+  const int* status;     // with fc32: a cell's negative status is written in its place (null: none)
   double dt;             // unflatten: rE = e + dt * rEsrc
   int reactor_type, clean;
   int divide;            // energy per mass as e / rho (ReactorBDF.cpp:379,469) instead of e * (1 / rho)
