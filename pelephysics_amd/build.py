@@ -29,7 +29,7 @@ MECHS = ["LiDryer", "drm19", "dodecane_lu", "heptane_lu_88sk", "CH4_lean_qss", "
 MODES = {"bdf": ("MODE", "MODE_BDF"), "rk64": ("MODE", "MODE_RK64"),
          "adaptive": ("MODE", "MODE_ADAPTIVE"), "erk": ("MODE", "MODE_ERK"),
          "bmixed": ("BATCHED", "MODE_BATCHED_MIXED"),
-         "bfp64": ("BATCHED", "MODE_BATCHED_FP64"), "cvode": ("BATCHED", "MODE_GROUP_CVODE"), "adjoint": ("ADJOINT", "MODE_BDF"),
+         "bfp64": ("BATCHED", "MODE_BATCHED_FP64"), "cvode": ("BATCHED", "MODE_GROUP_CVODE"), "gfixed": ("GFIXED", "MODE_BDF"), "adjoint": ("ADJOINT", "MODE_BDF"),
          "flatten": ("FLATTEN", "MODE_BDF")}
 ARCH = "gfx950"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -47,14 +47,21 @@ const MechLauncher* resolve_mech(const char* name, int manifold_dim) {
   return find_mech(name);
 }
 
-// Sums the per-cell counters and reduces min/max of the step counts.
+// Sums the per-cell counters and reduces min/max of the step counts into host
+// memory: sum of steps, rhs, jac, lu, newton, reject, failed cells, largest
+// and smallest step count.  The blocks add up in acc (9 words, the smallest as
+// the largest distance below INT_MAX, and a count of blocks done); the last
+// block hands the result to the host and leaves acc zero for the next call, so
+// a call needs one launch, no clearing and no copy (one drm19 box of 3360
+// cells: 360 us a call against 389 with a clearing launch, a copy and a
+// second wait).
+constexpr int NSTAT = 9;
 __global__ void __launch_bounds__(256) reduce_stats(const int* __restrict__ nsteps, const int* __restrict__ nrhs,
                                                     const int* __restrict__ njac, const int* __restrict__ nlu,
                                                     const int* __restrict__ nnewton,
                                                     const int* __restrict__ nreject, int ncells,
-                                                    unsigned long long* __restrict__ out) {
-  // out: [0] sum steps, [1] rhs, [2] jac, [3] lu, [4] newton, [5] reject,
-  //      [6] failed cells, [7] max steps, [8] min steps
+                                                    unsigned long long* __restrict__ acc,
+                                                    unsigned long long* __restrict__ host) {
   unsigned long long s[7] = {0, 0, 0, 0, 0, 0, 0};
   int mx = 0, mn = 0x7fffffff;
   for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncells; c += gridDim.x * blockDim.x) {
@@ -83,9 +90,23 @@ __global__ void __launch_bounds__(256) reduce_stats(const int* __restrict__ nste
   }
   if ((threadIdx.x & 63) == 0) {
     for (int i = 0; i < 7; ++i)
-      if (s[i]) atomicAdd(&out[i], s[i]);
-    atomicMax(&out[7], (unsigned long long)mx);
-    atomicMin(&out[8], (unsigned long long)mn);
+      if (s[i]) atomicAdd(&acc[i], s[i]);
+    atomicMax(&acc[7], (unsigned long long)mx);
+    atomicMax(&acc[8], (unsigned long long)(0x7fffffff - mn));
+    __threadfence();
+  }
+  __syncthreads();
+  __shared__ bool last;
+  if (threadIdx.x == 0) last = atomicAdd(&acc[NSTAT], 1ULL) == (unsigned long long)gridDim.x - 1;
+  __syncthreads();
+  if (last && threadIdx.x <= NSTAT) {
+    __threadfence();
+    const unsigned long long v = atomicExch(&acc[threadIdx.x], 0ULL);
+    if (threadIdx.x < NSTAT) {
+      __hip_atomic_store(&host[threadIdx.x], threadIdx.x == 8 ? 0x7fffffffULL - v : v, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+      __threadfence_system();
+    }
   }
 }
 
@@ -94,10 +115,6 @@ __global__ void __launch_bounds__(256) reduce_stats(const int* __restrict__ nste
 __global__ void __launch_bounds__(256) count_failed(const int* __restrict__ nsteps, int ncells, int* __restrict__ nfail) {
   for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncells; c += gridDim.x * blockDim.x)
     if (nsteps[c] < 0) atomicAdd(nfail, 1);
-}
-
-__global__ void init_stats(unsigned long long* out) {
-  if (threadIdx.x < 9) out[threadIdx.x] = (threadIdx.x == 8) ? 0x7fffffffULL : 0ULL;
 }
 
 // ---- work-queue order: counting sort of the cells by the previous call's RHS
@@ -173,10 +190,12 @@ struct pp_chem {
   ppc::ReactParamsDev P{};
   int device = 0;
   int ncu = 0;  // compute units
+  int fixed_cpw = 0;  // cells per wave of this call's RK64 / fixed-step BDF group kernel, 0: one lane per cell
   // per-cell counters (device), grown on demand
   int cap = 0;
   int* d_cnt = nullptr;  // 6 * cap ints
-  unsigned long long* d_red = nullptr;
+  unsigned long long* d_red = nullptr;  // reduce_stats' accumulators, zero between calls
+  unsigned long long* h_red = nullptr;  // its result (pinned host memory)
   // work queue of the batched forms: counter, visiting order, cost bins and
   // the identity of the last call (its per-cell costs order the next call)
   int* d_queue = nullptr;  // [0] counter, [1..NBINS] bins, [NBINS+1..2NBINS] offsets
@@ -276,25 +295,22 @@ ppc::CellStats counters(pp_chem* h) {
   return st;
 }
 
-// Reduces the counters st of the last launch (into the 9-word buffer red) and
+// Reduces the counters st of the call's kernels on stream s (accumulators red),
+// waits for the stream, takes the kernels' time from the events around them and
 // returns int(average steps) or an error.
-int finish_with(pp_chem* h, int ncells, hipStream_t s, float kernel_ms, const ppc::CellStats& st,
-                unsigned long long* red);
+int finish_with(pp_chem* h, int ncells, hipStream_t s, const ppc::CellStats& st, unsigned long long* red);
 
-int finish(pp_chem* h, int ncells, hipStream_t s, float kernel_ms) {
-  return finish_with(h, ncells, s, kernel_ms, counters(h), h->d_red);
-}
+int finish(pp_chem* h, int ncells, hipStream_t s) { return finish_with(h, ncells, s, counters(h), h->d_red); }
 
-int finish_with(pp_chem* h, int ncells, hipStream_t s, float kernel_ms, const ppc::CellStats& st,
-                unsigned long long* red) {
-  hipLaunchKernelGGL(init_stats, dim3(1), dim3(64), 0, s, red);
+int finish_with(pp_chem* h, int ncells, hipStream_t s, const ppc::CellStats& st, unsigned long long* red) {
   const int blocks = ncells > 0 ? (ncells + 255) / 256 < 1024 ? (ncells + 255) / 256 : 1024 : 1;
   hipLaunchKernelGGL(reduce_stats, dim3(blocks), dim3(256), 0, s, st.nsteps, st.nrhs, st.njac, st.nlu,
-                     st.nnewton, st.nreject, ncells, red);
+                     st.nnewton, st.nreject, ncells, red, h->h_red);
   HIPCHK(h, hipGetLastError());
-  unsigned long long r[9];
-  HIPCHK(h, hipMemcpyAsync(r, red, sizeof(r), hipMemcpyDeviceToHost, s));
   HIPCHK(h, hipStreamSynchronize(s));
+  float kernel_ms = 0.f;
+  HIPCHK(h, hipEventElapsedTime(&kernel_ms, h->ev0, h->ev1));
+  const unsigned long long* r = h->h_red;
   pp_chem_stats& S = h->stats;
   S.ncells = ncells;
   S.nsteps = (long long)r[0];
@@ -385,6 +401,35 @@ bool on_queue(const pp_chem* h) { return is_batched(h->cfg.mode) || (h->cfg.mode
 // Batched kernels of the handle's mode.
 int gmode(const pp_chem* h) { return h->cfg.mode == PP_CHEM_CVODE ? ppc::MODE_GROUP_CVODE : h->cfg.mode; }
 
+// Cells per wave of ReactorRK64's and the fixed-step ReactorBDF's group kernels
+// (group_fixed.h); 0: one lane per cell.  The one-lane kernels take about the
+// same time for any call up to the 65536 cells that give every SIMD a wave, the
+// group kernels' time grows with the cells once these fill the chip, and their
+// right-hand side spends more instructions per cell, so large calls go to the
+// lane kernels.  Measured (kernel us, one lane / group, drm19 with the box's
+// dt = 1e-6 s): BDF 2048 cells 388 / 59, 32768 795 / 415, 131072 2418 / 1630;
+// RK64 2048 cells 7899 / 2190, 24576 8220 / 7212, 32768 8290 / 9056; LiDryer
+// RK64 8192 cells 910 / 764, 24576 1029 / 1443.  RK64's state is three vectors:
+// the narrowest group that still gives every SIMD two waves; the BDF's group is
+// always 16 lanes.  The smallest mechanisms' BDF stays on one lane: LiDryer's
+// hot cells amplify the last bit of the Jacobian (ReactorBDFsolver.H's residual
+// test below rounding) and the group's order of its sums gives other results
+// there than the reference's order.
+int fixed_cells_per_wave(const pp_chem* h, long long ncells) {
+  const int mode = h->cfg.mode;
+  if (!h->GL || (mode != PP_CHEM_BDF && mode != PP_CHEM_RK64)) return 0;
+  if (h->GL->group_fixed(mode, h->P, nullptr, nullptr, nullptr, nullptr, nullptr, 0.0, 0, 1, {}, nullptr) != hipSuccess)
+    return 0;
+  const bool small = h->L->ns < 16;
+  if (mode == PP_CHEM_BDF) return 4;
+  if (ncells > (small ? 32LL : 96LL) * h->ncu) return 0;
+  const long long waves = 8LL * std::max(h->ncu, 1);
+  int cpw = 8;
+  while (cpw > 1 && (h->GL->group_ws_rows(cpw) <= 0 || (ncells < waves * cpw && h->GL->group_ws_rows(cpw / 2) > 0)))
+    cpw /= 2;
+  return cpw;
+}
+
 // Cells per wave of this call's group kernel; 0: one lane per cell.
 int cells_per_wave(const pp_chem* h, long long ncells) {
   if (!on_queue(h) || !h->GL) return 0;
@@ -423,6 +468,7 @@ void group_params(const pp_chem* h, int cpw, ppc::AdaptParamsDev& a) {
 int prepare_workspace(pp_chem* h, int ncells) {
   const int cpw = cells_per_wave(h, ncells);
   group_params(h, cpw, h->P.adapt);
+  h->fixed_cpw = fixed_cells_per_wave(h, ncells);
   h->P.ws = nullptr;
   h->P.ws_lanes = 0;
   long long rows = 0;
@@ -475,6 +521,8 @@ hipError_t enqueue_1d(pp_chem* h, double* y, double* ysrc, double* rX, double* r
   if (on_queue(h)) {
     const ppc::QueueArgs q = prepare_queue(h, ncells, key, s);
     e = (h->GL ? h->GL : h->L)->batched_1d(gmode(h), h->P, y, ysrc, rX, rXsrc, dt, q, counters(h), s);
+  } else if (h->fixed_cpw) {
+    e = h->GL->group_fixed(h->cfg.mode, h->P, y, ysrc, rX, rXsrc, nullptr, dt, ncells, h->fixed_cpw, counters(h), s);
   } else {
     e = h->L->react_1d(kmode(h->cfg.mode), h->P, y, ysrc, rX, rXsrc, dt, ncells, counters(h), h->cfg.block_size, s);
   }
@@ -723,9 +771,15 @@ int pp_chem_create(const pp_chem_config* cfg, pp_chem** out) {
   // one-lane-per-cell ones, or the group size the caller names
   if (cfg->batched_waves_per_cu > 0 && (!h->GL || cfg->batched_cells_per_wave != 0))
     h->max_blocks = cfg->batched_waves_per_cu * h->ncu;  // 64-lane waves
-  if (e == hipSuccess) e = hipMalloc(&h->d_red, sizeof(unsigned long long) * 9);
-  if (e == hipSuccess) e = hipMalloc(&h->d_queue, sizeof(int) * (1 + 2 * NBINS));
-  if (e == hipSuccess) e = hipMalloc(&h->d_fail, sizeof(int));
+  // one allocation: the accumulators, the queue and the failure count
+  constexpr size_t red_bytes = sizeof(unsigned long long) * (NSTAT + 1), queue_ints = 1 + 2 * NBINS;
+  if (e == hipSuccess) e = hipMalloc(&h->d_red, red_bytes + sizeof(int) * (queue_ints + 1));
+  if (e == hipSuccess) e = hipMemset(h->d_red, 0, red_bytes);
+  if (e == hipSuccess) {
+    h->d_queue = reinterpret_cast<int*>(h->d_red + NSTAT + 1);
+    h->d_fail = h->d_queue + queue_ints;
+  }
+  if (e == hipSuccess) e = hipHostMalloc(&h->h_red, sizeof(unsigned long long) * NSTAT, hipHostMallocDefault);
   if (e == hipSuccess) e = hipEventCreate(&h->ev0);
   if (e == hipSuccess) e = hipEventCreate(&h->ev1);
   if (e != hipSuccess) {
@@ -749,8 +803,7 @@ void pp_chem_destroy(pp_chem* h) {
   if (h->d_ws) (void)hipFree(h->d_ws);
   if (h->d_cnt) (void)hipFree(h->d_cnt);
   if (h->d_red) (void)hipFree(h->d_red);
-  if (h->d_queue) (void)hipFree(h->d_queue);
-  if (h->d_fail) (void)hipFree(h->d_fail);
+  if (h->h_red) (void)hipHostFree(h->h_red);
   if (h->d_order) (void)hipFree(h->d_order);
   if (h->d_stage) (void)hipFree(h->d_stage);
   if (h->d_atolv) (void)hipFree(h->d_atolv);
@@ -983,16 +1036,16 @@ int pp_chem_react_box(pp_chem* h, const int lo[3], const int hi[3], const pp_arr
         fa.status = h->P.adapt.fc_rhs ? counters(h).nsteps : nullptr;
         e = h->L->flatten(fa, 1, s);
       }
+    } else if (h->fixed_cpw) {
+      e = h->GL->group_fixed(h->cfg.mode, h->P, nullptr, nullptr, nullptr, nullptr, &b, *dt_react, ncells,
+                             h->fixed_cpw, counters(h), s);
     } else {
       e = h->L->react_box(kmode(h->cfg.mode), h->P, b, *dt_react, ncells, counters(h), h->cfg.block_size, s);
     }
     if (e != hipSuccess) return hip_fail(h, e, "react_box launch");
   }
   HIPCHK(h, hipEventRecord(h->ev1, s));
-  HIPCHK(h, hipEventSynchronize(h->ev1));
-  float ms = 0.f;
-  HIPCHK(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
-  const int r = finish(h, ncells, s, ms);
+  const int r = finish(h, ncells, s);
   if (h->cfg.mod_reactor) *time += *dt_react;
   return r;
 }
@@ -1036,10 +1089,7 @@ int pp_chem_react_1d(pp_chem* h, double* y, double* ysrc, double* rX, double* rX
     HIPCHK(h, hipMemcpyAsync(y, dy, ny * sizeof(double), hipMemcpyDeviceToHost, s));
     HIPCHK(h, hipMemcpyAsync(rX, dx, nx * sizeof(double), hipMemcpyDeviceToHost, s));
   }
-  HIPCHK(h, hipEventSynchronize(h->ev1));
-  float ms = 0.f;
-  HIPCHK(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
-  const int r = finish(h, ncells, s, ms);
+  const int r = finish(h, ncells, s);
   if (h->cfg.mod_reactor) *time += *dt_react;
   return r;
 }
@@ -1086,16 +1136,15 @@ int pp_chem_react_1d_noalloc(pp_chem* h, double* y, double* ysrc, double* rX, do
       hipLaunchKernelGGL(zero_ints, dim3(1), dim3(64), 0, s, counter, 1);
       const ppc::QueueArgs q{nullptr, counter, ncells, h->max_blocks};  // cells in index order
       e = (h->GL ? h->GL : h->L)->batched_1d(gmode(h), P, y, ysrc, rX, rXsrc, *dt_react, q, st, s);
+    } else if (const int fcpw = fixed_cells_per_wave(h, ncells)) {
+      e = h->GL->group_fixed(h->cfg.mode, P, y, ysrc, rX, rXsrc, nullptr, *dt_react, ncells, fcpw, st, s);
     } else {
       e = h->L->react_1d(kmode(h->cfg.mode), P, y, ysrc, rX, rXsrc, *dt_react, ncells, st, h->cfg.block_size, s);
     }
     if (e != hipSuccess) return hip_fail(h, e, "react_1d_noalloc launch");
   }
   HIPCHK(h, hipEventRecord(h->ev1, s));
-  HIPCHK(h, hipEventSynchronize(h->ev1));
-  float ms = 0.f;
-  HIPCHK(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
-  const int r = finish_with(h, ncells, s, ms, st, red);
+  const int r = finish_with(h, ncells, s, st, red);
   if (h->cfg.mod_reactor) *time += *dt_react;
   return r;
 }
@@ -1202,11 +1251,9 @@ int pp_chem_react_1d_chained(pp_chem* h, double* y, double* ysrc, double* rX, do
   }
   HIPCHK(h, hipEventRecord(h->ev1, s));
   HIPCHK(h, hipEventSynchronize(h->ev1));
-  float ms = 0.f;
-  HIPCHK(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
   int nfail = 0;
   HIPCHK(h, hipMemcpy(&nfail, h->d_fail, sizeof(int), hipMemcpyDeviceToHost));
-  const int r = finish(h, ncells, s, ms);
+  const int r = finish(h, ncells, s);
   if (h->cfg.mod_reactor) *time += ncalls * dt;
   if (r >= 0 && nfail > 0)
     return fail(h, PP_CHEM_EINTEGRATE,

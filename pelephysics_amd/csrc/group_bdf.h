@@ -163,6 +163,22 @@ PPC_DI typename T::Packed& lds_pack() {
   return p;
 }
 
+// Waves per block of the group kernels: they share one copy of the tables.
+constexpr int GROUP_WAVES = 4;
+
+// Fills it, by every thread of the block.
+template <class T>
+PPC_DI const typename T::Packed& load_pack() {
+  using PK = typename T::Packed;
+  PK& pk = lds_pack<T>();
+  const int4* from = reinterpret_cast<const int4*>(&T::pack());
+  int4* to = reinterpret_cast<int4*>(&pk);
+  static_assert(sizeof(PK) % 16 == 0, "packed tables in 16-byte words");
+  for (int i = threadIdx.x; i < (int)(sizeof(PK) / 16); i += 64 * GROUP_WAVES) to[i] = from[i];
+  __syncthreads();
+  return pk;
+}
+
 // The table accessors TabMech::jac_reaction reads, in packed reaction order.
 template <class T>
 struct PackTab : T {
@@ -462,17 +478,17 @@ struct GroupChem {
   }
 
   // The BDF Jacobian d f_i / d y_j (bdf_jacobian in chem_cell.h with s = 1) of
-  // one cell by the whole wave: y in wa[0..n) of the wave's area, accumulated
-  // column-major (aJacobian / DWDOT layout) in J, then element (i, j) stored at
-  // out[(e*n + j)*G + g] for i = e*G + g.  J is in LDS or, for the larger
-  // mechanisms, in the workspace.
-  template <int CONSP, typename JT>
-  PPC_DI static void jacobian(const PK& pk, double* wa, double* J, JT* out) {
-    constexpr int W = (NS + 63) / 64;
-    const int l = (int)__lane_id();
+  // one cell by WD lanes (the whole wave, or each group for its own cell): y in
+  // wa[0..n) of their area, accumulated column-major (aJacobian / DWDOT layout)
+  // in J, which is in LDS or, for the larger mechanisms, in the workspace;
+  // jac_elem gives its elements.
+  template <int CONSP, int WD>
+  PPC_DI static void jacobian(const PK& pk, double* wa, double* J) {
+    constexpr int W = (NS + WD - 1) / WD;
+    const int l = Grp<WD>::lane();
     const double* y = wa;
     double *c = wa + NP, *gk = wa + 2 * NP, *hh = wa + 3 * NP, *wd = wa + 4 * NP;
-    const auto ld = [&](int i) { return JLDS ? J[i] : ws_load(J + i); };
+    const auto ld = [&](int i) { return jload(J, i); };
     const auto st = [&](int i, double v) {
       if (JLDS)
         J[i] = v;
@@ -490,7 +506,7 @@ struct GroupChem {
     double msum = 0.0;
 #pragma unroll
     for (int e = 0; e < W; ++e) {
-      const int k = e * 64 + l;
+      const int k = e * WD + l;
       cR[e] = dcR[e] = eh[e] = sc[e] = 0.0;
       if (k < NS) {
         double a[7], imw;
@@ -508,11 +524,11 @@ struct GroupChem {
       }
     }
 #pragma unroll 1
-    for (int i = l; i < n * n; i += 64) st(i, 0.0);
-    const double mixture = wave::sum(msum);
+    for (int i = l; i < n * n; i += WD) st(i, 0.0);
+    const double mixture = Grp<WD>::sum(msum);
     jsync();
 #pragma unroll 1
-    for (int j = l; j < NR; j += 64)
+    for (int j = l; j < NR; j += WD)
       TM::template jac_reaction<CONSP>(
           j, c, gk, hh, mixture, Tv, invT, invT2, logT, refC, refCinv,
           [&](int idx, double v) {
@@ -529,7 +545,7 @@ struct GroupChem {
     double s_cm = 0.0, s_dcm = 0.0, s_eh = 0.0, s_deh = 0.0;
 #pragma unroll
     for (int e = 0; e < W; ++e) {
-      const int k = e * 64 + l;
+      const int k = e * WD + l;
       if (k < NS) {
         const double wdk = wd[k];
         s_cm += cR[e] * sc[e];
@@ -538,14 +554,14 @@ struct GroupChem {
         s_deh += invT * (cR[e] - eh[e]) * wdk + eh[e] * ld(NS * n + k);
       }
     }
-    const double cmix = wave::sum(s_cm), dcmixdT = wave::sum(s_dcm);
-    const double ehmix = wave::sum(s_eh), dehmixdT = wave::sum(s_deh);
+    const double cmix = Grp<WD>::sum(s_cm), dcmixdT = Grp<WD>::sum(s_dcm);
+    const double ehmix = Grp<WD>::sum(s_eh), dehmixdT = Grp<WD>::sum(s_deh);
     const double cmixinv = 1.0 / cmix;
     const double tmp1 = ehmix * cmixinv, tmp3 = cmixinv * Tv, tmp2 = tmp1 * tmp3;
     double trow[W];
 #pragma unroll
     for (int e = 0; e < W; ++e) {
-      const int k = e * 64 + l;
+      const int k = e * WD + l;
       trow[e] = 0.0;
       if (k < NS) {
         double d = 0.0;
@@ -557,20 +573,30 @@ struct GroupChem {
     jsync();
 #pragma unroll
     for (int e = 0; e < W; ++e)
-      if (e * 64 + l < NS) st((e * 64 + l) * n + NS, trow[e]);
+      if (e * WD + l < NS) st((e * WD + l) * n + NS, trow[e]);
     if (l == 0) st(n * n - 1, -tmp1 + tmp2 * dcmixdT - tmp3 * dehmixdT);
     jsync();
-    // DWDOT scaling (T column x1e-6, T row x1e6) and the molecular-weight
-    // scaling: row i, column j = d f_i / d y_j
+  }
+  PPC_DI static double jload(const double* J, const int i) { return JLDS ? J[i] : ws_load(J + i); }
+
+  // d f_i / d y_j of jacobian()'s J: the DWDOT scaling (T column x1e-6, T row
+  // x1e6) and the molecular-weight scaling
+  PPC_DI static double jac_elem(const PK& pk, const double* J, const int i, const int j) {
+    double v = jload(J, j * n + i);
+    if (i == j) return v;  // no scaling, and no rounding, on the diagonal
+    if (i == NS) v *= 1.0e6;
+    if (j == NS) v *= 1.0e-6;
+    v *= i < NS ? pk.mw[i] : 1.0;
+    v *= j < NS ? pk.sp[j].imw : 1.0;
+    return v;
+  }
+  // all of them, element (i, j) at out[(e*n + j)*G + g] for i = e*G + g
+  template <typename JT>
+  PPC_DI static void jac_rows(const PK& pk, const double* J, JT* out) {
 #pragma unroll 4
-    for (int t = l; t < n * n; t += 64) {
+    for (int t = (int)__lane_id(); t < n * n; t += 64) {
       const int j = t / n, i = t - j * n;
-      double v = ld(t);
-      v *= i < NS ? pk.mw[i] : 1.0;
-      v *= j < NS ? pk.sp[j].imw : 1.0;
-      if (i == NS && j < NS) v *= 1.0e6;
-      if (j == NS && i < NS) v *= 1.0e-6;
-      out[((i / G) * n + j) * G + i % G] = (JT)v;
+      out[((i / G) * n + j) * G + i % G] = (JT)jac_elem(pk, J, i, j);
     }
   }
 };
@@ -734,9 +760,6 @@ PPC_DI double ten_ulps(const double t) {
   return 10.0 * (__longlong_as_double(__double_as_longlong(t) + 1) - t);
 }
 
-// Waves per block: they share one copy of the tables.
-constexpr int GROUP_WAVES = 4;
-
 // Doubles of device workspace per wave: the Jacobian accumulator of the larger
 // mechanisms and the groups' Jacobian rows in JT.
 template <int n, int G, typename JT>
@@ -761,14 +784,7 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
   constexpr int n = C::n, NS = C::NS, EPL = C::EPL, SPL = C::SPL, NP = C::NP;
   __shared__ __attribute__((aligned(16))) double lds[GROUP_WAVES * C::WAREA];
   __shared__ double lvec[GROUP_WAVES * 4 * 64 * EPL];
-  PK& pk = lds_pack<T>();
-  {
-    const int4* from = reinterpret_cast<const int4*>(&T::pack());
-    int4* to = reinterpret_cast<int4*>(&pk);
-    static_assert(sizeof(PK) % 16 == 0, "packed tables in 16-byte words");
-    for (int i = threadIdx.x; i < (int)(sizeof(PK) / 16); i += 64 * GROUP_WAVES) to[i] = from[i];
-    __syncthreads();
-  }
+  const PK& pk = load_pack<T>();
   const int wv = (int)(threadIdx.x >> 6);
   const long long wid = (long long)blockIdx.x * GROUP_WAVES + wv;
   if (wid >= P.ws_lanes / 64) return;  // the workspace holds no more waves
@@ -944,9 +960,10 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
       }
       wave_sync();
       if (eform)
-        C::template jacobian<0, LU_T>(pk, wa, Jw, rows + s * GSTRIDE);
+        C::template jacobian<0, 64>(pk, wa, Jw);
       else
-        C::template jacobian<1, LU_T>(pk, wa, Jw, rows + s * GSTRIDE);
+        C::template jacobian<1, 64>(pk, wa, Jw);
+      C::template jac_rows<LU_T>(pk, Jw, rows + s * GSTRIDE);
       __threadfence_block();
       wave_sync();
       if (gi == s) {

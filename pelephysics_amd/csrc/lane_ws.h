@@ -97,6 +97,14 @@ constexpr bool group_ok() {
   return has_table<M>::value && !has_qss<M>::value && M::NEQ <= 3 * G && G <= 2 * M::NEQ;
 }
 
+// The fixed-step BDF's group kernel (16 lanes per cell) holds the Krylov bases
+// of a wave's four cells in LDS: 24 equations at most; below 17 the one-lane
+// kernel runs (fixed_cells_per_wave in capi.hip).
+template <class M>
+constexpr bool group_fixed_ok() {
+  return group_ok<M, 16>() && M::NEQ <= 24 && M::NEQ > 16;
+}
+
 // Device workspace of one wave of the group kernel (doubles, at most): an n x n
 // FP64 Jacobian accumulator and the Jacobian rows of its 64 / G groups.
 template <int n, int G>

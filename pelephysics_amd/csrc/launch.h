@@ -21,6 +21,12 @@ struct MechLauncher {
   // batched (persistent, work-queue) forms; grid = number of 64-lane blocks
   hipError_t (*batched_1d)(int mode, const ReactParamsDev& P, double* y, const double* ysrc, double* rX,
                            const double* rXsrc, double dt, QueueArgs q, CellStats st, hipStream_t s);
+  // MODE_RK64 and MODE_BDF with a group of cells_per_wave lanes' cells per wave
+  // (group_fixed.h), flat state or (b not null) a box; hipErrorNotSupported
+  // where there is no such kernel.  With ncells = 0 only the latter is asked.
+  hipError_t (*group_fixed)(int mode, const ReactParamsDev& P, double* y, const double* ysrc, double* rX,
+                            const double* rXsrc, const BoxArgs* b, double dt, int ncells, int cells_per_wave,
+                            CellStats st, hipStream_t s);
   // discrete adjoint of the fixed-step BDF (table-driven mechanisms only)
   hipError_t (*adjoint_1d)(const ReactParamsDev& P, const AdjointArgs& a, hipStream_t s);
   // workspace rows per lane a mode needs (lane_ws.h); 0: none
@@ -38,6 +44,11 @@ struct MechLauncher {
 
 template <class M>
 hipError_t launch_mech_eval(int what, const double* sc, const double* T, int ncells, double* out, hipStream_t s);
+
+template <class M>
+hipError_t launch_group_fixed(int mode, const ReactParamsDev& P, double* y, const double* ysrc, double* rX,
+                              const double* rXsrc, const BoxArgs* b, double dt, int ncells, int cells_per_wave,
+                              CellStats st, hipStream_t s);
 
 template <class M>
 hipError_t launch_flatten(const FlatArgs& a, int unflatten, hipStream_t s);
@@ -98,6 +109,7 @@ hipError_t launch_box(int mode, const ReactParamsDev& P, const BoxArgs& b, doubl
                                    1,                                                          \
                                    &launch_1d<TYPE>, &launch_box<TYPE>,                        \
                                    &launch_batched_1d<TYPE>,                                   \
+                                   &launch_group_fixed<TYPE>,                                  \
                                    &launch_adjoint<TYPE>, &integrator_ws_rows<TYPE>,           \
                                    &group_ws_rows<TYPE>,                                       \
                                    &launch_flatten<TYPE>, &launch_mech_eval<TYPE>};            \

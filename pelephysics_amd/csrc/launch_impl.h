@@ -7,6 +7,7 @@
 #include "wave_bdf.h"
 #include "wave_adjoint.h"
 #include "group_bdf.h"
+#include "group_fixed.h"
 #include "flatten.h"
 
 namespace ppc {
@@ -165,6 +166,74 @@ hipError_t batched_1d_mode(const ReactParamsDev& P, double* y, const double* ysr
   }
 }
 
+template <class T, int G, bool BOX>
+hipError_t launch_group_rk64(const ReactParamsDev& P, const GroupIO& io, double dt, int ncells, CellStats st,
+                             hipStream_t s) {
+  auto k = group_rk64_kernel<T, G, BOX>;
+  const int grid = resident_blocks(k, (long long)ncells * G, 64 * GROUP_WAVES);
+  if (grid < 0) return hipErrorInvalidDevice;
+  hipLaunchKernelGGL(k, dim3(grid), dim3(64 * GROUP_WAVES), 0, s, P, io, dt, ncells, st);
+  return hipGetLastError();
+}
+
+template <class T, bool BOX>
+hipError_t launch_group_bdf_fixed(const ReactParamsDev& P, const GroupIO& io, double dt, int ncells, CellStats st,
+                                  hipStream_t s) {
+  auto k = group_bdf_fixed_kernel<T, BOX>;
+  const int grid = resident_blocks(k, (long long)ncells * 16, 64 * GROUP_WAVES);
+  if (grid < 0) return hipErrorInvalidDevice;
+  hipLaunchKernelGGL(k, dim3(grid), dim3(64 * GROUP_WAVES), 0, s, P, io, dt, ncells, st);
+  return hipGetLastError();
+}
+
+template <class M>
+hipError_t launch_group_fixed(int mode, const ReactParamsDev& P, double* y, const double* ysrc, double* rX,
+                              const double* rXsrc, const BoxArgs* b, double dt, int ncells, int cells_per_wave,
+                              CellStats st, hipStream_t s) {
+  using Tab = typename wave_tables<M>::type;
+  if constexpr (!std::is_void<Tab>::value && !has_qss<M>::value) {
+    GroupIO io{};
+    io.f = IO1D{y, ysrc, rX, rXsrc};
+    if (b) io.b = *b;
+    if (mode == MODE_RK64) {
+      if (ncells == 0) return hipSuccess;
+      switch (cells_per_wave) {
+        case 8:
+          if constexpr (group_ok<M, 8>())
+            return b ? launch_group_rk64<Tab, 8, true>(P, io, dt, ncells, st, s)
+                     : launch_group_rk64<Tab, 8, false>(P, io, dt, ncells, st, s);
+          break;
+        case 4:
+          if constexpr (group_ok<M, 16>())
+            return b ? launch_group_rk64<Tab, 16, true>(P, io, dt, ncells, st, s)
+                     : launch_group_rk64<Tab, 16, false>(P, io, dt, ncells, st, s);
+          break;
+        case 2:
+          if constexpr (group_ok<M, 32>())
+            return b ? launch_group_rk64<Tab, 32, true>(P, io, dt, ncells, st, s)
+                     : launch_group_rk64<Tab, 32, false>(P, io, dt, ncells, st, s);
+          break;
+        case 1:
+          if constexpr (group_ok<M, 64>())
+            return b ? launch_group_rk64<Tab, 64, true>(P, io, dt, ncells, st, s)
+                     : launch_group_rk64<Tab, 64, false>(P, io, dt, ncells, st, s);
+          break;
+        default:
+          break;
+      }
+      return hipErrorInvalidValue;
+    }
+    if constexpr (group_fixed_ok<M>()) {
+      if (mode == MODE_BDF) {
+        if (ncells == 0) return hipSuccess;
+        return b ? launch_group_bdf_fixed<Tab, true>(P, io, dt, ncells, st, s)
+                 : launch_group_bdf_fixed<Tab, false>(P, io, dt, ncells, st, s);
+      }
+    }
+  }
+  return hipErrorNotSupported;
+}
+
 template <class M>
 hipError_t launch_adjoint(const ReactParamsDev& P, const AdjointArgs& a, hipStream_t s) {
   using Tab = typename wave_tables<M>::type;
@@ -237,6 +306,13 @@ hipError_t launch_mech_eval(int what, const double* sc, const double* T, int nce
   template hipError_t launch_flatten<TYPE>(const FlatArgs&, int, hipStream_t);                   \
   template hipError_t launch_mech_eval<TYPE>(int, const double*, const double*, int, double*,     \
                                              hipStream_t);                                        \
+  }
+
+#define PPC_INSTANTIATE_GFIXED(TYPE, MODE)                                                             \
+  namespace ppc {                                                                                    \
+  template hipError_t launch_group_fixed<TYPE>(int, const ReactParamsDev&, double*, const double*, double*, \
+                                               const double*, const BoxArgs*, double, int, int, CellStats,  \
+                                               hipStream_t);                                          \
   }
 
 #define PPC_INSTANTIATE_ADJOINT(TYPE, MODE)                                                           \

@@ -29,6 +29,10 @@ hipError_t no_batched_1d(int, const ReactParamsDev&, double*, const double*, dou
                          QueueArgs, CellStats, hipStream_t) {
   return hipErrorInvalidValue;
 }
+hipError_t no_fixed(int, const ReactParamsDev&, double*, const double*, double*, const double*, const BoxArgs*, double,
+                    int, int, CellStats, hipStream_t) {
+  return hipErrorNotSupported;
+}
 hipError_t no_adjoint(const ReactParamsDev&, const AdjointArgs&, hipStream_t) { return hipErrorNotSupported; }
 long long no_ws(int) { return 0; }
 long long no_group(int) { return 0; }
@@ -38,7 +42,7 @@ hipError_t no_eval(int, const double*, const double*, int, double*, hipStream_t)
 template <int D>
 const MechLauncher* man_launcher() {
   static const MechLauncher L = {"Manifold", D + 1, 0, 0, &man_1d<D>, &man_box<D>, &no_batched_1d,
-                                 &no_adjoint, &no_ws, &no_group, &no_flatten, &no_eval};
+                                 &no_fixed, &no_adjoint, &no_ws, &no_group, &no_flatten, &no_eval};
   return &L;
 }
 
