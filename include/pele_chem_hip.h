@@ -90,9 +90,9 @@ typedef struct {
    * increment conservatively (pp_chem_flatten / pp_chem_unflatten). */
   int clean_init_massfrac;
   /* Batched forms: persistent waves per compute unit (0: every wave that fits,
-   * 8 at the kernels' 2 waves per SIMD) of the kernels the caller names
-   * (batched_cells_per_wave) and of the QSS mechanisms' one-cell-per-lane
-   * kernels; a tuning parameter (python -m pelephysics_amd.autotune). */
+   * 8 at the kernels' 2 waves per SIMD) of the group size the caller names
+   * (batched_cells_per_wave), not read otherwise; a tuning parameter
+   * (python -m pelephysics_amd.autotune). */
   int batched_waves_per_cu;
   /* Batched forms: a wave factors the Newton matrices of its waiting cells
    * together once batched_lu_batch cells (1..64) wait or a request has waited
@@ -102,10 +102,8 @@ typedef struct {
   /* Batched forms, box call: 0 or 1.  Both run box -> flat, the 1-D kernel,
    * flat -> box; results do not depend on it. */
   int batched_box_direct;
-  /* The kernel build a launch uses.  Batched forms: the one-cell-per-lane
-   * kernels of the QSS mechanisms held to 2 waves per SIMD (0 or 2, the
-   * default) or to 1 (more registers per lane, fewer spills; not with
-   * batched_box_direct = 1); the other mechanisms accept and do not read it.
+  /* The kernel build a launch uses.  Batched forms: 0, 1 (not with
+   * batched_box_direct = 1) or 2, not read: the group kernels have one build.
    * The plain adaptive BDF (PP_CHEM_BDF_ADAPTIVE): 0 (the compiler's choice),
    * 2 or 4.  The parity integrators: 0. */
   int batched_waves_per_simd;
@@ -114,7 +112,7 @@ typedef struct {
    * Newton-matrix rows, so its state stays in registers (table-driven
    * mechanism kernels only; the values a mechanism supports depend on its
    * size); 0 (default): the library chooses by the mechanism's size and the
-   * number of cells (QSS mechanisms: one cell per lane). */
+   * number of cells (the only choice for QSS mechanisms). */
   int batched_cells_per_wave;
   /* PP_CHEM_BDF_ADAPTIVE and PP_CHEM_CVODE (0 elsewhere): order cap 1..5
    * (cvode.max_order; 0: 5), Newton iterations per step attempt

@@ -336,8 +336,8 @@ int finish_with(pp_chem* h, int ncells, hipStream_t s, const ppc::CellStats& st,
 }
 
 bool is_batched(int mode) { return mode == ppc::MODE_BATCHED_MIXED || mode == ppc::MODE_BATCHED_FP64; }
-// Kernels of a mode: ReactorCvode runs the plain FP64 adaptive BDF with its
-// options (QSS mechanisms; the others its group form, gmode).
+// One-lane-per-cell kernels of a mode: ReactorCvode is the plain FP64 adaptive
+// BDF with its options (its calls run on the group form, gmode).
 int kmode(int mode) {
   return mode == PP_CHEM_CVODE ? ppc::MODE_ADAPTIVE : (mode == PP_CHEM_ARKODE ? ppc::MODE_ERK : mode);
 }
@@ -395,9 +395,8 @@ int auto_cells_per_wave(const pp_chem* h, long long ncells) {
   return cpw;
 }
 
-// The handle's calls run on the work queue: the batched forms, and ReactorCvode
-// where there are group kernels.
-bool on_queue(const pp_chem* h) { return is_batched(h->cfg.mode) || (h->cfg.mode == PP_CHEM_CVODE && h->GL); }
+// The handle's calls run on the work queue: the batched forms and ReactorCvode.
+bool on_queue(const pp_chem* h) { return is_batched(h->cfg.mode) || h->cfg.mode == PP_CHEM_CVODE; }
 // Batched kernels of the handle's mode.
 int gmode(const pp_chem* h) { return h->cfg.mode == PP_CHEM_CVODE ? ppc::MODE_GROUP_CVODE : h->cfg.mode; }
 
@@ -432,7 +431,7 @@ int fixed_cells_per_wave(const pp_chem* h, long long ncells) {
 
 // Cells per wave of this call's group kernel; 0: one lane per cell.
 int cells_per_wave(const pp_chem* h, long long ncells) {
-  if (!on_queue(h) || !h->GL) return 0;
+  if (!on_queue(h)) return 0;
   return h->cfg.batched_cells_per_wave != 0 ? h->cfg.batched_cells_per_wave : auto_cells_per_wave(h, ncells);
 }
 
@@ -445,8 +444,7 @@ int cells_per_wave(const pp_chem* h, long long ncells) {
 long long workspace_blocks(const pp_chem* h, long long ncells, int cpw, long long& rows) {
   rows = cpw ? h->GL->group_ws_rows(cpw) : h->L->ws_rows(kmode(h->cfg.mode));
   if (rows == 0 || ncells == 0) return 0;
-  const long long per_cu =
-      (cpw || (is_batched(h->cfg.mode) && h->cfg.batched_waves_per_simd != 1)) ? 8 : 4;
+  const long long per_cu = cpw ? 8 : 4;
   const long long lanes_per_cell = cpw ? 64 / cpw : 1;
   long long blocks = std::min<long long>((ncells * lanes_per_cell + 63) / 64, per_cu * std::max(h->ncu, 1));
   if (h->max_blocks > 0) blocks = std::min<long long>(blocks, h->max_blocks);
@@ -520,7 +518,7 @@ hipError_t enqueue_1d(pp_chem* h, double* y, double* ysrc, double* rX, double* r
   hipError_t e;
   if (on_queue(h)) {
     const ppc::QueueArgs q = prepare_queue(h, ncells, key, s);
-    e = (h->GL ? h->GL : h->L)->batched_1d(gmode(h), h->P, y, ysrc, rX, rXsrc, dt, q, counters(h), s);
+    e = h->GL->batched_1d(gmode(h), h->P, y, ysrc, rX, rXsrc, dt, q, counters(h), s);
   } else if (h->fixed_cpw) {
     e = h->GL->group_fixed(h->cfg.mode, h->P, y, ysrc, rX, rXsrc, nullptr, dt, ncells, h->fixed_cpw, counters(h), s);
   } else {
@@ -725,7 +723,8 @@ int pp_chem_create(const pp_chem_config* cfg, pp_chem** out) {
   if (cfg->batched_cells_per_wave != 0) {
     // a group kernel of this size must exist for the mechanism; box calls go through flat state
     if (!is_batched(cfg->mode) || cfg->batched_box_direct == 1) return PP_CHEM_EINVAL;
-    if (L->group_ws_rows(cfg->batched_cells_per_wave) <= 0) return PP_CHEM_EINVAL;
+    // (QSS mechanisms: the size is the library's choice)
+    if (L->group_ws_rows(cfg->batched_cells_per_wave) <= 0 || L->qss) return PP_CHEM_EINVAL;
   }
   const int bs = cfg->block_size > 0 ? cfg->block_size : 64;
   if (bs > 64 || bs % 64 != 0) return PP_CHEM_EINVAL;  // kernels are built for 64-lane blocks
@@ -767,9 +766,8 @@ int pp_chem_create(const pp_chem_config* cfg, pp_chem** out) {
   }
   hipError_t e = hipGetDevice(&h->device);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&h->ncu, hipDeviceAttributeMultiprocessorCount, h->device);
-  // persistent-grid bound of the kernels it was chosen for: the
-  // one-lane-per-cell ones, or the group size the caller names
-  if (cfg->batched_waves_per_cu > 0 && (!h->GL || cfg->batched_cells_per_wave != 0))
+  // persistent-grid bound of the group size it was chosen for
+  if (cfg->batched_waves_per_cu > 0 && cfg->batched_cells_per_wave != 0)
     h->max_blocks = cfg->batched_waves_per_cu * h->ncu;  // 64-lane waves
   // one allocation: the accumulators, the queue and the failure count
   constexpr size_t red_bytes = sizeof(unsigned long long) * (NSTAT + 1), queue_ints = 1 + 2 * NBINS;
@@ -1135,7 +1133,7 @@ int pp_chem_react_1d_noalloc(pp_chem* h, double* y, double* ysrc, double* rX, do
     if (on_queue(h)) {
       hipLaunchKernelGGL(zero_ints, dim3(1), dim3(64), 0, s, counter, 1);
       const ppc::QueueArgs q{nullptr, counter, ncells, h->max_blocks};  // cells in index order
-      e = (h->GL ? h->GL : h->L)->batched_1d(gmode(h), P, y, ysrc, rX, rXsrc, *dt_react, q, st, s);
+      e = h->GL->batched_1d(gmode(h), P, y, ysrc, rX, rXsrc, *dt_react, q, st, s);
     } else if (const int fcpw = fixed_cells_per_wave(h, ncells)) {
       e = h->GL->group_fixed(h->cfg.mode, P, y, ysrc, rX, rXsrc, nullptr, *dt_react, ncells, fcpw, st, s);
     } else {

@@ -22,14 +22,10 @@
 // the QSS concentration factored out, eliminated by the program the table
 // generator wrote), then evaluates all reactions with those concentrations.
 #pragma once
-#include "ppc_common.h"
+#include "pack.h"
 #include "dual.h"
 
 namespace ppc {
-
-// regularisation of the QSS balances (comp_sc_qss epsilon of the reference's
-// generated QSS mechanisms)
-constexpr double QSS_EPS = 1e-12;
 
 template <class T>
 struct TabMech {
@@ -591,6 +587,65 @@ struct TabMech {
     J[n * n - 1] = -tmp1 + tmp2 * dcmixdT - tmp3 * dehmixdT;
   }
 
+  // The derivatives of the QSS balances by the transported concentrations that
+  // come from QSS reaction i (the i-th of qRx): addG(row * NS + k, v) for each,
+  // and its forward and reverse rates, all with the QSS concentrations (1 in
+  // sc1, b1 with them) factored out; x: those concentrations.
+  template <class AG>
+  PPC_DI static void qss_balance_terms(const int i, const double* sc1, const double* a, const double* b1,
+                                       const double* x, const double mixture, const double Tv, const double invT,
+                                       const double logT, const double refC, const double refCinv, double& qf,
+                                       double& qr, const AG& addG) {
+    const int j = T::qRx_(i);
+    double dlnc, kfc;
+    rate_any<true>(j, sc1, a, b1, mixture, Tv, invT, logT, refC, refCinv, qf, qr, dlnc, kfc);
+    const bool tb = j >= T::N_EL;
+    // k_r corr = kfc refC^delta prod a_reactants / prod a_products
+    double krc = 0.0;
+    if (T::rxRev_(j)) {
+      krc = kfc * refc_pow(T::rxDelta_(j), refC, refCinv);
+      for (int l = 0; l < 3; ++l) {
+        const int r = T::rxR_(3 * j + l), p = T::rxP_(3 * j + l);
+        if (r >= 0) krc *= a[r];
+        if (p >= 0) krc /= a[p];
+      }
+    }
+#pragma unroll 1
+    for (int t = T::qTermPtr_(i); t < T::qTermPtr_(i + 1); ++t) {
+      const int dir = T::tDir_(t), row = T::tRow_(t), cq = T::tCol_(t);
+      if (dir == 0 && T::rxFwdOff_(j)) continue;
+      const double w = cq < 0 ? -T::tMul_(t) : T::tMul_(t) * x[cq];
+      const double qco = dir ? qr : qf;
+      const double kd = dir ? krc : kfc;
+      int sl[3];
+      for (int l = 0; l < 3; ++l) sl[l] = dir ? T::rxP_(3 * j + l) : T::rxR_(3 * j + l);
+      for (int l = 0; l < 3; ++l) {
+        const int k = sl[l];
+        if (k < 0 || k >= NS || (l > 0 && k == sl[l - 1])) continue;
+        int mult = 0;
+        double rest = 1.0;
+        for (int u = 0; u < 3; ++u) {
+          if (sl[u] < 0) continue;
+          if (sl[u] == k) {
+            if (mult > 0) rest *= sc1[k];
+            ++mult;
+          } else {
+            rest *= sc1[sl[u]];
+          }
+        }
+        addG(row * NS + k, w * kd * (double)mult * rest);
+      }
+      if (tb) {
+        const double d = w * dlnc * qco;
+#pragma unroll 1
+        for (int k = 0; k < NS; ++k) addG(row * NS + k, d);
+        const int e0 = T::rxEff0_(j), en = T::rxEffN_(j);
+#pragma unroll 1
+        for (int e = 0; e < en; ++e) addG(row * NS + T::effK_(e0 + e), T::effV_(e0 + e) * d);
+      }
+    }
+  }
+
   // QSS mechanisms: the species block is the exact derivative of the
   // QSS-reduced production rates (the reference differentiates the same
   // expressions symbolically, Support/ceptr/ceptr/jacobian.py ajac_symbolic):
@@ -640,54 +695,9 @@ struct TabMech {
     for (int i = 0; i < NQ * NS; ++i) G[i] = 0.0;
 #pragma unroll 1
     for (int i = 0; i < T::NQR; ++i) {
-      const int j = T::qRx_(i);
-      double qf, qr, dlnc, kfc;
-      rate_any<true>(j, sc1, a, b1, mixture, Tv, invT, logT, refC, refCinv, qf, qr, dlnc, kfc);
-      const bool tb = j >= T::N_EL;
-      // k_r corr = kfc refC^delta prod a_reactants / prod a_products
-      double krc = 0.0;
-      if (T::rxRev_(j)) {
-        krc = kfc * refc_pow(T::rxDelta_(j), refC, refCinv);
-        for (int l = 0; l < 3; ++l) {
-          const int r = T::rxR_(3 * j + l), p = T::rxP_(3 * j + l);
-          if (r >= 0) krc *= a[r];
-          if (p >= 0) krc /= a[p];
-        }
-      }
-#pragma unroll 1
-      for (int t = T::qTermPtr_(i); t < T::qTermPtr_(i + 1); ++t) {
-        const int dir = T::tDir_(t), row = T::tRow_(t), cq = T::tCol_(t);
-        if (dir == 0 && T::rxFwdOff_(j)) continue;
-        const double w = cq < 0 ? -T::tMul_(t) : T::tMul_(t) * x[cq];
-        const double qco = dir ? qr : qf;
-        const double kd = dir ? krc : kfc;
-        int sl[3];
-        for (int l = 0; l < 3; ++l) sl[l] = dir ? T::rxP_(3 * j + l) : T::rxR_(3 * j + l);
-        for (int l = 0; l < 3; ++l) {
-          const int k = sl[l];
-          if (k < 0 || k >= NS || (l > 0 && k == sl[l - 1])) continue;
-          int mult = 0;
-          double rest = 1.0;
-          for (int u = 0; u < 3; ++u) {
-            if (sl[u] < 0) continue;
-            if (sl[u] == k) {
-              if (mult > 0) rest *= sc1[k];
-              ++mult;
-            } else {
-              rest *= sc1[sl[u]];
-            }
-          }
-          G[row * NS + k] += w * kd * (double)mult * rest;
-        }
-        if (tb) {
-          const double d = w * dlnc * qco;
-#pragma unroll 1
-          for (int k = 0; k < NS; ++k) G[row * NS + k] += d;
-          const int e0 = T::rxEff0_(j), en = T::rxEffN_(j);
-#pragma unroll 1
-          for (int e = 0; e < en; ++e) G[row * NS + T::effK_(e0 + e)] += T::effV_(e0 + e) * d;
-        }
-      }
+      double qf, qr;
+      qss_balance_terms(i, sc1, a, b1, x, mixture, Tv, invT, logT, refC, refCinv, qf, qr,
+                        [&](int idx, double v) { G[idx] += v; });
     }
     // X = -A^-1 G, column by column, in place
 #pragma unroll 1

@@ -32,18 +32,19 @@
 // 105000.  Measured (one MI355X, box or 1-D call of 1e-5 s at rtol 1e-10, state
 // restored before each call), against one cell per lane: drm19 64^3 cells 222 ->
 // 70 ms, 2898 cells 95 -> 5.9 ms; dodecane_lu 10000 cells 1558 -> 13.6 ms;
-// heptane_lu_88sk 2048 cells, 1e-6 s at rtol 1e-8, 1169 -> 11.0 ms.
+// heptane_lu_88sk 2048 cells, 1e-6 s at rtol 1e-8, 1169 -> 11.0 ms;
+// LuEthylene_qss 4096 cells 198 -> 7.4 ms.
 //
 // Every group reduction returns the bitwise-identical value in all lanes of
 // the group (pairs are always added in commuted order on both partners), so
 // the integrator's control flow is uniform within a group.  Different groups
-// of a wave follow their own cells; as in batched.h every trip of the
+// of a wave follow their own cells; every trip of the
 // persistent loop evaluates one right-hand side for every group that is not
 // waiting for a factorisation, and the groups' LU requests are served together
 // once enough of them wait.  A cell's arithmetic does not depend on which
 // groups share its wave, so results do not depend on the queue's order.
 //
-// The step / order / Newton logic is that of batched_kernel (batched.h), the
+// The step / order / Newton logic is that of adaptive_cell (reactors.h), the
 // NDF family of SciPy's BDF integrator; every loop over a cell's work is
 // bounded (queue length, RHS budget, the 200-iteration temperature inversion).
 // The algorithm follows SciPy's scipy/integrate/_ivp/bdf.py (BSD-3-Clause,
@@ -53,10 +54,20 @@
 #include "chem_table.h"
 #include "reactors.h"
 #include "wave.h"
-#include "batched.h"
 #include "pack.h"
 
 namespace ppc {
+
+// Cell input/output of the 1-D (YCOrder) form.
+struct IO1D {
+  double* y;
+  const double* ysrc;
+  double* rX;
+  const double* rXsrc;
+};
+
+// phases of a cell's integration
+enum : int { PH_F0 = 0, PH_F1 = 1, PH_NEWTON = 2 };
 
 // ------------------------------------------------ group lane primitives --
 template <int G>
@@ -190,6 +201,7 @@ struct PackTab : T {
   PPC_DI static int rxP_(int i) { return sp(lds_pack<T>().rx[i / 3].p[i % 3]); }
   PPC_DI static int rxDelta_(int j) { return lds_pack<T>().rx[j].delta; }
   PPC_DI static int rxRev_(int j) { return lds_pack<T>().rx[j].flags & 1; }
+  PPC_DI static int rxFwdOff_(int j) { return lds_pack<T>().rx[j].flags & 2; }
   PPC_DI static int rxNet_(int i) {
     return T::rxNet_(T::MAXNET * (int)lds_pack<T>().perm[i / T::MAXNET] + i % T::MAXNET);
   }
@@ -220,6 +232,7 @@ struct GroupChem {
   static constexpr int NG = 64 / G;
   static constexpr int EPL = (n + G - 1) / G;    // equation slots per lane
   static constexpr int SPL = (NS + G - 1) / G;   // species slots per lane
+  static constexpr int SPX = (NX + G - 1) / G;   // with the QSS species
   static constexpr int TL = NS % G, TS = NS / G;  // lane and slot of the temperature equation
   static constexpr int NP = (n + 1) & ~1;        // vectors of n, 16-byte aligned
 
@@ -230,13 +243,21 @@ struct GroupChem {
   // the groups' broadcasts fall into different banks.
   static constexpr int cmax(int a, int b) { return a > b ? a : b; }
   static constexpr int S_CA = 0, S_B = 2 * (NX + 1);
-  static constexpr int S_Q = (cmax(3 * (NX + 1), NCH) + 1) & ~1;
-  static constexpr int S_RAW = S_Q + cmax(NR + 1, 3 * NP);
+  static constexpr int NQ = T::NQ, NROW = NQ > 0 ? T::NSLOT + NQ : 0;  // QSS balances: entries and right-hand sides
+  static constexpr int S_Q = (cmax(cmax(3 * (NX + 1), NCH), 2 * (NX + 1) + NROW) + 1) & ~1;
+  static constexpr int NRATE = NQ > 0 ? 2 * NR + 1 : NR + 1;  // QSS: forward and reverse rates apart
+  static constexpr int S_RAW = S_Q + cmax(NRATE, 3 * NP);
   static constexpr int AREA = ((S_RAW + 3) / 8) * 8 + 4;
   // The wave's Jacobian area overlays its groups' areas: 5 species vectors and,
   // where n is small enough, the n x n accumulator.
-  static constexpr bool JLDS = n <= 32;
+  // (QSS mechanisms: each group works on its own cell's Jacobian, in the workspace.)
+  static constexpr bool JLDS = n <= 32 && NQ == 0;
   static constexpr int J_AT = (5 * NP + 1) & ~1;
+  // Jacobian accumulators in the workspace (doubles): n x n (JSQ) of the wave,
+  // or of each group with the QSS terms after it (JSTRIDE); of a wave
+  static constexpr int JSQ = (n * n + 1) & ~1;
+  static constexpr int JSTRIDE = NQ > 0 ? (JSQ + NQ * NS + 2 * T::NQR + 1) & ~1 : JSQ;
+  static constexpr int JSPACE = NQ > 0 ? NG * JSTRIDE : JSTRIDE;
   static constexpr int WAREA = (cmax(NG * AREA, J_AT + (JLDS ? n * n : 0)) + 3) & ~3;
 
   PPC_DI static void coefs(const PK& pk, const int k, const double Tv, double (&a)[7], double& imw) {
@@ -340,12 +361,13 @@ struct GroupChem {
     return r;
   }
 
-  // net rate of progress of reaction j (packed order) of KIND (0 elementary, 1
-  // three-body, 2 Troe, 3 Lindemann falloff) from the group's LDS area
+  // rate of progress of reaction j (packed order) of KIND (0 elementary, 1
+  // three-body, 2 Troe, 3 Lindemann falloff) from the group's LDS area: net
+  // into q[j], or (QSS mechanisms) forward into q[j] and reverse into q[NR + j]
   template <int KIND>
-  PPC_DI static double rate(const PK& pk, const double* ca, const double* b, const int j, const double mixture,
-                            const double Tv, const double invT, const double logT, const double refC,
-                            const double refCinv) {
+  PPC_DI static void rate(const PK& pk, const double* ca, const double* b, double* q, const int j,
+                          const double mixture, const double Tv, const double invT, const double logT,
+                          const double refC, const double refCinv) {
     const tab::PackRx rx = pk.rx[j];
     const double kf0 = rx.A * exp(rx.b * logT - rx.E * invT);
     double kf = kf0;
@@ -389,17 +411,74 @@ struct GroupChem {
       qr = kf * refc_pow(rx.delta, refC, refCinv) * a0 * b[rx.p[0]] * a1 * a2 * b[rx.p[1]];
       if (p2 != NX) qr *= b[p2];
     }
-    return qf - qr;
+    if constexpr (NQ > 0) {
+      q[j] = rx.flags & 2 ? 0.0 : qf;
+      q[NR + j] = qr;
+    } else {
+      q[j] = qf - qr;
+    }
   }
 
-  // fKernelSpec (Source/Reactions/ReactorUtils.H:358-415) for the group's
-  // cell: y (this lane's equation slots), f = ydot of the same slots.
-  PPC_DI static void rhs(const PK& pk, double* sh, const int g, const bool eform, const double dt_save,
-                         const double (&y)[EPL], const double (&src)[SPL], const double rhoe_init,
-                         const double rhoesrc_ext, double (&f)[EPL]) {
-    double hk[SPL], cs;
-    const double Tv = T_from_energy(pk, g, eform, rhoe_init + rhoesrc_ext * dt_save, y, Gr::bcast(y[TS], TL), cs, hk);
-    const double invT = 1.0 / Tv, logT = log(Tv), RT = RU * Tv;
+  // sum of the terms of one chunk over the values in q
+  PPC_DI static double chunk(const tab::PackCh& ch, const double* q) {
+    double w = 0.0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w += (double)((int)(ch.e[i] >> 12) - 8) * q[ch.e[i] & 0xfff];
+    return w;
+  }
+
+  // QSS mechanisms: q holds the forward and reverse rates with the QSS
+  // concentrations factored out.  Assembles the balances a row per lane (rows:
+  // over the product exponentials, which are done with), solves them on
+  // registers in every lane, puts the concentrations into ca, and makes q the
+  // net rates.
+  PPC_DI static void qss(const PK& pk, double* ca, double* q, double* rows, const int g) {
+    if constexpr (NQ > 0) {
+      wave_sync();
+#pragma unroll 1
+      for (int r = g; r < NROW; r += G) {
+        double w = pk.qInit[r];
+        const int v1 = pk.qRow[r + 1];
+#pragma unroll 1
+        for (int v = pk.qRow[r]; v < v1; ++v) w += chunk(pk.qch[v], q);
+        rows[r] = w;
+      }
+      wave_sync();
+      double A[T::NSLOT], x[NQ];
+#pragma unroll
+      for (int i = 0; i < T::NSLOT; ++i) A[i] = rows[i];
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) x[i] = rows[T::NSLOT + i];
+      T::qss_eliminate(A, x);
+#pragma unroll
+      for (int i = 0; i < NQ; ++i)
+        if (g == i % G) ca[2 * (NS + i)] = x[i];
+      wave_sync();
+#pragma unroll 2
+      for (int j = g; j < NR; j += G) {
+        const tab::PackRx& rx = pk.rx[j];
+        double f = q[j], r = q[NR + j];
+#pragma unroll
+        for (int l = 0; l < 3; ++l) {
+          const int kr = rx.r[l], kp = rx.p[l];
+          if (kr >= NS && kr < NX) f *= ca[2 * kr];
+          if (kp >= NS && kp < NX) r *= ca[2 * kp];
+        }
+        q[j] = f - r;
+      }
+      if (g == 0) q[NR] = 0.0;
+    }
+  }
+
+  // w = production rates (mol/m^3/s) of this lane's species slots at Tv and the
+  // densities y; hk[e] *= RT / molecular weight.  The group's LDS area is
+  // overwritten; keep() runs when the rates are in q, the concentrations (the
+  // QSS ones included) in ca and the QSS balances in b.
+  template <class KEEP>
+  PPC_DI static void production(const PK& pk, double* sh, const int g, const double Tv, const double invT,
+                                const double (&y)[EPL], const double RT, double (&hk)[SPL], double (&w)[SPL],
+                                const KEEP& keep) {
+    const double logT = log(Tv);
     double* ca = sh + S_CA;
     double* b = sh + S_B;
     double* q = sh + S_Q;
@@ -408,54 +487,73 @@ struct GroupChem {
       ca[2 * NX] = 1.0;
       ca[2 * NX + 1] = 1.0;
       b[NX] = 1.0;
-      q[NR] = 0.0;
+      q[NRATE - 1] = 0.0;
     }
 #pragma unroll
-    for (int e = 0; e < SPL; ++e) {
+    for (int e = 0; e < SPX; ++e) {
       const int k = e * G + g;
-      if (k < NS) {
-        double a[7], imw;
+      if (k < NX) {
+        double a[7], imw, sc = 1.0;  // QSS species: concentration factored out
         coefs(pk, k, Tv, a, imw);
-        hk[e] *= RT * imw;  // CKUMS / CKHMS
-        const double sc = (y[e] * imw) * 1.0e6;  // CKYTCR, SI
+        if (k < NS) {
+          hk[e < SPL ? e : 0] *= RT * imw;  // CKUMS / CKHMS
+          sc = (y[e < EPL ? e : 0] * imw) * 1.0e6;  // CKYTCR, SI
+        }
         const double eg = exp(TM::g_poly(a, Tv, invT, logT));
         ca[2 * k] = sc;
         ca[2 * k + 1] = 1.0 / eg;
         b[k] = sc * eg;
-        msum += sc;
+        if (k < NS) msum += sc;
       }
     }
     const double mixture = Gr::sum(msum);
     const double refC = 101325.0 / 8.31446 * invT, refCinv = 1.0 / refC;
     wave_sync();
 #pragma unroll 1
-    for (int j = g; j < T::N_EL; j += G) q[j] = rate<0>(pk, ca, b, j, mixture, Tv, invT, logT, refC, refCinv);
+    for (int j = g; j < T::N_EL; j += G) rate<0>(pk, ca, b, q, j, mixture, Tv, invT, logT, refC, refCinv);
     if constexpr (T::N_TB > 0) {
 #pragma unroll 1
       for (int j = T::N_EL + g; j < T::N_EL + T::N_TB; j += G)
-        q[j] = rate<1>(pk, ca, b, j, mixture, Tv, invT, logT, refC, refCinv);
+        rate<1>(pk, ca, b, q, j, mixture, Tv, invT, logT, refC, refCinv);
     }
     if constexpr (T::N_TROE > 0) {
 #pragma unroll 1
       for (int j = T::N_EL + T::N_TB + g; j < NR - T::N_LIND; j += G)
-        q[j] = rate<2>(pk, ca, b, j, mixture, Tv, invT, logT, refC, refCinv);
+        rate<2>(pk, ca, b, q, j, mixture, Tv, invT, logT, refC, refCinv);
     }
     if constexpr (T::N_LIND > 0) {
 #pragma unroll 1
       for (int j = NR - T::N_LIND + g; j < NR; j += G)
-        q[j] = rate<3>(pk, ca, b, j, mixture, Tv, invT, logT, refC, refCinv);
+        rate<3>(pk, ca, b, q, j, mixture, Tv, invT, logT, refC, refCinv);
     }
+    qss(pk, ca, q, b, g);
     wave_sync();
+    keep();
     double* part = sh;
 #pragma unroll 1
-    for (int v = g; v < NCH; v += G) {
-      const tab::PackCh ch = pk.ch[v];
-      double w = 0.0;
+    for (int v = g; v < NCH; v += G) part[v] = chunk(pk.ch[v], q);
+    wave_sync();
 #pragma unroll
-      for (int i = 0; i < 8; ++i) w += (double)((int)(ch.e[i] >> 12) - 8) * q[ch.e[i] & 0xfff];
-      part[v] = w;
+    for (int e = 0; e < SPL; ++e) {
+      const int k = e * G + g;
+      w[e] = 0.0;
+      if (k < NS) {
+        const int v1 = pk.spCh[k + 1];
+#pragma unroll 2
+        for (int v = pk.spCh[k]; v < v1; ++v) w[e] += part[v];
+      }
     }
     wave_sync();
+  }
+
+  // fKernelSpec (Source/Reactions/ReactorUtils.H:358-415) for the group's
+  // cell: y (this lane's equation slots), f = ydot of the same slots.
+  PPC_DI static void rhs(const PK& pk, double* sh, const int g, const bool eform, const double dt_save,
+                         const double (&y)[EPL], const double (&src)[SPL], const double rhoe_init,
+                         const double rhoesrc_ext, double (&f)[EPL]) {
+    double hk[SPL], cs, w[SPL];
+    const double Tv = T_from_energy(pk, g, eform, rhoe_init + rhoesrc_ext * dt_save, y, Gr::bcast(y[TS], TL), cs, hk);
+    production(pk, sh, g, Tv, 1.0 / Tv, y, RU * Tv, hk, w, [] {});
     double esum = 0.0;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) f[e] = 0.0;
@@ -463,16 +561,11 @@ struct GroupChem {
     for (int e = 0; e < SPL; ++e) {
       const int k = e * G + g;
       if (k < NS) {
-        double w = 0.0;
-        const int v1 = pk.spCh[k + 1];
-#pragma unroll 2
-        for (int v = pk.spCh[k]; v < v1; ++v) w += part[v];
-        const double s = w * 1.0e-6 * pk.mw[k] + src[e];  // RTY2WDOT (CKWC units) + source
+        const double s = w[e] * 1.0e-6 * pk.mw[k] + src[e];  // RTY2WDOT (CKWC units) + source
         f[e] = s;
         esum += s * hk[e];
       }
     }
-    wave_sync();
     const double srcT = rhoesrc_ext - Gr::sum(esum);
     if (g == TL) f[TS] = srcT / (cs * RU);
   }
@@ -600,6 +693,173 @@ struct GroupChem {
     }
   }
 };
+
+// The QSS mechanisms' Jacobian (TabMech::jacobian_qss) of a group's cell by its
+// lanes: y in the group's LDS area sh, which is overwritten; J (n x n, column
+// major) in the workspace, followed by the derivatives of the balances
+// (NQ x NS) and the QSS reactions' rates (2 NQR).  Reactions are split over the
+// lanes, with atomic sums; the QSS solves, and d wdot / d x, over the columns.
+// Out of line: it is rare (about one per cell and call) and must not weigh on
+// the registers of the steps.  By one lane per cell it was 90% of a call
+// (LuEthylene_qss, 4096 cells, 1e-5 s: 14 ms per Jacobian).
+template <class T, int G>
+__device__ __noinline__ void group_qss_jacobian(double* sh, double* J, const bool eform) {
+  using C = GroupChem<T, G>;
+  using Gr = Grp<G>;
+  using TM = TabMech<PackTab<T>>;
+  constexpr int NS = T::NS, n = T::NEQ, NX = T::NX, NQ = T::NQ, SPL = C::SPL, SPX = C::SPX, NROW = C::NROW;
+  constexpr int RPL = (NROW + G - 1) / G;
+  static_assert(6 * NX + NROW <= C::AREA, "the Jacobian's vectors fit the group's area");
+  const typename T::Packed& pk = lds_pack<T>();
+  const int g = Gr::lane();
+  double* const X = J + C::JSQ;
+  double* const qq = X + NQ * NS;
+  double y[C::EPL], w1[SPL], w0[SPL] = {}, hk[SPL], sce[SPX], rw[RPL];
+  const double Tv = sh[NS];
+#pragma unroll
+  for (int e = 0; e < C::EPL; ++e) y[e] = e * G + g < n ? sh[e * G + g] : 0.0;
+#pragma unroll 1
+  for (int i = g; i < C::JSQ + NQ * NS; i += G) ws_store(J + i, 0.0);
+  wave_sync();
+  // the rates at T + 1e-2 K (temperature column), then at T
+#pragma unroll 1
+  for (int pass = 0; pass < 2; ++pass) {
+    const double Tq = pass == 0 ? Tv + 1.0e-2 : Tv;
+#pragma unroll
+    for (int e = 0; e < SPL; ++e) {
+      w1[e] = w0[e];
+      hk[e] = 0.0;
+    }
+    C::production(pk, sh, g, Tq, 1.0 / Tq, y, 1.0, hk, w0, [&] {
+#pragma unroll
+      for (int e = 0; e < SPX; ++e) sce[e] = e * G + g < NX ? sh[C::S_CA + 2 * (e * G + g)] : 0.0;
+#pragma unroll
+      for (int e = 0; e < RPL; ++e) rw[e] = e * G + g < NROW ? sh[C::S_B + e * G + g] : 0.0;
+      wave_sync();
+    });
+  }
+  double *c = sh, *gk = sh + NX, *hh = sh + 2 * NX, *c1 = sh + 3 * NX, *a = sh + 4 * NX, *b1 = sh + 5 * NX;
+  double* const rows = sh + 6 * NX;
+  const double invT = 1.0 / Tv, invT2 = invT * invT, logT = log(Tv);
+  const double refC = 101325.0 / 8.31446 * invT, refCinv = 1.0 / refC;
+  double cR[SPL], dcR[SPL], eh[SPL];
+  double msum = 0.0;
+#pragma unroll
+  for (int e = 0; e < SPX; ++e) {
+    const int k = e * G + g;
+    if (k < NX) {
+      double p[7], imw;
+      C::coefs(pk, k, Tv, p, imw);
+      const double gr = TM::g_poly(p, Tv, invT, logT), hr = TM::h_poly(p, Tv, invT), eg = exp(gr);
+      const double s1 = k < NS ? sce[e] : 1.0;
+      c[k] = sce[e];
+      gk[k] = gr;
+      hh[k] = hr;
+      c1[k] = s1;
+      a[k] = 1.0 / eg;
+      b1[k] = s1 * eg;
+      if (e < SPL) {
+        const double cp = TM::cp_poly(p, Tv);
+        cR[e < SPL ? e : 0] = eform ? cp - 1.0 : cp;
+        dcR[e < SPL ? e : 0] = TM::dcp_poly(p, Tv);
+        eh[e < SPL ? e : 0] = eform ? hr - 1.0 : hr;
+      }
+      if (k < NS) msum += sce[e];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < RPL; ++e)
+    if (e * G + g < NROW) rows[e * G + g] = rw[e];
+  const double mixture = Gr::sum(msum);
+  __threadfence();
+  wave_sync();
+  const double* const x = c + NS;
+#pragma unroll 1
+  for (int i = g; i < T::NQR; i += G) {
+    double qf, qr;
+    TabMech<T>::qss_balance_terms(i, c1, a, b1, x, mixture, Tv, invT, logT, refC, refCinv, qf, qr,
+                                  [&](int idx, double v) { unsafeAtomicAdd(X + idx, v); });
+    ws_store(qq + 2 * i, qf);
+    ws_store(qq + 2 * i + 1, qr);
+  }
+#pragma unroll 1
+  for (int j = g; j < T::NR; j += G)
+    TM::template jac_reaction<0>(
+        j, c, gk, hh, mixture, Tv, invT, invT2, logT, refC, refCinv,
+        [&](int idx, double v) {
+          if (idx < NS * n) unsafeAtomicAdd(J + idx, v);
+        },
+        [&](int, double) {});
+  __threadfence();
+  wave_sync();
+  // d x / d c = -A^-1 d(balance)/d c and J += (d wdot / d x)(d x / d c), a column a lane
+#pragma unroll 1
+  for (int k = g; k < NS; k += G) {
+    double A[T::NSLOT], col[NQ];
+#pragma unroll
+    for (int i = 0; i < T::NSLOT; ++i) A[i] = rows[i];
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) col[i] = -ws_load(X + i * NS + k);
+    T::qss_eliminate(A, col);
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) ws_store(X + i * NS + k, col[i]);
+    double* const Jk = J + k * n;
+#pragma unroll 2
+    for (int i = 0; i < T::NQR; ++i) {
+      const int j = T::qRx_(i);
+      int qR = -1, qP = -1;
+#pragma unroll
+      for (int l = 0; l < 3; ++l) {
+        const int r = T::rxR_(3 * j + l), p = T::rxP_(3 * j + l);
+        if (r >= NS) qR = r - NS;
+        if (p >= NS) qP = p - NS;
+      }
+      if (T::rxFwdOff_(j)) qR = -1;
+      if (!T::rxRev_(j)) qP = -1;
+      double d = 0.0;
+      if (qR >= 0) d += ws_load(qq + 2 * i) * ws_load(X + qR * NS + k);
+      if (qP >= 0) d -= ws_load(qq + 2 * i + 1) * ws_load(X + qP * NS + k);
+#pragma unroll 1
+      for (int l = 0; l < T::MAXNET; ++l) {
+        const int m = T::rxNet_(T::MAXNET * j + l);
+        if (m < 0) break;
+        unsafeAtomicAdd(Jk + m, T::rxNu_(T::MAXNET * j + l) * d);
+      }
+    }
+  }
+  __threadfence();
+  wave_sync();
+  // temperature column and row
+  double s_cm = 0.0, s_dcm = 0.0, s_eh = 0.0, s_deh = 0.0;
+#pragma unroll
+  for (int e = 0; e < SPL; ++e) {
+    const int k = e * G + g;
+    if (k < NS) {
+      const double dT = (w1[e] - w0[e]) / 1.0e-2;
+      ws_store(J + NS * n + k, dT);
+      s_cm += cR[e] * sce[e];
+      s_dcm += dcR[e] * sce[e];
+      s_eh += eh[e] * w0[e];
+      s_deh += invT * (cR[e] - eh[e]) * w0[e] + eh[e] * dT;
+    }
+  }
+  const double cmix = Gr::sum(s_cm), dcmixdT = Gr::sum(s_dcm);
+  const double ehmix = Gr::sum(s_eh), dehmixdT = Gr::sum(s_deh);
+  const double cmixinv = 1.0 / cmix;
+  const double tmp1 = ehmix * cmixinv, tmp3 = cmixinv * Tv, tmp2 = tmp1 * tmp3;
+#pragma unroll 1
+  for (int k = g, e = 0; k < NS; k += G, ++e) {
+    double d = 0.0, ck = 0.0;
+#pragma unroll 8
+    for (int m = 0; m < NS; ++m) d += (eform ? hh[m] - 1.0 : hh[m]) * ws_load(J + k * n + m);
+#pragma unroll
+    for (int u = 0; u < SPL; ++u) ck = u == e ? cR[u] : ck;
+    ws_store(J + k * n + NS, tmp2 * ck - tmp3 * d);
+  }
+  if (g == 0) ws_store(J + n * n - 1, -tmp1 + tmp2 * dcmixdT - tmp3 * dehmixdT);
+  __threadfence();
+  wave_sync();
+}
 
 // ------------------------------------------- group Newton-matrix inverse --
 // Gauss-Jordan exchange steps on the row-distributed n x n matrix a (lane g
@@ -761,15 +1021,17 @@ PPC_DI double ten_ulps(const double t) {
 }
 
 // Doubles of device workspace per wave: the Jacobian accumulator of the larger
-// mechanisms and the groups' Jacobian rows in JT.
-template <int n, int G, typename JT>
+// mechanisms (of every group's cell for the QSS ones) and the groups' Jacobian
+// rows in JT.
+template <class T, int G, typename JT>
 constexpr long long group_ws_doubles() {
+  constexpr int n = T::NEQ;
   constexpr long long epl = (n + G - 1) / G;
-  return (long long)((n * n + 1) & ~1) + (64 / G) * ((epl * n * G * (long long)sizeof(JT) + 15) / 16 * 2);
+  return GroupChem<T, G>::JSPACE + (64 / G) * ((epl * n * G * (long long)sizeof(JT) + 15) / 16 * 2);
 }
 
 // Persistent kernel: each group of G lanes integrates cells from the queue
-// until it is empty.  P.ws holds group_ws_doubles<NEQ, G, LU_T>() doubles for
+// until it is empty.  P.ws holds group_ws_doubles<T, G, LU_T>() doubles for
 // each of P.ws_lanes / 64 waves; waves beyond that leave at once.
 //
 // CV: ReactorCvode's options (AdaptParamsDev), as adaptive_cell takes them: the
@@ -798,9 +1060,9 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
   LU_T* const prow = reinterpret_cast<LU_T*>(sw + NP);
   constexpr long long GROWS = (long long)EPL * n * G;
   constexpr long long GSTRIDE = (GROWS * (long long)sizeof(LU_T) + 15) / 16 * 16 / (long long)sizeof(LU_T);
-  double* const Jw = C::JLDS ? wa + C::J_AT : P.ws + wid * group_ws_doubles<n, G, LU_T>();
+  double* const Jw = C::JLDS ? wa + C::J_AT : P.ws + wid * group_ws_doubles<T, G, LU_T>();
   // the groups' Jacobian rows: element (e, j) of lane g at [(e * n + j) * G + g]
-  LU_T* const rows = reinterpret_cast<LU_T*>(P.ws + wid * group_ws_doubles<n, G, LU_T>() + ((n * n + 1) & ~1));
+  LU_T* const rows = reinterpret_cast<LU_T*>(P.ws + wid * group_ws_doubles<T, G, LU_T>() + C::JSPACE);
   const LU_T* const jrow = rows + gi * GSTRIDE + g;
 
   const AdaptParamsDev& ap = P.adapt;
@@ -949,7 +1211,34 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
   while (__ballot(active)) {
     // ---- Jacobian requests, one cell at a time by the whole wave
     unsigned long long jreq = __ballot(active && need_jac != 0 && g == 0);
-    while (__builtin_expect(jreq != 0, 0)) {
+    if constexpr (T::NQ > 0) {
+      if (__builtin_expect(jreq != 0, 0)) {
+        const bool mine = active && need_jac != 0;
+        double* const Jq = Jw + (long long)gi * C::JSTRIDE;
+        if (mine) {
+#pragma unroll
+          for (int e = 0; e < EPL; ++e)
+            if (valid[e]) sh[e * G + g] = need_jac == 1 ? D[0][e] : ypred[e];
+        }
+        wave_sync();
+        if (mine) group_qss_jacobian<T, G>(sh, Jq, eform);
+        wave_sync();
+        if (mine) {
+          LU_T* const out = rows + gi * GSTRIDE;
+#pragma unroll 2
+          for (int t = g; t < n * n; t += G) {
+            const int j = t / n, i = t - j * n;
+            out[((i / G) * n + j) * G + i % G] = (LU_T)C::jac_elem(pk, Jq, i, j);
+          }
+          need_jac = 0;
+          njac++;
+        }
+        __threadfence_block();
+        wave_sync();
+        jreq = 0;
+      }
+    }
+    while (__builtin_expect(T::NQ == 0 && jreq != 0, 0)) {
       const int lead = __ffsll((long long)jreq) - 1, s = lead / G;
       jreq &= jreq - 1;
       wave_sync();

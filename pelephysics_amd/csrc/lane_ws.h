@@ -71,8 +71,6 @@ constexpr long long integrator_ws_rows(int mode) {
   switch (mode) {
     case MODE_BDF: return nn + 2 * (n + 1) * n;                   // A, Krylov basis V, Hessenberg H
     case MODE_ADAPTIVE: return 2 * nn;                            // J, LU (FP64)
-    case MODE_BATCHED_MIXED: return 2 * ws_rows<float>(nn) + nn;  // LU (FP32), Jf, Jd
-    case MODE_BATCHED_FP64: return nn + ws_rows<float>(nn) + nn;  // LU (FP64), Jf, Jd
     default: return 0;
   }
 }
@@ -91,10 +89,13 @@ struct has_qss : std::false_type {};
 template <class M>
 struct has_qss<M, std::void_t<decltype(M::NQ)>> : std::integral_constant<bool, (M::NQ > 0)> {};
 
-// (QSS mechanisms run one lane per cell.)
+// QSS mechanisms: at most one equation in four is in a second slot (NEQ <=
+// 4 G / 3).  A group keeps its forward and reverse rates apart, twice the LDS,
+// so a narrow group's waves do not share a SIMD (LuEthylene_qss, 65536 cells:
+// 16 lanes 81 ms, 32 lanes 60 ms; 4096 cells 9.1 and 7.0 ms).
 template <class M, int G>
 constexpr bool group_ok() {
-  return has_table<M>::value && !has_qss<M>::value && M::NEQ <= 3 * G && G <= 2 * M::NEQ;
+  return has_table<M>::value && M::NEQ <= 3 * G && G <= 2 * M::NEQ && (!has_qss<M>::value || 3 * M::NEQ <= 4 * G);
 }
 
 // The fixed-step BDF's group kernel (16 lanes per cell) holds the Krylov bases
@@ -102,26 +103,31 @@ constexpr bool group_ok() {
 // kernel runs (fixed_cells_per_wave in capi.hip).
 template <class M>
 constexpr bool group_fixed_ok() {
-  return group_ok<M, 16>() && M::NEQ <= 24 && M::NEQ > 16;
+  return group_ok<M, 16>() && !has_qss<M>::value && M::NEQ <= 24 && M::NEQ > 16;
 }
 
 // Device workspace of one wave of the group kernel (doubles, at most): an n x n
-// FP64 Jacobian accumulator and the Jacobian rows of its 64 / G groups.
-template <int n, int G>
+// FP64 Jacobian accumulator (QSS mechanisms: one per group, with the terms of
+// the QSS balances) and the Jacobian rows of its 64 / G groups.
+template <class M, int G>
 constexpr long long group_wave_doubles() {
-  return (long long)n * n + 1 + (64 / G) * ((long long)((n + G - 1) / G) * n * G + 1);
+  constexpr long long n = M::NEQ, acc = n * n + 1, groups = 64 / G;
+  constexpr long long rows = groups * ((n + G - 1) / G * n * G + 1);
+  if constexpr (has_qss<M>::value)
+    return groups * (acc + M::NQ * (n - 1) + 2 * M::NR + 1) + rows;
+  else
+    return acc + rows;
 }
 
 // Workspace rows per lane (doubles, 64-lane blocks as lane_ws) of the group
 // kernel with cells_per_wave cells per wave; 0 when there is no such kernel.
 template <class M>
 long long group_ws_rows(int cells_per_wave) {
-  constexpr int n = M::NEQ;
   switch (cells_per_wave) {
-    case 8: return group_ok<M, 8>() ? (group_wave_doubles<n, 8>() + 63) / 64 : 0;
-    case 4: return group_ok<M, 16>() ? (group_wave_doubles<n, 16>() + 63) / 64 : 0;
-    case 2: return group_ok<M, 32>() ? (group_wave_doubles<n, 32>() + 63) / 64 : 0;
-    case 1: return group_ok<M, 64>() ? (group_wave_doubles<n, 64>() + 63) / 64 : 0;
+    case 8: return group_ok<M, 8>() ? (group_wave_doubles<M, 8>() + 63) / 64 : 0;
+    case 4: return group_ok<M, 16>() ? (group_wave_doubles<M, 16>() + 63) / 64 : 0;
+    case 2: return group_ok<M, 32>() ? (group_wave_doubles<M, 32>() + 63) / 64 : 0;
+    case 1: return group_ok<M, 64>() ? (group_wave_doubles<M, 64>() + 63) / 64 : 0;
     default: return 0;
   }
 }

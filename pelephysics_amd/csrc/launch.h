@@ -40,6 +40,7 @@ struct MechLauncher {
   // 1 / 2 aJacobian with consP = 0 / 1, 3 net rates of progress (SI units, as
   // the reference's)
   hipError_t (*mech_eval)(int what, const double* sc, const double* T, int ncells, double* out, hipStream_t s);
+  bool qss;  // quasi-steady-state species eliminated
 };
 
 template <class M>
@@ -112,7 +113,8 @@ hipError_t launch_box(int mode, const ReactParamsDev& P, const BoxArgs& b, doubl
                                    &launch_group_fixed<TYPE>,                                  \
                                    &launch_adjoint<TYPE>, &integrator_ws_rows<TYPE>,           \
                                    &group_ws_rows<TYPE>,                                       \
-                                   &launch_flatten<TYPE>, &launch_mech_eval<TYPE>};            \
+                                   &launch_flatten<TYPE>, &launch_mech_eval<TYPE>,             \
+                                   has_qss<TYPE>::value};                                      \
     return &L;                                                                                 \
   }                                                                                            \
   }

@@ -3,7 +3,6 @@
 #pragma once
 #include <type_traits>
 #include "launch.h"
-#include "batched.h"
 #include "wave_bdf.h"
 #include "wave_adjoint.h"
 #include "group_bdf.h"
@@ -82,28 +81,13 @@ int resident_blocks(K kernel, long long lanes, int block = 64) {
   return (int)(blocks < need ? blocks : need);
 }
 
-// Persistent grid of a batched launch: every resident block, at most
-// q.max_blocks when set and at most the lanes the workspace holds (-1: no
-// device, -2: workspace missing).
-template <class M, int MODE, class K>
-int batched_grid(K kernel, const ReactParamsDev& P, const QueueArgs& q) {
-  int grid = resident_blocks(kernel, q.ncells);
-  if (grid < 0) return -1;
-  if (q.max_blocks > 0 && q.max_blocks < grid) grid = q.max_blocks;
-  if (integrator_ws_rows<M>(MODE) > 0) {
-    if (!P.ws || P.ws_lanes < 64 || P.ws_lanes % 64 != 0) return -2;
-    if (P.ws_lanes / 64 < grid) grid = (int)(P.ws_lanes / 64);
-  }
-  return grid;
-}
-
 // The group kernel (group_bdf.h) with G lanes per cell: a persistent grid of
 // every resident block of GROUP_WAVES waves, at most q.max_blocks waves and the
 // waves the workspace holds (group_ws_rows rows of 64 lanes per wave).
 template <class T, typename LU_T, int G, bool CV>
 hipError_t launch_group(const ReactParamsDev& P, double* y, const double* ysrc, double* rX, const double* rXsrc,
                         double dt, QueueArgs q, CellStats st, hipStream_t s) {
-  static_assert(group_ws_doubles<T::NEQ, G, LU_T>() <= group_wave_doubles<T::NEQ, G>(), "workspace layout");
+  static_assert(group_ws_doubles<T, G, LU_T>() <= group_wave_doubles<TabMech<T>, G>(), "workspace layout");
   // registers of the inverse's rows: above ~100 VGPRs hold the build to one wave per SIMD
   constexpr int lu_vgprs = (int)(((T::NEQ + G - 1) / G) * T::NEQ * sizeof(LU_T) / 4);
   auto k = group_bdf_kernel<T, LU_T, G, (lu_vgprs > 100 ? 1 : 2), CV>;
@@ -149,21 +133,10 @@ hipError_t batched_1d_mode(const ReactParamsDev& P, double* y, const double* ysr
                            double dt, QueueArgs q, CellStats st, hipStream_t s) {
   using LU_T = typename std::conditional<MODE == MODE_BATCHED_MIXED, float, double>::type;
   constexpr bool CV = MODE == MODE_GROUP_CVODE;
-  if constexpr (!has_qss<M>::value) {
-    // a group of lanes per cell at every size (group_bdf.h): one cell per lane
-    // measured 3.2 times as long on 64^3 drm19 cells and 16 to 115 times on
-    // calls that do not fill the chip (figures there)
-    return batched_group<M, LU_T, CV>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
-  } else if constexpr (CV) {
-    return hipErrorInvalidValue;
-  } else {
-    auto k = P.adapt.lane_occ == 1 ? batched_kernel<M, LU_T, IO1D, 1> : batched_kernel<M, LU_T, IO1D, 2>;
-    const int grid = batched_grid<M, MODE>(k, P, q);
-    if (grid < 0) return grid == -2 ? hipErrorInvalidValue : hipErrorInvalidDevice;
-    IO1D io{y, ysrc, rX, rXsrc};
-    hipLaunchKernelGGL(k, dim3(grid), dim3(64), 0, s, P, io, dt, q, st);
-    return hipGetLastError();
-  }
+  // a group of lanes per cell at every size (group_bdf.h): one cell per lane
+  // measured 3.2 times as long on 64^3 drm19 cells and 16 to 115 times on
+  // calls that do not fill the chip (figures there)
+  return batched_group<M, LU_T, CV>(P, y, ysrc, rX, rXsrc, dt, q, st, s);
 }
 
 template <class T, int G, bool BOX>
@@ -191,7 +164,7 @@ hipError_t launch_group_fixed(int mode, const ReactParamsDev& P, double* y, cons
                               const double* rXsrc, const BoxArgs* b, double dt, int ncells, int cells_per_wave,
                               CellStats st, hipStream_t s) {
   using Tab = typename wave_tables<M>::type;
-  if constexpr (!std::is_void<Tab>::value && !has_qss<M>::value) {
+  if constexpr (!std::is_void<Tab>::value) {
     GroupIO io{};
     io.f = IO1D{y, ysrc, rX, rXsrc};
     if (b) io.b = *b;

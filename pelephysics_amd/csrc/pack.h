@@ -4,6 +4,11 @@
 #include "ppc_common.h"
 
 namespace ppc {
+
+// regularisation of the QSS balances (comp_sc_qss epsilon of the reference's
+// generated QSS mechanisms)
+constexpr double QSS_EPS = 1e-12;
+
 namespace tab {
 
 // NASA7 coefficients below and above tmid, and the inverse molecular weight

@@ -34,7 +34,10 @@ unused place is reaction NR with coefficient 0; ``spCh``: first chunk of each
 species), so that the lanes of a group share the long rows.  Its reaction
 order is the table order with the reversible elementary reactions first
 (``perm``: position in the tables above), so that a wave's lanes agree on
-whether there is a reverse rate.
+whether there is a reverse rate.  QSS mechanisms add the balances' terms in the
+same chunks (``qch``, reaction + NR for a reverse rate), by matrix entry, then by
+right-hand side (``qRow``: first chunk of each; ``qInit``: the entries' constant
+parts), and the elimination as code (``qss_eliminate``).
 
 QSS mechanisms (``NQ`` > 0) index their quasi-steady-state species NS..NS+NQ-1
 in ``rxR``/``rxP`` and the thermo tables; ``rxNet`` and ``spPtr`` keep the
@@ -155,6 +158,22 @@ def qss_elimination(m: Mechanism):
 CHUNK = 8
 
 
+def qss_program(w, lu, fs, bs) -> None:
+    """The elimination and the solution of the QSS balances as straight-line
+    code: every lane of a group runs it on registers."""
+    w("  // QSS balances A x = r, factors and solution in place (no pivoting)")
+    w("  PPC_DI static void qss_eliminate(double* A, double* r) {")
+    for a, b, c in lu:
+        w(f"    A[{a}] /= A[{b}];" if c < 0 else f"    A[{a}] -= A[{b}] * A[{c}];")
+    for i, sl, p in fs:
+        w(f"    r[{i}] -= A[{sl}] * r[{p}];")
+    for row, d, ents in bs:
+        for sl, c in ents:
+            w(f"    r[{row}] -= A[{sl}] * r[{c}];")
+        w(f"    r[{row}] /= A[{d}];")
+    w("  }")
+
+
 def emit_pack(w, m: Mechanism, R: List[Reaction], n_el: int) -> None:
     """The Packed struct and its values (see the module's docstring); R is in
     table order, its first n_el reactions elementary."""
@@ -207,11 +226,36 @@ def emit_pack(w, m: Mechanism, R: List[Reaction], n_el: int) -> None:
             c = terms[i:i + CHUNK] + [(nr, 0)] * (CHUNK - len(terms[i:i + CHUNK]))
             chunks.append("{" + ", ".join(str(((v + 8) << 12) | j) for j, v in c) + "}")
         first.append(len(chunks))
+    qch, qfirst, qinit = [], [], []
+    if m.n_qss:
+        if any(k >= ns for r in R for k in r.efficiencies):
+            raise ValueError("a QSS species as a third body is not supported")
+        terms, slot, init, _, _, _ = qss_elimination(m)
+        order = ordered(m)
+        yaml_pos = {order[j]: i for j, i in pos.items()}
+        qrows = [[] for _ in range(len(slot) + m.n_qss)]
+        for q, c, j, d, cf in terms:
+            row = len(slot) + q if c < 0 else slot[(q, c)]
+            mul = cf if c < 0 or c == q else -cf
+            if mul != int(mul) or not -8 <= mul <= 7:
+                raise ValueError("QSS balance coefficient out of range")
+            qrows[row].append((yaml_pos[j] + (nr if d else 0), int(mul)))
+        if 2 * nr > 4095:
+            raise ValueError("mechanism too large for the packed QSS balances")
+        qfirst = [0]
+        for t in qrows:
+            for i in range(0, len(t), CHUNK):
+                c = t[i:i + CHUNK] + [(2 * nr, 0)] * (CHUNK - len(t[i:i + CHUNK]))
+                qch.append("{" + ", ".join(str(((v + 8) << 12) | j) for j, v in c) + "}")
+            qfirst.append(len(qch))
+        qinit = [_f(v) for v in init] + ["QSS_EPS"] * m.n_qss
     rows = [("PackSp", "sp", sp), ("PackRx", "rx", rx), ("PackFo", "fo", fo or ["{}"]),
             ("PackCh", "ch", chunks), ("double", "mw", [_f(s.mw) for s in m.species]),
             ("double", "effV", effv or ["0.0"]), ("PackEff", "eff", rx_eff or ["{0, 0}"]),
             ("unsigned short", "spCh", list(map(str, first))), ("unsigned short", "perm", list(map(str, perm))),
             ("unsigned char", "effK", effk or ["0"])]
+    if m.n_qss:
+        rows += [("PackCh", "qch", qch), ("double", "qInit", qinit), ("unsigned short", "qRow", list(map(str, qfirst)))]
     w("struct alignas(16) Packed {")
     for t, nm, v in rows:
         w(f"  {t} {nm}[{len(v)}];")
@@ -390,6 +434,7 @@ def emit(m: Mechanism, source: str) -> str:
                "rxIndex", "spPtr", "spRx"):
         w(f"  PPC_DI static int {nm}_(int i) {{ return {m.name}_t::kTab.{nm}[i]; }}")
     if nq:
+        qss_program(w, lu, fs, bs)
         for nm in ("tMul", "slotInit"):
             w(f"  PPC_DI static double {nm}_(int i) {{ return {m.name}_t::kTab.{nm}[i]; }}")
         for nm in ("rxFwdOff", "qRx", "qTermPtr", "tSlot", "tDir", "tRow", "tCol", "luA", "luB", "luC", "fsI",
