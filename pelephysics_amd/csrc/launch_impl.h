@@ -240,27 +240,47 @@ hipError_t launch_flatten(const FlatArgs& a, int unflatten, hipStream_t s) {
 // one cell per lane: sc[c*NS + k] (mol/m^3), T[c] (K); out[c*NS + k] = wdot_k
 // (mol/m^3/s), out[c*n*n + ...] = the column-major Jacobian of cell c, or
 // out[c*NR + j] = q_j (mol/m^3/s), written in place in the output array.
-template <class M>
-__global__ void __launch_bounds__(64) mech_eval_kernel(int what, const double* __restrict__ sc,
-                                                       const double* __restrict__ T, int ncells, double* out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncells) return;
-  double s[M::NS];
-  for (int k = 0; k < M::NS; ++k) s[k] = sc[(long long)c * M::NS + k];
-  const double Tv = T[c];
-  if (what == 0) {
-    double w[M::NS];
-    M::production_rate(w, s, Tv);
-    for (int k = 0; k < M::NS; ++k) out[(long long)c * M::NS + k] = w[k];
-  } else if (what == 3) {
-    double* q = out + (long long)c * M::NR;  // written in place: NR can be large
-    M::progress_rates(q, s, Tv);
+//
+// One kernel per function: with the four in one, all took the Jacobian's 512
+// registers, one wave per SIMD (drm19 rates: 203, two).  The rates' flat arrays
+// pass through LDS in whole lines (a row is 65 cells: no bank conflicts either
+// way) where a wave's cells take little of it.  Bound by the FP64 vector issue:
+// drm19 is 7800 vector instructions per wave, 57 us at the full rate for 262144
+// cells; a call of them 99.1 -> 86.6 us.
+template <class M, int WHAT>
+__global__ void __launch_bounds__(64) mech_eval_kernel(const double* __restrict__ sc, const double* __restrict__ T,
+                                                       int ncells, double* out) {
+  constexpr int NS = M::NS;
+  const int l = threadIdx.x, c0 = blockIdx.x * 64, nc = min(64, ncells - c0);
+  double s[NS];
+  if constexpr (WHAT == 0 && NS <= 32) {
+    __shared__ double row[NS * 65];
+    const double* const from = sc + (long long)c0 * NS;
+    for (int i = l; i < nc * NS; i += 64) row[i % NS * 65 + i / NS] = from[i];
+    __syncthreads();
+    const int m = min(l, nc - 1);  // lanes past the end repeat the last cell
+    double w[NS];
+    for (int k = 0; k < NS; ++k) s[k] = row[k * 65 + m];
+    M::production_rate(w, s, T[c0 + m]);
+    __syncthreads();
+    for (int k = 0; k < NS; ++k) row[k * 65 + l] = w[k];
+    __syncthreads();
+    double* const to = out + (long long)c0 * NS;
+    for (int i = l; i < nc * NS; i += 64) to[i] = row[i % NS * 65 + i / NS];
   } else {
-    double* J = out + (long long)c * M::NEQ * M::NEQ;
-    if (what == 1)
-      M::template jacobian<0>(J, s, Tv);
-    else
-      M::template jacobian<1>(J, s, Tv);
+    if (l >= nc) return;
+    const long long c = c0 + l;
+    for (int k = 0; k < NS; ++k) s[k] = sc[c * NS + k];
+    const double Tv = T[c];
+    if constexpr (WHAT == 0) {
+      double w[NS];
+      M::production_rate(w, s, Tv);
+      for (int k = 0; k < NS; ++k) out[c * NS + k] = w[k];
+    } else if constexpr (WHAT == 3) {
+      M::progress_rates(out + c * M::NR, s, Tv);  // written in place: NR can be large
+    } else {
+      M::template jacobian<WHAT - 1>(out + c * M::NEQ * M::NEQ, s, Tv);
+    }
   }
 }
 
@@ -268,7 +288,11 @@ template <class M>
 hipError_t launch_mech_eval(int what, const double* sc, const double* T, int ncells, double* out, hipStream_t s) {
   if (what < 0 || what > 3) return hipErrorInvalidValue;
   if (ncells <= 0) return hipSuccess;
-  hipLaunchKernelGGL(mech_eval_kernel<M>, dim3((ncells + 63) / 64), dim3(64), 0, s, what, sc, T, ncells, out);
+  auto k = what == 0   ? mech_eval_kernel<M, 0>
+           : what == 1 ? mech_eval_kernel<M, 1>
+           : what == 2 ? mech_eval_kernel<M, 2>
+                       : mech_eval_kernel<M, 3>;
+  hipLaunchKernelGGL(k, dim3((ncells + 63) / 64), dim3(64), 0, s, sc, T, ncells, out);
   return hipGetLastError();
 }
 

@@ -97,3 +97,22 @@ def test_rk64_on_both_sides_of_the_lane_kernel(models):
         out.append((y[:st.ncells], R.cell_steps(n)[:st.ncells]))
     assert (out[0][1] == out[1][1]).all()
     _compare_y(m.n_species + 1, out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("mech", ["drm19", "LiDryer", "dodecane_lu"])
+def test_production_rate_counts(models, oracles, mech):
+    """64 cells per block: the last block's remainder.  The tolerance is the mechanism tests'."""
+    import torch
+    from pelephysics_amd.reactor import ReactorBase
+    m, st, _, _ = _cells(models, mech, 130)
+    y = st.y_1d().reshape(st.ncells, -1)
+    sc = torch.from_numpy(y[:, :-1] * np.array([s.imw for s in m.species]) * 1e6).cuda().contiguous()
+    T = torch.from_numpy(y[:, -1].copy()).cuda()
+    R = ReactorBase.create("ReactorBDF")
+    R.init(2, 1, mechanism=mech)
+    w = R.production_rate(sc, T)
+    for c in (0, 63, 64, 129):
+        wo = oracles[mech].wdot(sc[c].cpu().numpy(), float(T[c]))
+        assert np.abs(w[c].cpu().numpy() - wo).max() <= 1e-10 * np.abs(wo).max(), c
+    for n in (1, 63, 64, 65, 129):
+        assert torch.equal(R.production_rate(sc[:n].contiguous(), T[:n].contiguous()), w[:n]), n
