@@ -10,22 +10,17 @@ keeps the fastest:
 * kernels: the compiled implementations of the mechanism, the generated
   straight-line code ("<mech>") and the constant-memory tables
   ("<mech>_table"), where both exist;
-* batched_waves_per_simd / batched_waves_per_cu (batched forms only): the
-  kernel build held to 2 waves per SIMD (8, 6 or 4 persistent waves per
-  compute unit) or to 1 (4 or 3 per CU).  Fewer waves contend less for the
-  caches that back private memory but hide less latency; the 1-wave build
-  spills less;
-* batched_lu_batch / batched_lu_wait (batched forms only): how many waiting
-  lanes, or how many trips of waiting, make a wave factor its lanes' Newton
-  matrices together (16 lanes or 4 trips; 64 lanes or 8 trips; 64 lanes or
-  32 trips, i.e. nearly always the whole wave at once);
-* batched_box_direct (batched forms, box calls): the box kernel itself (1) or
-  box -> flat state, the 1-D kernel, flat -> box (0);
-* batched_cells_per_wave (batched forms, table-driven kernels): one cell per
-  lane (0) or a group of 8, 16, 32 or 64 lanes per cell (8, 4, 2, 1 cells per
-  wave; the sizes a mechanism's kernels are built for), with 8 or 4 waves
-  per CU and the LU service serving each group at once (1 cell, 1 trip) or
-  all of a wave's waiting groups together (64, 8 or 32 trips).
+* batched_cells_per_wave (batched forms, table-driven kernels): the library's
+  choice by mechanism and number of cells (0), or a group of 8, 16, 32 or 64
+  lanes per cell (8, 4, 2, 1 cells per wave; the sizes a mechanism's kernels
+  are built for);
+* batched_waves_per_cu (8, 6, 4 or 3 persistent waves per compute unit) and
+  batched_lu_batch / batched_lu_wait (how many waiting cells, or how many trips
+  of waiting, make a wave factor its cells' Newton matrices together): read
+  where batched_cells_per_wave names a size, as is the launch shape;
+* batched_waves_per_simd and batched_box_direct (batched forms): accepted, the
+  kernels have one build and one box route; candidates that differ in them
+  only, or in what is not read, time the same launch.
 
 Each candidate runs `calls` calls on the same cells and arrays; its time is
 the kernel time of the last one (the queue in the cost order of the call
