@@ -54,8 +54,10 @@ const MechLauncher* resolve_mech(const char* name, int manifold_dim) {
 // block hands the result to the host and leaves acc zero for the next call, so
 // a call needs one launch, no clearing and no copy (one drm19 box of 3360
 // cells: 360 us a call against 389 with a clearing launch, a copy and a
-// second wait).
+// second wait).  acc is the handle's own: what an interrupted sum leaves there
+// would keep every later call from finding its last block (finish).
 constexpr int NSTAT = 9;
+constexpr unsigned long long NOT_DELIVERED = ~0ULL;  // no sum, and no step count, is this large
 __global__ void __launch_bounds__(256) reduce_stats(const int* __restrict__ nsteps, const int* __restrict__ nrhs,
                                                     const int* __restrict__ njac, const int* __restrict__ nlu,
                                                     const int* __restrict__ nnewton,
@@ -295,22 +297,30 @@ ppc::CellStats counters(pp_chem* h) {
   return st;
 }
 
-// Reduces the counters st of the call's kernels on stream s (accumulators red),
-// waits for the stream, takes the kernels' time from the events around them and
-// returns int(average steps) or an error.
-int finish_with(pp_chem* h, int ncells, hipStream_t s, const ppc::CellStats& st, unsigned long long* red);
+// Clears reduce_stats' accumulators, and waits: the calls run on streams that
+// the null stream does not order.
+hipError_t clear_stats(pp_chem* h) {
+  const hipError_t e = hipMemset(h->d_red, 0, sizeof(unsigned long long) * (NSTAT + 1));
+  return e == hipSuccess ? hipStreamSynchronize(nullptr) : e;
+}
 
-int finish(pp_chem* h, int ncells, hipStream_t s) { return finish_with(h, ncells, s, counters(h), h->d_red); }
-
-int finish_with(pp_chem* h, int ncells, hipStream_t s, const ppc::CellStats& st, unsigned long long* red) {
+// Reduces the counters st of the call's kernels on stream s, waits for the
+// stream, takes the kernels' time from the events around them and returns
+// int(average steps) or an error.
+int finish(pp_chem* h, int ncells, hipStream_t s, const ppc::CellStats& st) {
+  h->h_red[NSTAT - 1] = NOT_DELIVERED;
   const int blocks = ncells > 0 ? (ncells + 255) / 256 < 1024 ? (ncells + 255) / 256 : 1024 : 1;
   hipLaunchKernelGGL(reduce_stats, dim3(blocks), dim3(256), 0, s, st.nsteps, st.nrhs, st.njac, st.nlu,
-                     st.nnewton, st.nreject, ncells, red, h->h_red);
+                     st.nnewton, st.nreject, ncells, h->d_red, h->h_red);
   HIPCHK(h, hipGetLastError());
   HIPCHK(h, hipStreamSynchronize(s));
   float kernel_ms = 0.f;
   HIPCHK(h, hipEventElapsedTime(&kernel_ms, h->ev0, h->ev1));
   const unsigned long long* r = h->h_red;
+  if (r[NSTAT - 1] == NOT_DELIVERED) {
+    HIPCHK(h, clear_stats(h));
+    return fail(h, PP_CHEM_EHIP, "the call's statistics were not delivered");
+  }
   pp_chem_stats& S = h->stats;
   S.ncells = ncells;
   S.nsteps = (long long)r[0];
@@ -343,10 +353,9 @@ int kmode(int mode) {
 }
 
 // ---- device scratch of pp_chem_react_1d_noalloc: one array per GPU, held
-// until the process ends.  Layout: [0, 256) queue counter, [256, 512) the
-// statistics reduction, then the per-cell step counts (up to kScratchCells
-// bytes from the start), then the integrator workspace, which finds at least
-// kScratchWs bytes whatever the number of cells.
+// until the process ends.  Layout: [0, 512) queue counter, then the per-cell
+// step counts (up to kScratchCells bytes from the start), then the integrator
+// workspace, which finds at least kScratchWs bytes whatever the number of cells.
 constexpr size_t kScratchCells = 64ull << 20, kScratchWs = 64ull << 20;
 constexpr size_t kScratchBytes = kScratchCells + kScratchWs;
 constexpr size_t kScratchCounts = 512;
@@ -772,7 +781,7 @@ int pp_chem_create(const pp_chem_config* cfg, pp_chem** out) {
   // one allocation: the accumulators, the queue and the failure count
   constexpr size_t red_bytes = sizeof(unsigned long long) * (NSTAT + 1), queue_ints = 1 + 2 * NBINS;
   if (e == hipSuccess) e = hipMalloc(&h->d_red, red_bytes + sizeof(int) * (queue_ints + 1));
-  if (e == hipSuccess) e = hipMemset(h->d_red, 0, red_bytes);
+  if (e == hipSuccess) e = clear_stats(h);
   if (e == hipSuccess) {
     h->d_queue = reinterpret_cast<int*>(h->d_red + NSTAT + 1);
     h->d_fail = h->d_queue + queue_ints;
@@ -1043,7 +1052,7 @@ int pp_chem_react_box(pp_chem* h, const int lo[3], const int hi[3], const pp_arr
     if (e != hipSuccess) return hip_fail(h, e, "react_box launch");
   }
   HIPCHK(h, hipEventRecord(h->ev1, s));
-  const int r = finish(h, ncells, s);
+  const int r = finish(h, ncells, s, counters(h));
   if (h->cfg.mod_reactor) *time += *dt_react;
   return r;
 }
@@ -1087,7 +1096,7 @@ int pp_chem_react_1d(pp_chem* h, double* y, double* ysrc, double* rX, double* rX
     HIPCHK(h, hipMemcpyAsync(y, dy, ny * sizeof(double), hipMemcpyDeviceToHost, s));
     HIPCHK(h, hipMemcpyAsync(rX, dx, nx * sizeof(double), hipMemcpyDeviceToHost, s));
   }
-  const int r = finish(h, ncells, s);
+  const int r = finish(h, ncells, s, counters(h));
   if (h->cfg.mod_reactor) *time += *dt_react;
   return r;
 }
@@ -1105,7 +1114,6 @@ int pp_chem_react_1d_noalloc(pp_chem* h, double* y, double* ysrc, double* rX, do
                 "ncells = " + std::to_string(ncells) + " exceeds the device scratch of pp_chem_react_1d_noalloc (" +
                     std::to_string((kScratchCells - kScratchCounts) / sizeof(int)) + " cells at most)");
   int* counter = reinterpret_cast<int*>(h->scratch);
-  unsigned long long* red = reinterpret_cast<unsigned long long*>(h->scratch + 256);
   int* nsteps = reinterpret_cast<int*>(h->scratch + kScratchCounts);
   unsigned char* ws = h->scratch + kScratchCounts + counts;
   const size_t ws_bytes = kScratchBytes - kScratchCounts - counts;
@@ -1142,7 +1150,7 @@ int pp_chem_react_1d_noalloc(pp_chem* h, double* y, double* ysrc, double* rX, do
     if (e != hipSuccess) return hip_fail(h, e, "react_1d_noalloc launch");
   }
   HIPCHK(h, hipEventRecord(h->ev1, s));
-  const int r = finish_with(h, ncells, s, st, red);
+  const int r = finish(h, ncells, s, st);
   if (h->cfg.mod_reactor) *time += *dt_react;
   return r;
 }
@@ -1251,7 +1259,7 @@ int pp_chem_react_1d_chained(pp_chem* h, double* y, double* ysrc, double* rX, do
   HIPCHK(h, hipEventSynchronize(h->ev1));
   int nfail = 0;
   HIPCHK(h, hipMemcpy(&nfail, h->d_fail, sizeof(int), hipMemcpyDeviceToHost));
-  const int r = finish(h, ncells, s);
+  const int r = finish(h, ncells, s, counters(h));
   if (h->cfg.mod_reactor) *time += ncalls * dt;
   if (r >= 0 && nfail > 0)
     return fail(h, PP_CHEM_EINTEGRATE,

@@ -1,0 +1,225 @@
+// The C-ABI's host logic (pelephysics_amd/csrc/capi.hip) without a GPU: the HIP
+// runtime and the mechanism launchers are restated here as recorders, so that
+// what a call allocates, clears, launches and returns can be looked at.
+//
+//   capi_host SCENARIO   prints "key value" lines
+//
+// Device memory is host memory from a pool in which a freed block is the next
+// one handed out (oldest first), as a device allocator may do.  Kernels do not
+// run; reduce_stats hands over a preset result unless `deliver` is off.
+#include "../../pelephysics_amd/csrc/capi.hip"
+
+#include <deque>
+#include <map>
+
+namespace fake {
+constexpr size_t BLOCK = 1 << 20;
+std::deque<char*> freed;
+int malloc_fails_in = -1;  // allocations until one fails (-1: none)
+int captures = 0, replays = 0;
+bool deliver = true;
+unsigned long long result[NSTAT] = {};
+const void *acc = nullptr;           // reduce_stats' accumulators of the last call
+bool memset_pending = false;         // a hipMemset nothing has waited for
+char symbol[1024];                   // the device scratch's address (never dereferenced)
+// last integrator launch
+std::string launched;
+int mode = -1, ncells = -1;
+ppc::CellStats st{};
+ppc::ReactParamsDev P{};
+
+hipError_t react_1d(int m, const ppc::ReactParamsDev& p, double*, const double*, double*, const double*, double,
+                    int n, ppc::CellStats s, int, hipStream_t) {
+  launched = "lane_1d", mode = m, ncells = n, st = s, P = p;
+  return hipSuccess;
+}
+hipError_t react_box(int m, const ppc::ReactParamsDev& p, const ppc::BoxArgs&, double, int n, ppc::CellStats s, int,
+                     hipStream_t) {
+  launched = "lane_box", mode = m, ncells = n, st = s, P = p;
+  return hipSuccess;
+}
+hipError_t batched_1d(int m, const ppc::ReactParamsDev& p, double*, const double*, double*, const double*, double,
+                      ppc::QueueArgs q, ppc::CellStats s, hipStream_t) {
+  launched = "group_1d", mode = m, ncells = q.ncells, st = s, P = p;
+  return hipSuccess;
+}
+hipError_t group_fixed(int, const ppc::ReactParamsDev&, double*, const double*, double*, const double*,
+                       const ppc::BoxArgs*, double, int, int, ppc::CellStats, hipStream_t) {
+  return hipErrorNotSupported;
+}
+hipError_t adjoint(const ppc::ReactParamsDev&, const ppc::AdjointArgs&, hipStream_t) { return hipSuccess; }
+hipError_t flatten(const ppc::FlatArgs&, int, hipStream_t) { return hipSuccess; }
+hipError_t mech_eval(int, const double*, const double*, int, double*, hipStream_t) { return hipSuccess; }
+long long no_rows(int) { return 0; }
+long long lane_rows(int) { return 5000; }
+long long group_rows(int cpw) { return cpw == 4 ? 52 : (cpw == 2 ? 30 : 0); }
+
+// 20 species; a workspace of the one-lane kernels and group kernels as asked
+MechLauncher mech(const char* name, bool lane_ws, bool groups) {
+  MechLauncher L{};
+  L.name = name, L.ns = 20, L.nr = 30, L.batched_ok = 1;
+  L.react_1d = &react_1d, L.react_box = &react_box, L.batched_1d = &batched_1d, L.group_fixed = &group_fixed;
+  L.adjoint_1d = &adjoint, L.flatten = &flatten, L.mech_eval = &mech_eval;
+  L.ws_rows = lane_ws ? &lane_rows : &no_rows;
+  L.group_ws_rows = groups ? &group_rows : &no_rows;
+  return L;
+}
+}  // namespace fake
+
+// The mechanisms: "heptane_lu_88sk" with a workspace, "dodecane_lu" without
+// group kernels, the others with both unneeded or present.
+namespace ppc {
+#define PPC_MECH(M)                                                                                        \
+  const MechLauncher* launcher_##M() {                                                                     \
+    static const MechLauncher L = fake::mech(#M, !std::strcmp(#M, "heptane_lu_88sk"), std::strcmp(#M, "dodecane_lu") != 0); \
+    return &L;                                                                                             \
+  }
+#include "../../pelephysics_amd/csrc/inst/registry.inc"
+#undef PPC_MECH
+const MechLauncher* manifold_launcher(int) { return nullptr; }
+}  // namespace ppc
+
+// ---------------------------------------------------- the HIP runtime --
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) {
+  *p = nullptr;
+  if (fake::malloc_fails_in >= 0 && fake::malloc_fails_in-- == 0) return hipErrorOutOfMemory;
+  if (n > fake::BLOCK) return hipErrorOutOfMemory;
+  if (fake::freed.empty()) {
+    *p = std::calloc(1, fake::BLOCK);
+  } else {
+    *p = fake::freed.front();
+    fake::freed.pop_front();
+  }
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+  if (p) fake::freed.push_back((char*)p);
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return (*p = std::calloc(1, n)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
+hipError_t hipMemset(void* p, int v, size_t n) {
+  std::memset(p, v, n);
+  fake::memset_pending = true;
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { std::memcpy(d, s, n); return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) {
+  if (!s) fake::memset_pending = false;
+  return hipSuccess;
+}
+hipError_t hipDeviceSynchronize() { fake::memset_pending = false; return hipSuccess; }
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 2; return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "error"; }
+hipError_t hipGetSymbolAddress(void** p, const void*) { *p = fake::symbol; return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { *e = (hipEvent_t)fake::symbol; return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* t, hipEvent_t, hipEvent_t) { *t = 1.f; return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)fake::symbol; return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { ++fake::captures; return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { *g = (hipGraph_t)fake::symbol; return hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) { *e = (hipGraphExec_t)fake::symbol; return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { ++fake::replays; return hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+
+static dim3 cfg_grid, cfg_block;
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t, hipStream_t) { cfg_grid = g, cfg_block = b; return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* m, hipStream_t* s) {
+  *g = cfg_grid, *b = cfg_block, *m = 0, *s = nullptr;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t) {
+  if (f == (const void*)&reduce_stats) {
+    fake::acc = *(const void**)args[7];
+    unsigned long long* host = *(unsigned long long**)args[8];
+    if (fake::deliver)
+      for (int i = 0; i < NSTAT; ++i) host[i] = fake::result[i];
+  }
+  return hipSuccess;
+}
+void** __hipRegisterFatBinary(const void*) { return nullptr; }
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void**, const void*, char*, const char*, unsigned, uint3*, uint3*, dim3*, dim3*, int*) {}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+}
+
+// --------------------------------------------------------- scenarios --
+namespace {
+
+double buf[1 << 16];  // stands for every device array; kernels do not run
+
+pp_chem* handle(const char* name, int mode, long long workspace_bytes = 0) {
+  pp_chem_config c;
+  pp_chem* h = nullptr;
+  if (pp_chem_config_init(&c, name, mode, 2) != 0) std::abort();
+  c.workspace_bytes = workspace_bytes;
+  std::printf("create %d\n", pp_chem_create(&c, &h));
+  return h;
+}
+
+int call_1d(pp_chem* h, int n) {
+  double dt = 1e-5, t = 0;
+  return pp_chem_react_1d(h, buf, buf, buf, buf, &dt, &t, n, 1, nullptr);
+}
+int call_chained(pp_chem* h, int n, int calls) {
+  double dt = 1e-5, t = 0;
+  return pp_chem_react_1d_chained(h, buf, buf, buf, buf, &dt, &t, n, calls, nullptr);
+}
+int call_noalloc(pp_chem* h, int n) {
+  double dt = 1e-5, t = 0;
+  return pp_chem_react_1d_noalloc(h, buf, buf, buf, buf, &dt, &t, n, nullptr);
+}
+int call_box(pp_chem* h, int n) {
+  pp_array4 a{};
+  a.p = buf, a.jstride = n, a.kstride = n, a.nstride = n, a.ncomp = 20;
+  a.end[0] = n, a.end[1] = a.end[2] = 1;
+  const int lo[3] = {0, 0, 0}, hi[3] = {n - 1, 0, 0};
+  double dt = 1e-5, t = 0;
+  return pp_chem_react_box(h, lo, hi, &a, &a, &a, &a, &a, &a, nullptr, &dt, &t, nullptr);
+}
+
+// a call's statistics do not arrive: an error, and the next call is sound again
+void undelivered() {
+  pp_chem* h = handle("drm19", PP_CHEM_RK64);
+  std::printf("memset_pending_after_create %d\n", (int)fake::memset_pending);
+  fake::result[0] = 800;  // 8 steps a cell
+  std::printf("first %d\n", call_1d(h, 100));
+  fake::deliver = false;
+  h->d_red[0] = 5, h->d_red[NSTAT] = 3;  // what such a call leaves behind
+  std::printf("undelivered %d\n", call_1d(h, 100));
+  fake::deliver = true;
+  bool clear = true;
+  for (int i = 0; i <= NSTAT; ++i) clear = clear && h->d_red[i] == 0;
+  std::printf("accumulators_clear %d\n", (int)clear);
+  std::printf("next %d\n", call_1d(h, 100));
+}
+
+// two handles' calls without allocation share no accumulators
+void noalloc_shared() {
+  pp_chem *a = handle("drm19", PP_CHEM_RK64), *b = handle("drm19", PP_CHEM_RK64);
+  call_noalloc(a, 100);
+  const void* first = fake::acc;
+  call_noalloc(b, 100);
+  std::printf("shared %d\n", (int)(first == fake::acc));
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::string s = argc > 1 ? argv[1] : "";
+  if (s == "undelivered") undelivered();
+  else if (s == "noalloc_shared") noalloc_shared();
+  else return 2;
+  return 0;
+}

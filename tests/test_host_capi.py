@@ -1,0 +1,54 @@
+"""The C-ABI's host logic on recorders of the HIP runtime and of the mechanism
+launchers (tests/host/capi_host.cpp): what a call does when something it relies
+on is missing, without a GPU."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    if not os.path.exists(HIPCC) or shutil.which("g++") is None:
+        pytest.skip("no hipcc or g++")
+    d = tmp_path_factory.mktemp("host")
+    src = os.path.join(ROOT, "tests", "host", "capi_host.cpp")
+    # the host side only, linked against no HIP runtime
+    for cmd in ([HIPCC, "-x", "hip", "--cuda-host-only", "-O1", "-fPIE", "-std=c++17", "--offload-arch=gfx950", "-Xclang", "-target-feature",
+                 "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument", "-c", src, "-o", str(d / "h.o")],
+                ["g++", str(d / "h.o"), "-o", str(d / "capi_host"), "-lpthread"]):
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr[-3000:]
+
+    def run(scenario):
+        r = subprocess.run([str(d / "capi_host"), scenario], capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, (r.returncode, r.stdout, r.stderr[-2000:])
+        out = {}
+        for line in r.stdout.splitlines():
+            k, v = line.split(None, 1)
+            out[k] = int(v) if v.lstrip("-").isdigit() else v
+        return out
+
+    return run
+
+
+def test_undelivered_statistics_are_an_error(host):
+    """The kernel that sums up a call hands its result to host memory.  A call
+    whose result does not arrive must not return an earlier call's, and must
+    leave nothing behind that spoils the next."""
+    s = host("undelivered")
+    assert s["create"] == 0 and s["memset_pending_after_create"] == 0
+    assert s["first"] == 8
+    assert s["undelivered"] == -3  # EHIP
+    assert s["accumulators_clear"] == 1
+    assert s["next"] == 8
+
+
+def test_noalloc_calls_share_no_accumulators(host):
+    """Overlapping pp_chem_react_1d_noalloc calls of two handles race on the
+    device scratch and spoil those calls, not every later one."""
+    assert host("noalloc_shared")["shared"] == 0
