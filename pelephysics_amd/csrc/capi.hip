@@ -175,10 +175,11 @@ struct GraphKey {
   int ncells;
   double dt;
   const void *cnt, *order, *ws;
+  int cap;  // distance of the counters' arrays in cnt
   long long ws_lanes;
   bool operator==(const GraphKey& o) const {
     return std::memcmp(arrays, o.arrays, sizeof(arrays)) == 0 && ncells == o.ncells && dt == o.dt &&
-           cnt == o.cnt && order == o.order && ws == o.ws && ws_lanes == o.ws_lanes;
+           cnt == o.cnt && order == o.order && ws == o.ws && cap == o.cap && ws_lanes == o.ws_lanes;
   }
 };
 
@@ -1233,7 +1234,7 @@ int pp_chem_react_1d_chained(pp_chem* h, double* y, double* ysrc, double* rX, do
     done = 1;
   }
   if (ncells > 0 && done < ncalls) {
-    const GraphKey key{{y, ysrc, rX, rXsrc}, ncells, dt, h->d_cnt, h->d_order, h->P.ws, h->P.ws_lanes};
+    const GraphKey key{{y, ysrc, rX, rXsrc}, ncells, dt, h->d_cnt, h->d_order, h->P.ws, h->cap, h->P.ws_lanes};
     if (!h->gexec || !(key == h->gkey)) {
       drop_graph(h);
       HIPCHK(h, hipStreamBeginCapture(h->gstream, hipStreamCaptureModeThreadLocal));

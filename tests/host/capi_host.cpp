@@ -214,12 +214,30 @@ void noalloc_shared() {
   std::printf("shared %d\n", (int)(first == fake::acc));
 }
 
+// counters that grew between two chained calls, at the address they had: the
+// captured launches hold their old layout
+void graph_counters() {
+  pp_chem* h = handle("drm19", PP_CHEM_BDF_ADAPTIVE_MIXED);
+  call_chained(h, 100, 3);
+  const int* nrhs = fake::st.nrhs;
+  const void* cnt = h->d_cnt;
+  std::printf("captures %d\n", fake::captures);
+  call_1d(h, 200);
+  std::printf("same_address %d\n", (int)(cnt == h->d_cnt));
+  call_chained(h, 100, 3);
+  std::printf("same_layout %d\n", (int)(nrhs == fake::st.nrhs));
+  std::printf("captures_after_growth %d\n", fake::captures);
+  call_chained(h, 100, 3);
+  std::printf("captures_again %d\n", fake::captures);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "undelivered") undelivered();
   else if (s == "noalloc_shared") noalloc_shared();
+  else if (s == "graph_counters") graph_counters();
   else return 2;
   return 0;
 }

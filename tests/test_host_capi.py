@@ -52,3 +52,13 @@ def test_noalloc_calls_share_no_accumulators(host):
     """Overlapping pp_chem_react_1d_noalloc calls of two handles race on the
     device scratch and spoil those calls, not every later one."""
     assert host("noalloc_shared")["shared"] == 0
+
+
+def test_chained_graph_follows_the_counters_layout(host):
+    """The per-cell counters are one allocation whose arrays' distances depend
+    on its capacity: a graph captured before it grew is not replayed after, also
+    where the new allocation has the old address."""
+    s = host("graph_counters")
+    assert s["captures"] == 1 and s["same_address"] == 1 and s["same_layout"] == 0
+    assert s["captures_after_growth"] == 2
+    assert s["captures_again"] == 2  # and the new one is kept
