@@ -275,13 +275,20 @@ int hip_fail(pp_chem* h, hipError_t e, const char* where) {
 
 int ensure_counters(pp_chem* h, int ncells) {
   if (ncells <= h->cap) return 0;
-  if (h->d_cnt) HIPCHK(h, hipFree(h->d_cnt));
-  if (h->d_order) HIPCHK(h, hipFree(h->d_order));
+  int *cnt = h->d_cnt, *order = h->d_order;
+  h->cap = 0;  // until both are there again
   h->d_cnt = nullptr;
   h->d_order = nullptr;
   h->hist_valid = false;
+  if (cnt) HIPCHK(h, hipFree(cnt));
+  if (order) HIPCHK(h, hipFree(order));
   HIPCHK(h, hipMalloc(&h->d_cnt, sizeof(int) * 6 * (size_t)ncells));
-  HIPCHK(h, hipMalloc(&h->d_order, sizeof(int) * (size_t)ncells));
+  const hipError_t e = hipMalloc(&h->d_order, sizeof(int) * (size_t)ncells);
+  if (e != hipSuccess) {
+    (void)hipFree(h->d_cnt);
+    h->d_cnt = nullptr;
+    return hip_fail(h, e, "hipMalloc");
+  }
   h->cap = ncells;
   return 0;
 }
@@ -974,6 +981,7 @@ int pp_chem_adjoint_1d(pp_chem* h, double* y, const double* rX, int ncells, int 
   if (need > h->ckpt_cap) {
     if (h->d_ckpt) HIPCHK(h, hipFree(h->d_ckpt));
     h->d_ckpt = nullptr;
+    h->ckpt_cap = 0;
     HIPCHK(h, hipMalloc(&h->d_ckpt, need * sizeof(double)));
     h->ckpt_cap = need;
   }
@@ -1075,6 +1083,7 @@ int pp_chem_react_1d(pp_chem* h, double* y, double* ysrc, double* rX, double* rX
     if (need > h->stage_cap) {
       if (h->d_stage) HIPCHK(h, hipFree(h->d_stage));
       h->d_stage = nullptr;
+      h->stage_cap = 0;
       HIPCHK(h, hipMalloc(&h->d_stage, need * sizeof(double)));
       h->stage_cap = need;
     }

@@ -231,6 +231,30 @@ void graph_counters() {
   std::printf("captures_again %d\n", fake::captures);
 }
 
+// an allocation that fails while a buffer grows: the next call that fitted
+// before allocates again
+void failed_growth(int which) {
+  pp_chem* h = handle("drm19", which == 2 ? PP_CHEM_BDF : PP_CHEM_BDF_ADAPTIVE);
+  const auto call = [&](int n) {
+    double dt = 1e-5, t = 0, g[4] = {};
+    switch (which) {
+      case 1: return pp_chem_react_1d(h, buf, buf, buf, buf, &dt, &t, n, 0, nullptr);
+      case 2: return pp_chem_adjoint_1d(h, buf, buf, n, 1, dt, 0, 1, g, buf, nullptr);
+      default: return call_1d(h, n);
+    }
+  };
+  std::printf("before %d\n", call(10));
+  // counters: the first or the second of their two; staging and checkpoints: their one
+  if (which == 1) call_1d(h, 20);  // the counters have grown already
+  fake::malloc_fails_in = which == 3 ? 1 : 0;
+  std::printf("failed %d\n", call(20));
+  fake::malloc_fails_in = -1;
+  std::printf("after %d\n", call(10));
+  std::printf("counters %d\n", (int)(which == 2 || (h->d_cnt && h->d_order)));
+  std::printf("staging %d\n", (int)(which != 1 || h->d_stage));
+  std::printf("checkpoints %d\n", (int)(which != 2 || h->d_ckpt));
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -238,6 +262,7 @@ int main(int argc, char** argv) {
   if (s == "undelivered") undelivered();
   else if (s == "noalloc_shared") noalloc_shared();
   else if (s == "graph_counters") graph_counters();
+  else if (s.rfind("failed_growth", 0) == 0) failed_growth(s.back() - '0');
   else return 2;
   return 0;
 }

@@ -62,3 +62,14 @@ def test_chained_graph_follows_the_counters_layout(host):
     assert s["captures"] == 1 and s["same_address"] == 1 and s["same_layout"] == 0
     assert s["captures_after_growth"] == 2
     assert s["captures_again"] == 2  # and the new one is kept
+
+
+@pytest.mark.parametrize("which", [0, 1, 2, 3])
+def test_failed_growth_leaves_no_stale_capacity(host, which):
+    """A buffer is freed before its larger successor is allocated.  When that
+    fails (0, 3: the per-cell counters and the queue order; 1: the staging of
+    host arrays; 2: the adjoint's checkpoints), a call of the old size must not
+    take the missing buffer for a present one."""
+    s = host(f"failed_growth{which}")
+    assert s["before"] >= 0 and s["failed"] == -3 and s["after"] >= 0
+    assert s["counters"] and s["staging"] and s["checkpoints"]
