@@ -355,9 +355,11 @@ int finish(pp_chem* h, int ncells, hipStream_t s, const ppc::CellStats& st) {
 
 bool is_batched(int mode) { return mode == ppc::MODE_BATCHED_MIXED || mode == ppc::MODE_BATCHED_FP64; }
 // One-lane-per-cell kernels of a mode: ReactorCvode is the plain FP64 adaptive
-// BDF with its options (its calls run on the group form, gmode).
+// BDF with its options, and the batched forms are that BDF too; their calls run
+// on the group kernels (gmode) where the mechanism has any.
 int kmode(int mode) {
-  return mode == PP_CHEM_CVODE ? ppc::MODE_ADAPTIVE : (mode == PP_CHEM_ARKODE ? ppc::MODE_ERK : mode);
+  if (mode == PP_CHEM_CVODE || is_batched(mode)) return ppc::MODE_ADAPTIVE;
+  return mode == PP_CHEM_ARKODE ? ppc::MODE_ERK : mode;
 }
 
 // ---- device scratch of pp_chem_react_1d_noalloc: one array per GPU, held
@@ -412,8 +414,10 @@ int auto_cells_per_wave(const pp_chem* h, long long ncells) {
   return cpw;
 }
 
-// The handle's calls run on the work queue: the batched forms and ReactorCvode.
-bool on_queue(const pp_chem* h) { return is_batched(h->cfg.mode) || h->cfg.mode == PP_CHEM_CVODE; }
+// The handle's calls run on the work queue: the batched forms and ReactorCvode,
+// on the group kernels.  A mechanism that has none (three equations or fewer, or
+// more than three per lane of the widest group) runs them one cell per lane.
+bool on_queue(const pp_chem* h) { return h->GL && (is_batched(h->cfg.mode) || h->cfg.mode == PP_CHEM_CVODE); }
 // Batched kernels of the handle's mode.
 int gmode(const pp_chem* h) { return h->cfg.mode == PP_CHEM_CVODE ? ppc::MODE_GROUP_CVODE : h->cfg.mode; }
 
@@ -1043,8 +1047,7 @@ int pp_chem_react_box(pp_chem* h, const int lo[3], const int hi[3], const pp_arr
       e = h->L->flatten(fa, 0, s);
       if (e == hipSuccess) {
         const ppc::QueueArgs q = prepare_queue(h, ncells, rY->p, s);
-        e = (h->GL ? h->GL : h->L)
-                ->batched_1d(gmode(h), h->P, fa.y, fa.ysrc, fa.e, fa.esrc, *dt_react, q, counters(h), s);
+        e = h->GL->batched_1d(gmode(h), h->P, fa.y, fa.ysrc, fa.e, fa.esrc, *dt_react, q, counters(h), s);
       }
       if (e == hipSuccess) {
         fa.dt = 0.0;  // the 1-D kernel has already advanced e by dt * rEsrc

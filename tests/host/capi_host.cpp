@@ -255,6 +255,22 @@ void failed_growth(int which) {
   std::printf("checkpoints %d\n", (int)(which != 2 || h->d_ckpt));
 }
 
+// a mechanism without group kernels: the batched forms and ReactorCvode run on
+// the one-lane-per-cell kernels of the adaptive BDF
+void no_groups(int mode) {
+  pp_chem* h = handle("dodecane_lu", mode);
+  const auto say = [&](const char* what, int r) {
+    std::printf("%s %d\n%s_kernel %s\n%s_adaptive %d\n", what, r, what, fake::launched.c_str(), what,
+                (int)(fake::mode == ppc::MODE_ADAPTIVE && fake::P.adapt.fc_rhs == (mode == PP_CHEM_CVODE)));
+  };
+  fake::launched = "none";
+  say("react_1d", call_1d(h, 10));
+  say("box", call_box(h, 10));
+  say("chained", call_chained(h, 10, 2));
+  say("noalloc", call_noalloc(h, 10));
+  std::printf("rows %lld\n", pp_chem_workspace_rows(h));
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -263,6 +279,7 @@ int main(int argc, char** argv) {
   else if (s == "noalloc_shared") noalloc_shared();
   else if (s == "graph_counters") graph_counters();
   else if (s.rfind("failed_growth", 0) == 0) failed_growth(s.back() - '0');
+  else if (s.rfind("no_groups", 0) == 0) no_groups(s.back() - '0');
   else return 2;
   return 0;
 }

@@ -73,3 +73,14 @@ def test_failed_growth_leaves_no_stale_capacity(host, which):
     s = host(f"failed_growth{which}")
     assert s["before"] >= 0 and s["failed"] == -3 and s["after"] >= 0
     assert s["counters"] and s["staging"] and s["checkpoints"]
+
+
+@pytest.mark.parametrize("mode", [3, 4, 5])
+def test_mechanism_without_group_kernels(host, mode):
+    """A mechanism too small or too large for a group of lanes per cell has the
+    batched forms (3, 4) and ReactorCvode (5) on the one-lane kernels."""
+    s = host(f"no_groups{mode}")
+    for call, kernel in (("react_1d", "lane_1d"), ("box", "lane_box"), ("chained", "lane_1d"),
+                         ("noalloc", "lane_1d")):
+        assert s[call] == 0 and s[call + "_kernel"] == kernel and s[call + "_adaptive"] == 1, call
+    assert s["rows"] == 0
