@@ -409,6 +409,9 @@ int auto_cells_per_wave(const pp_chem* h, long long ncells) {
   int lanes = 64;
   while (lanes > 8 && lanes / 2 >= n) lanes /= 2;
   int cpw = 64 / lanes;
+  // (narrow groups of large tables do not fit the LDS: the next size there is)
+  while (cpw > 1 && h->GL->group_ws_rows(cpw) <= 0) cpw /= 2;
+  while (cpw < 8 && h->GL->group_ws_rows(cpw) <= 0) cpw *= 2;
   const long long waves = 8LL * std::max(h->ncu, 1);
   if (n <= 32 && h->GL->group_ws_rows(2 * cpw) > 0 && ncells >= kGroupRounds * waves * 2 * cpw) cpw *= 2;
   return cpw;

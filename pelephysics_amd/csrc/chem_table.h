@@ -29,6 +29,7 @@ namespace ppc {
 
 template <class T>
 struct TabMech {
+  using Tables = T;
   static constexpr int NS = T::NS, NR = T::NR, NEQ = T::NEQ;
   static constexpr int NQ = T::NQ, NX = T::NX;
   static constexpr bool kTable = true;

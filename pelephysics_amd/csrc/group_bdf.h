@@ -55,6 +55,7 @@
 #include "reactors.h"
 #include "wave.h"
 #include "pack.h"
+#include "group_layout.h"
 
 namespace ppc {
 
@@ -174,9 +175,6 @@ PPC_DI typename T::Packed& lds_pack() {
   return p;
 }
 
-// Waves per block of the group kernels: they share one copy of the tables.
-constexpr int GROUP_WAVES = 4;
-
 // Fills it, by every thread of the block.
 template <class T>
 PPC_DI const typename T::Packed& load_pack() {
@@ -228,37 +226,14 @@ struct GroupChem {
   using TM = TabMech<PackTab<T>>;
   using PK = typename T::Packed;
   using Gr = Grp<G>;
-  static constexpr int NS = T::NS, NR = T::NR, n = T::NEQ, NX = T::NX, NCH = T::NCH;
-  static constexpr int NG = 64 / G;
-  static constexpr int EPL = (n + G - 1) / G;    // equation slots per lane
-  static constexpr int SPL = (NS + G - 1) / G;   // species slots per lane
-  static constexpr int SPX = (NX + G - 1) / G;   // with the QSS species
+  using L = GroupLayout<T, G>;
+  static constexpr int NS = L::NS, NR = L::NR, n = L::n, NX = L::NX, NCH = L::NCH, NQ = L::NQ, NROW = L::NROW;
+  static constexpr int NG = L::NG, EPL = L::EPL, SPL = L::SPL, SPX = L::SPX, NP = L::NP, NRATE = L::NRATE;
   static constexpr int TL = NS % G, TS = NS / G;  // lane and slot of the temperature equation
-  static constexpr int NP = (n + 1) & ~1;        // vectors of n, 16-byte aligned
-
-  // A group's LDS area (doubles): concentrations with exp(-g/RT) and
-  // c exp(g/RT) of every species, an unused place's ones after them (later
-  // the chunk sums), then the rates of progress with a zero after them (later
-  // the vectors of the Newton solve).  Its size is 4 modulo 8 doubles, so that
-  // the groups' broadcasts fall into different banks.
-  static constexpr int cmax(int a, int b) { return a > b ? a : b; }
-  static constexpr int S_CA = 0, S_B = 2 * (NX + 1);
-  static constexpr int NQ = T::NQ, NROW = NQ > 0 ? T::NSLOT + NQ : 0;  // QSS balances: entries and right-hand sides
-  static constexpr int S_Q = (cmax(cmax(3 * (NX + 1), NCH), 2 * (NX + 1) + NROW) + 1) & ~1;
-  static constexpr int NRATE = NQ > 0 ? 2 * NR + 1 : NR + 1;  // QSS: forward and reverse rates apart
-  static constexpr int S_RAW = S_Q + cmax(NRATE, 3 * NP);
-  static constexpr int AREA = ((S_RAW + 3) / 8) * 8 + 4;
-  // The wave's Jacobian area overlays its groups' areas: 5 species vectors and,
-  // where n is small enough, the n x n accumulator.
-  // (QSS mechanisms: each group works on its own cell's Jacobian, in the workspace.)
-  static constexpr bool JLDS = n <= 32 && NQ == 0;
-  static constexpr int J_AT = (5 * NP + 1) & ~1;
-  // Jacobian accumulators in the workspace (doubles): n x n (JSQ) of the wave,
-  // or of each group with the QSS terms after it (JSTRIDE); of a wave
-  static constexpr int JSQ = (n * n + 1) & ~1;
-  static constexpr int JSTRIDE = NQ > 0 ? (JSQ + NQ * NS + 2 * T::NQR + 1) & ~1 : JSQ;
-  static constexpr int JSPACE = NQ > 0 ? NG * JSTRIDE : JSTRIDE;
-  static constexpr int WAREA = (cmax(NG * AREA, J_AT + (JLDS ? n * n : 0)) + 3) & ~3;
+  static constexpr int S_CA = L::S_CA, S_B = L::S_B, S_Q = L::S_Q, AREA = L::AREA, WAREA = L::WAREA;
+  static constexpr bool JLDS = L::JLDS;
+  static constexpr int J_AT = L::J_AT, JSQ = L::JSQ, JSTRIDE = L::JSTRIDE, JSPACE = L::JSPACE;
+  static constexpr int cmax(int a, int b) { return L::cmax(a, b); }
 
   PPC_DI static void coefs(const PK& pk, const int k, const double Tv, double (&a)[7], double& imw) {
     const double* s = pk.sp[k].lo;
@@ -709,7 +684,6 @@ __device__ __noinline__ void group_qss_jacobian(double* sh, double* J, const boo
   using TM = TabMech<PackTab<T>>;
   constexpr int NS = T::NS, n = T::NEQ, NX = T::NX, NQ = T::NQ, SPL = C::SPL, SPX = C::SPX, NROW = C::NROW;
   constexpr int RPL = (NROW + G - 1) / G;
-  static_assert(6 * NX + NROW <= C::AREA, "the Jacobian's vectors fit the group's area");
   const typename T::Packed& pk = lds_pack<T>();
   const int g = Gr::lane();
   double* const X = J + C::JSQ;
@@ -1045,7 +1019,7 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
   using PK = typename T::Packed;
   constexpr int n = C::n, NS = C::NS, EPL = C::EPL, SPL = C::SPL, NP = C::NP;
   __shared__ __attribute__((aligned(16))) double lds[GROUP_WAVES * C::WAREA];
-  __shared__ double lvec[GROUP_WAVES * 4 * 64 * EPL];
+  __shared__ double lvec[GROUP_WAVES * C::L::LVEC];
   const PK& pk = load_pack<T>();
   const int wv = (int)(threadIdx.x >> 6);
   const long long wid = (long long)blockIdx.x * GROUP_WAVES + wv;
@@ -1053,7 +1027,7 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
   const int g = Gr::lane();
   const int gi = (int)__lane_id() / G;
   double* const wa = lds + wv * C::WAREA;
-  double* const lv = lvec + wv * (4 * 64 * EPL) + (threadIdx.x & 63);
+  double* const lv = lvec + wv * C::L::LVEC + (threadIdx.x & 63);
   double* const sh = wa + gi * C::AREA;
   double* const sv = sh + C::S_Q;
   double* const sw = sv + NP;

@@ -399,6 +399,21 @@ struct RowSolve {
   }
 };
 
+// A group's Jacobian, right-hand side and Krylov space share one area (doubles).
+template <class T>
+constexpr int group_fixed_area() {
+  using L = GroupLayout<T, 16>;
+  return ((L::cmax(L::cmax(RowSolve<L::n, L::EPL>::SIZE, L::AREA), L::J_AT + L::n * L::n) + 3) / 8) * 8 + 4;
+}
+template <class M>
+constexpr bool group_fixed_fits() {
+  if constexpr (group_fixed_ok<M>()) {
+    using T = typename packed_tables<M>::type;
+    return (long long)sizeof(typename T::Packed) + 8LL * GROUP_WAVES * 4 * group_fixed_area<T>() <= LDS_BYTES;
+  }
+  return false;
+}
+
 template <class T, bool BOX>
 __global__ void __launch_bounds__(64 * GROUP_WAVES) __attribute__((amdgpu_waves_per_eu(1, 8)))
 group_bdf_fixed_kernel(ReactParamsDev P, GroupIO io, double dt_react, int ncells, CellStats st) {
@@ -408,8 +423,7 @@ group_bdf_fixed_kernel(ReactParamsDev P, GroupIO io, double dt_react, int ncells
   using Cell = GroupCell<T, G, BOX>;
   constexpr int n = C::n, EPL = C::EPL, SPL = C::SPL;
   using RS = RowSolve<n, EPL>;
-  // a group's Jacobian, right-hand side and Krylov space share one area
-  constexpr int RSIZE = ((C::cmax(C::cmax(RS::SIZE, C::AREA), C::J_AT + n * n) + 3) / 8) * 8 + 4;
+  constexpr int RSIZE = group_fixed_area<T>();
   static_assert(C::JLDS, "the Jacobian of these mechanisms is in LDS");
   __shared__ __attribute__((aligned(16))) double lds[GROUP_WAVES * NG * RSIZE];
   const auto& pk = load_pack<T>();

@@ -13,6 +13,7 @@
 #pragma once
 #include <type_traits>
 #include "erk_tables.h"
+#include "group_layout.h"
 #include "ppc_common.h"
 #include "reactors_fwd.h"
 
@@ -89,13 +90,33 @@ struct has_qss : std::false_type {};
 template <class M>
 struct has_qss<M, std::void_t<decltype(M::NQ)>> : std::integral_constant<bool, (M::NQ > 0)> {};
 
+// The packed tables the group kernels read (the generator leaves them out for a
+// mechanism that their records cannot hold).
+template <class M, class = void>
+struct packed_tables {
+  using type = void;
+};
+template <class M>
+struct packed_tables<M, std::void_t<typename M::Tables::Packed>> {
+  using type = typename M::Tables;
+};
+
 // QSS mechanisms: at most one equation in four is in a second slot (NEQ <=
 // 4 G / 3).  A group keeps its forward and reverse rates apart, twice the LDS,
 // so a narrow group's waves do not share a SIMD (LuEthylene_qss, 65536 cells:
-// 16 lanes 81 ms, 32 lanes 60 ms; 4096 cells 9.1 and 7.0 ms).
+// 16 lanes 81 ms, 32 lanes 60 ms; 4096 cells 9.1 and 7.0 ms).  The tables and
+// the areas of a block must fit the LDS: the narrower the groups, the more of
+// them a wave has.
 template <class M, int G>
 constexpr bool group_ok() {
-  return has_table<M>::value && M::NEQ <= 3 * G && G <= 2 * M::NEQ && (!has_qss<M>::value || 3 * M::NEQ <= 4 * G);
+  using T = typename packed_tables<M>::type;
+  if constexpr (std::is_void<T>::value) {
+    return false;
+  } else if constexpr (!(M::NEQ <= 3 * G && G <= 2 * M::NEQ && (!has_qss<M>::value || 3 * M::NEQ <= 4 * G))) {
+    return false;
+  } else {
+    return has_table<M>::value && GroupLayout<T, G>::fits();
+  }
 }
 
 // The fixed-step BDF's group kernel (16 lanes per cell) holds the Krylov bases

@@ -196,7 +196,7 @@ hipError_t launch_group_fixed(int mode, const ReactParamsDev& P, double* y, cons
       }
       return hipErrorInvalidValue;
     }
-    if constexpr (group_fixed_ok<M>()) {
+    if constexpr (group_fixed_fits<M>()) {
       if (mode == MODE_BDF) {
         if (ncells == 0) return hipSuccess;
         return b ? launch_group_bdf_fixed<Tab, true>(P, io, dt, ncells, st, s)

@@ -34,7 +34,8 @@ unused place is reaction NR with coefficient 0; ``spCh``: first chunk of each
 species), so that the lanes of a group share the long rows.  Its reaction
 order is the table order with the reversible elementary reactions first
 (``perm``: position in the tables above), so that a wave's lanes agree on
-whether there is a reverse rate.  QSS mechanisms add the balances' terms in the
+whether there is a reverse rate.  A mechanism beyond those records (254 species,
+4095 reactions) gets no ``kPack``.  QSS mechanisms add the balances' terms in the
 same chunks (``qch``, reaction + NR for a reverse rate), by matrix entry, then by
 right-hand side (``qRow``: first chunk of each; ``qInit``: the entries' constant
 parts), and the elimination as code (``qss_eliminate``).
@@ -158,6 +159,11 @@ def qss_elimination(m: Mechanism):
 CHUNK = 8
 
 
+class Unpackable(ValueError):
+    """A mechanism that the packed tables cannot hold: its header has none, and
+    its calls run on the one-lane-per-cell kernels."""
+
+
 def qss_program(w, lu, fs, bs) -> None:
     """The elimination and the solution of the QSS balances as straight-line
     code: every lane of a group runs it on registers."""
@@ -179,7 +185,7 @@ def emit_pack(w, m: Mechanism, R: List[Reaction], n_el: int) -> None:
     table order, its first n_el reactions elementary."""
     ns, nx, nr = m.n_species, m.n_species + m.n_qss, len(R)
     if nx > 254 or nr > 4095:
-        raise ValueError("mechanism too large for the packed tables")
+        raise Unpackable("mechanism too large for the packed tables")
 
     def shape(j):
         r = R[j]
@@ -193,7 +199,7 @@ def emit_pack(w, m: Mechanism, R: List[Reaction], n_el: int) -> None:
         pp = [nx if k < 0 else k for k in (_expand(r.products) if r.reversible else [-1] * MAXR)]
         d = int(round(r.delta_order()))
         if r.reversible and abs(d) > 100:
-            raise ValueError("reaction order out of range")
+            raise Unpackable("reaction order out of range")
         flags = (1 if r.reversible else 0) + (2 if r.fwd_removed else 0)
         rx.append(f"{{{_f(r.rate.A)}, {_f(r.rate.b)}, {_f(r.rate.EaR)}, "
                   f"{{{', '.join(map(str, rr))}}}, {{{', '.join(map(str, pp))}}}, {d if r.reversible else 0}, {flags}}}")
@@ -219,7 +225,7 @@ def emit_pack(w, m: Mechanism, R: List[Reaction], n_el: int) -> None:
             v = r.net_stoich().get(k, 0.0)
             if v:
                 if v != int(v) or not -8 <= v <= 7:
-                    raise ValueError("net coefficient out of range")
+                    raise Unpackable("net coefficient out of range")
                 terms.append((pos[j], int(v)))
         terms.sort()
         for i in range(0, len(terms), CHUNK):
@@ -229,7 +235,7 @@ def emit_pack(w, m: Mechanism, R: List[Reaction], n_el: int) -> None:
     qch, qfirst, qinit = [], [], []
     if m.n_qss:
         if any(k >= ns for r in R for k in r.efficiencies):
-            raise ValueError("a QSS species as a third body is not supported")
+            raise Unpackable("a QSS species as a third body is not supported")
         terms, slot, init, _, _, _ = qss_elimination(m)
         order = ordered(m)
         yaml_pos = {order[j]: i for j, i in pos.items()}
@@ -238,10 +244,10 @@ def emit_pack(w, m: Mechanism, R: List[Reaction], n_el: int) -> None:
             row = len(slot) + q if c < 0 else slot[(q, c)]
             mul = cf if c < 0 or c == q else -cf
             if mul != int(mul) or not -8 <= mul <= 7:
-                raise ValueError("QSS balance coefficient out of range")
+                raise Unpackable("QSS balance coefficient out of range")
             qrows[row].append((yaml_pos[j] + (nr if d else 0), int(mul)))
         if 2 * nr > 4095:
-            raise ValueError("mechanism too large for the packed QSS balances")
+            raise Unpackable("mechanism too large for the packed QSS balances")
         qfirst = [0]
         for t in qrows:
             for i in range(0, len(t), CHUNK):
@@ -412,7 +418,12 @@ def emit(m: Mechanism, source: str) -> str:
         qss_counts = {"NQR": len(qrx), "NSLOT": len(slot), "NLU": len(lu), "NFS": len(fs)}
     tab.emit(w, "Tables")
     w("")
-    emit_pack(w, m, R, n_el)
+    try:
+        emit_pack(w, m, R, n_el)
+        packed = True
+    except Unpackable as e:
+        w(f"// no packed tables: {e}")
+        packed = False
     w("")
     w("}  // namespace")
     w("")
@@ -424,9 +435,10 @@ def emit(m: Mechanism, source: str) -> str:
     w("  static constexpr int " + ", ".join(f"{k} = {v}" for k, v in qss_counts.items()) + ";")
     w(f"  static constexpr int N_EL = {n_el}, N_TB = {n_tb}, N_TROE = {n_troe}, N_LIND = {n_lind};")
     w(f"  static constexpr int MAXR = {MAXR}, MAXNET = {MAXNET};")
-    w(f"  static constexpr int NCH = {m.name}_t::kChunks;")
-    w(f"  using Packed = {m.name}_t::Packed;")
-    w(f"  PPC_DI static const Packed& pack() {{ return {m.name}_t::kPack; }}")
+    if packed:
+        w(f"  static constexpr int NCH = {m.name}_t::kChunks;")
+        w(f"  using Packed = {m.name}_t::Packed;")
+        w(f"  PPC_DI static const Packed& pack() {{ return {m.name}_t::kPack; }}")
     for nm in ("nasaLo", "nasaHi", "tmid", "mw", "imw", "rxA", "rxB", "rxE", "rxNu", "effV", "foA",
                "foB", "foE", "troe", "spNu"):
         w(f"  PPC_DI static double {nm}_(int i) {{ return {m.name}_t::kTab.{nm}[i]; }}")

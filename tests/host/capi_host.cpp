@@ -53,6 +53,7 @@ hipError_t mech_eval(int, const double*, const double*, int, double*, hipStream_
 long long no_rows(int) { return 0; }
 long long lane_rows(int) { return 5000; }
 long long group_rows(int cpw) { return cpw == 4 ? 52 : (cpw == 2 ? 30 : 0); }
+long long wide_rows(int cpw) { return cpw == 1 ? 20 : 0; }
 
 // 20 species; a workspace of the one-lane kernels and group kernels as asked
 MechLauncher mech(const char* name, bool lane_ws, bool groups) {
@@ -66,13 +67,19 @@ MechLauncher mech(const char* name, bool lane_ws, bool groups) {
 }
 }  // namespace fake
 
-// The mechanisms: "heptane_lu_88sk" with a workspace, "dodecane_lu" without
-// group kernels, the others with both unneeded or present.
+// The mechanisms: "heptane_lu_88sk" with a workspace of the one-lane kernels,
+// "dodecane_lu" without group kernels, "LuEthylene_qss" with the widest groups
+// only, the others with groups of 16 and 32 lanes and no such workspace.
 namespace ppc {
-#define PPC_MECH(M)                                                                                        \
-  const MechLauncher* launcher_##M() {                                                                     \
-    static const MechLauncher L = fake::mech(#M, !std::strcmp(#M, "heptane_lu_88sk"), std::strcmp(#M, "dodecane_lu") != 0); \
-    return &L;                                                                                             \
+#define PPC_MECH(M)                                                                   \
+  const MechLauncher* launcher_##M() {                                                \
+    static const MechLauncher L = [] {                                                \
+      const std::string name = #M;                                                    \
+      MechLauncher l = fake::mech(#M, name == "heptane_lu_88sk", name != "dodecane_lu"); \
+      if (name == "LuEthylene_qss") l.group_ws_rows = &fake::wide_rows;               \
+      return l;                                                                       \
+    }();                                                                              \
+    return &L;                                                                        \
   }
 #include "../../pelephysics_amd/csrc/inst/registry.inc"
 #undef PPC_MECH
@@ -271,6 +278,17 @@ void no_groups(int mode) {
   std::printf("rows %lld\n", pp_chem_workspace_rows(h));
 }
 
+// cells per wave of a call, where the caller leaves them to the library
+void group_size() {
+  for (const char* name : {"drm19", "LuEthylene_qss"}) {
+    pp_chem* h = handle(name, PP_CHEM_BDF_BATCHED_FP64);
+    for (int n : {1, 10000}) {
+      const int r = call_1d(h, n);
+      std::printf("%s_%d %d\n", name, n, r == 0 ? fake::P.adapt.group : r);
+    }
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -280,6 +298,7 @@ int main(int argc, char** argv) {
   else if (s == "graph_counters") graph_counters();
   else if (s.rfind("failed_growth", 0) == 0) failed_growth(s.back() - '0');
   else if (s.rfind("no_groups", 0) == 0) no_groups(s.back() - '0');
+  else if (s == "group_size") group_size();
   else return 2;
   return 0;
 }

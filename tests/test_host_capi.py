@@ -84,3 +84,11 @@ def test_mechanism_without_group_kernels(host, mode):
                          ("noalloc", "lane_1d")):
         assert s[call] == 0 and s[call + "_kernel"] == kernel and s[call + "_adaptive"] == 1, call
     assert s["rows"] == 0
+
+
+def test_group_size_there_is(host):
+    """A call takes the narrowest group with a lane per equation (large calls
+    half of it), or the next size that the mechanism has kernels of."""
+    s = host("group_size")
+    assert s["drm19_1"] == 2 and s["drm19_10000"] == 4
+    assert s["LuEthylene_qss_1"] == 1 and s["LuEthylene_qss_10000"] == 1
