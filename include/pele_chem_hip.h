@@ -82,8 +82,10 @@ typedef struct {
   int block_size; /* threads per block, 0: default (64) */
   /* Upper bound on the device workspace that holds the per-cell matrices of
    * mechanisms with more than 31 species (Jacobian, LU, Krylov basis; too large
-   * for a lane's private memory); 0: default (32 GiB).  Fewer resident cells
-   * are integrated at once when it is reached. */
+   * for a lane's private memory), and where batched_cells_per_wave names a group
+   * size, its Jacobians; 0: default (32 GiB).  Fewer resident cells are
+   * integrated at once when it is reached.  The other mechanisms' groups keep
+   * Jacobians of at most some 60 MB there, which it does not limit. */
   long long workspace_bytes;
   /* ode.clean_init_massfrac (ReactorBDF.cpp:127, ReactorRK64.cpp:18): the
    * box <-> flat conversion clips rhoY to [0, rho] and re-applies the
@@ -307,9 +309,10 @@ int pp_chem_num_reactions(const pp_chem* h);
  * the kernel is in pp_chem_get_stats().kernel_ms. */
 int pp_chem_adjoint_1d(pp_chem* h, double* y, const double* rX, int ncells, int nmacro, double dt,
                        int spec_a, int spec_b, double* out, double* grad, void* stream);
-/* Doubles per resident cell of the per-cell matrix workspace the handle's
- * integrator uses (0: the matrices stay in private memory).  No counterpart in
- * the reference; for sizing pp_chem_config.workspace_bytes. */
+/* Doubles per lane of the matrix workspace the handle's integrator uses (0: the
+ * matrices stay in private memory); 64 lanes hold 64 cells of the one-lane
+ * kernels, 64 / (lanes per cell) of the group kernels (a large call's groups).
+ * No counterpart in the reference; for sizing pp_chem_config.workspace_bytes. */
 long long pp_chem_workspace_rows(const pp_chem* h);
 /* Per-cell accepted step counts of the last call (host copy). */
 int pp_chem_copy_cell_steps(pp_chem* h, int* host_out, int ncells);

@@ -496,7 +496,11 @@ int prepare_workspace(pp_chem* h, int ncells) {
   long long rows = 0;
   long long blocks = workspace_blocks(h, ncells, cpw, rows);
   if (blocks == 0) return 0;
-  const long long cap = h->cfg.workspace_bytes > 0 ? h->cfg.workspace_bytes : kWsMaxBytes;
+  // workspace_bytes limits the mechanisms whose one-lane kernels keep their
+  // matrices there too, and a named group; the other mechanisms' groups need
+  // at most some 60 MB, for 8 waves per CU
+  const bool limited = h->cfg.batched_cells_per_wave != 0 || h->L->ws_rows(kmode(h->cfg.mode)) > 0;
+  const long long cap = limited && h->cfg.workspace_bytes > 0 ? h->cfg.workspace_bytes : kWsMaxBytes;
   const long long lane_bytes = 64 * rows * (long long)sizeof(double);  // one 64-lane block
   if (lane_bytes > cap) return fail(h, PP_CHEM_EINVAL, "workspace_bytes below one 64-cell block");
   blocks = std::min(blocks, cap / lane_bytes);

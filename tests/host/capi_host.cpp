@@ -289,6 +289,23 @@ void group_size() {
   }
 }
 
+// workspace_bytes below one wave's workspace
+void small_workspace() {
+  pp_chem* h = handle("drm19", PP_CHEM_BDF_ADAPTIVE_MIXED, 1000);
+  std::printf("small_mechanism %d\n", call_1d(h, 100));
+  std::printf("workspace_lanes %lld\n", fake::P.ws_lanes);
+  h = handle("drm19", PP_CHEM_CVODE, 1000);
+  std::printf("small_mechanism_cvode %d\n", call_box(h, 100));
+  h = handle("heptane_lu_88sk", PP_CHEM_BDF_ADAPTIVE_MIXED, 1000);
+  std::printf("large_mechanism %d\n", call_1d(h, 100));
+  pp_chem_config c;
+  pp_chem_config_init(&c, "drm19_table", PP_CHEM_BDF_ADAPTIVE_MIXED, 2);
+  c.workspace_bytes = 1000;
+  c.batched_cells_per_wave = 4;
+  pp_chem_create(&c, &h);
+  std::printf("named_group %d\n", call_1d(h, 100));
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -299,6 +316,7 @@ int main(int argc, char** argv) {
   else if (s.rfind("failed_growth", 0) == 0) failed_growth(s.back() - '0');
   else if (s.rfind("no_groups", 0) == 0) no_groups(s.back() - '0');
   else if (s == "group_size") group_size();
+  else if (s == "small_workspace") small_workspace();
   else return 2;
   return 0;
 }

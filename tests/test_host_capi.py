@@ -92,3 +92,13 @@ def test_group_size_there_is(host):
     s = host("group_size")
     assert s["drm19_1"] == 2 and s["drm19_10000"] == 4
     assert s["LuEthylene_qss_1"] == 1 and s["LuEthylene_qss_10000"] == 1
+
+
+def test_workspace_bytes_limits_the_large_mechanisms(host):
+    """workspace_bytes is a limit for mechanisms with more than 31 species, whose
+    matrices are in device memory, and where the caller names a group size; the
+    others' calls took any value before their groups kept Jacobians there."""
+    s = host("small_workspace")
+    assert s["small_mechanism"] == 0 and s["small_mechanism_cvode"] == 0
+    assert s["workspace_lanes"] == 64 * 16  # every wave it can use (two compute units)
+    assert s["large_mechanism"] == -1 and s["named_group"] == -1
