@@ -1301,6 +1301,10 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
           for (int e = 0; e < EPL; ++e) D[1][e] *= h_abs;
           need_jac = 1;
           new_step = true;
+          if (CV && !(t < t_bound)) {  // nothing to integrate (dt <= 0): no step, as adaptive_cell
+            attempt = false;
+            finish = true;
+          }
         }
       } else {
         // one modified-Newton iteration with f = f(t_new, yv)

@@ -102,3 +102,22 @@ def test_cvode_options_refused_elsewhere(ident):
     R = ReactorBase.create(ident)
     with pytest.raises(ReactorError):
         R.init(2, 8, mechanism="drm19", max_order=2)
+
+
+@pytest.mark.parametrize("dt", [0.0, -1e-7])
+def test_cvode_nothing_to_integrate(models, oracles, dt):
+    """dt = 0 (or less): no step is taken, no cell fails and the state stays, as
+    in the oracle; the right-hand side was evaluated twice for the first step
+    size."""
+    torch = _torch()
+    m, st, _, _ = _cells(models, n=70)
+    rng = np.random.default_rng(2)
+    ysrc, esrc = 1e-2 * rng.standard_normal(st.rY.shape) * st.rY, 10.0 * np.abs(st.rE)
+    ret, y, rX, R = _run_1d(torch, "drm19", "ReactorCvode", st, ysrc, esrc, dt)
+    oret, oy, orX, ost = _oracle_1d(oracles["drm19"], "adaptive", st, ysrc, esrc, dt,
+                                    params=oracle.adapt_params(**CVODE))
+    s = R.stats()
+    assert oret == 0 and s["nsteps"] == 0 and s["nfailed"] == 0
+    assert ret == 2 and s["nrhs"] == ost["nrhs"] == 2 * st.ncells
+    assert np.array_equal(y, st.y_1d()) and np.array_equal(oy, y)
+    assert np.allclose(rX, orX, rtol=4e-16, atol=0.0)  # one rounding less with a fused multiply-add
