@@ -99,6 +99,33 @@ def test_rk64_on_both_sides_of_the_lane_kernel(models):
     _compare_y(m.n_species + 1, out[0][0], out[1][0])
 
 
+def test_statistics_and_cost_order_of_a_large_call(models):
+    """More cells than the bookkeeping kernels have threads, an odd number of
+    them: the statistics are those of the per-cell counts, and the second call,
+    which visits the cells in the order of the first one's costs, integrates each
+    of them once (the same state, from the same start)."""
+    torch = _torch()
+    from pelephysics_amd.reactor import ReactorBase
+    m, st, _, _ = _cells(models, "LiDryer", 4096)
+    n = 1024 * 256 + 4099
+    s = W.subsample(st, np.arange(n) % st.ncells)
+    R = ReactorBase.create("ReactorBDFAdaptiveMixed")
+    R.init(2, n, mechanism="LiDryer", rtol=1e-6, atol=1e-10)
+    dev = torch.device("cuda:0")
+    y0, x0 = torch.from_numpy(s.y_1d()).to(dev), torch.from_numpy(s.rE.copy()).to(dev)
+    ys, xs = torch.zeros(n * m.n_species, dtype=torch.float64, device=dev), torch.zeros(n, dtype=torch.float64, device=dev)
+    y, x = y0.clone(), x0.clone()
+    R.react_1d(y, ys, x, xs, 2e-6)
+    first, steps = y.clone(), R.cell_steps(n)
+    y.copy_(y0)
+    x.copy_(x0)
+    R.react_1d(y, ys, x, xs, 2e-6)
+    assert torch.equal(y, first) and np.array_equal(R.cell_steps(n), steps)
+    t = R.stats()
+    assert (t["nsteps"], t["max_steps_cell"], t["min_steps_cell"]) == (steps.sum(), steps.max(), steps.min())
+    assert t["ncells"] == n and t["nfailed"] == 0 and steps.max() > steps.min() > 0
+
+
 @pytest.mark.parametrize("mech", ["drm19", "LiDryer", "dodecane_lu"])
 def test_production_rate_counts(models, oracles, mech):
     """64 cells per block: the last block's remainder.  The tolerance is the mechanism tests'."""
