@@ -90,11 +90,22 @@ __global__ void __launch_bounds__(256) reduce_stats(const int* __restrict__ nste
     mx = omx > mx ? omx : mx;
     mn = omn < mn ? omn : mn;
   }
+  __shared__ unsigned long long part[4][NSTAT];
   if ((threadIdx.x & 63) == 0) {
-    for (int i = 0; i < 7; ++i)
-      if (s[i]) atomicAdd(&acc[i], s[i]);
-    atomicMax(&acc[7], (unsigned long long)mx);
-    atomicMax(&acc[8], (unsigned long long)(0x7fffffff - mn));
+    unsigned long long* const p = part[threadIdx.x >> 6];
+    for (int i = 0; i < 7; ++i) p[i] = s[i];
+    p[7] = (unsigned long long)mx;
+    p[8] = (unsigned long long)(0x7fffffff - mn);
+  }
+  __syncthreads();
+  if (threadIdx.x < NSTAT) {
+    const int i = threadIdx.x;
+    unsigned long long v = part[0][i];
+    for (int w = 1; w < 4; ++w) v = i < 7 ? v + part[w][i] : (part[w][i] > v ? part[w][i] : v);
+    if (i < 7)
+      atomicAdd(&acc[i], v);
+    else
+      atomicMax(&acc[i], v);
     __threadfence();
   }
   __syncthreads();
@@ -327,7 +338,8 @@ hipError_t clear_stats(pp_chem* h) {
 // int(average steps) or an error.
 int finish(pp_chem* h, int ncells, hipStream_t s, const ppc::CellStats& st) {
   h->h_red[NSTAT - 1] = NOT_DELIVERED;
-  const int blocks = ncells > 0 ? (ncells + 255) / 256 < 1024 ? (ncells + 255) / 256 : 1024 : 1;
+  // a block per compute unit: its sums meet the others' on nine words
+  const int blocks = std::max(1, std::min(std::max(h->ncu, 1), (ncells + 255) / 256));
   hipLaunchKernelGGL(reduce_stats, dim3(blocks), dim3(256), 0, s, st.nsteps, st.nrhs, st.njac, st.nlu,
                      st.nnewton, st.nreject, ncells, h->d_red, h->h_red);
   HIPCHK(h, hipGetLastError());
