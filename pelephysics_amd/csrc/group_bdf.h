@@ -221,6 +221,10 @@ struct PackTab : T {
 };
 
 // ------------------------------------------- the mechanism on a group --
+typedef __attribute__((address_space(3))) double lds_double;
+template <class T, int G, int WD>
+__device__ void group_qss_jacobian(lds_double* area, double* Jws, const bool eform);
+
 template <class T, int G>
 struct GroupChem {
   using TM = TabMech<PackTab<T>>;
@@ -231,7 +235,7 @@ struct GroupChem {
   static constexpr int NG = L::NG, EPL = L::EPL, SPL = L::SPL, SPX = L::SPX, NP = L::NP, NRATE = L::NRATE;
   static constexpr int TL = NS % G, TS = NS / G;  // lane and slot of the temperature equation
   static constexpr int S_CA = L::S_CA, S_B = L::S_B, S_Q = L::S_Q, AREA = L::AREA, WAREA = L::WAREA;
-  static constexpr bool JLDS = L::JLDS;
+  static constexpr bool JLDS = L::JLDS, JOWN = L::JOWN;
   static constexpr int J_AT = L::J_AT, JSQ = L::JSQ, JSTRIDE = L::JSTRIDE, JSPACE = L::JSPACE;
   static constexpr int cmax(int a, int b) { return L::cmax(a, b); }
 
@@ -647,6 +651,19 @@ struct GroupChem {
   }
   PPC_DI static double jload(const double* J, const int i) { return JLDS ? J[i] : ws_load(J + i); }
 
+  // The Jacobian of one cell by WD lanes, y in their area wa: in wa at J_AT or
+  // (Jws) in the workspace.
+  template <int WD>
+  PPC_DI static void cell_jacobian(const PK& pk, double* wa, double* J, const bool eform) {
+    if constexpr (NQ > 0) {
+      group_qss_jacobian<T, G, WD>((lds_double*)wa, J, eform);
+    } else if (eform) {
+      jacobian<0, WD>(pk, wa, J);
+    } else {
+      jacobian<1, WD>(pk, wa, J);
+    }
+  }
+
   // d f_i / d y_j of jacobian()'s J: the DWDOT scaling (T column x1e-6, T row
   // x1e6) and the molecular-weight scaling
   PPC_DI static double jac_elem(const PK& pk, const double* J, const int i, const int j) {
@@ -658,42 +675,63 @@ struct GroupChem {
     v *= j < NS ? pk.sp[j].imw : 1.0;
     return v;
   }
-  // all of them, element (i, j) at out[(e*n + j)*G + g] for i = e*G + g
-  template <typename JT>
+  // all of them by WD lanes, element (i, j) at out[(e*n + j)*G + g] for i = e*G + g
+  template <int WD, typename JT>
   PPC_DI static void jac_rows(const PK& pk, const double* J, JT* out) {
 #pragma unroll 4
-    for (int t = (int)__lane_id(); t < n * n; t += 64) {
+    for (int t = Grp<WD>::lane(); t < n * n; t += WD) {
       const int j = t / n, i = t - j * n;
       out[((i / G) * n + j) * G + i % G] = (JT)jac_elem(pk, J, i, j);
     }
   }
 };
 
-// The QSS mechanisms' Jacobian (TabMech::jacobian_qss) of a group's cell by its
-// lanes: y in the group's LDS area sh, which is overwritten; J (n x n, column
-// major) in the workspace, followed by the derivatives of the balances
-// (NQ x NS) and the QSS reactions' rates (2 NQR).  Reactions are split over the
-// lanes, with atomic sums; the QSS solves, and d wdot / d x, over the columns.
-// Out of line: it is rare (about one per cell and call) and must not weigh on
-// the registers of the steps.  By one lane per cell it was 90% of a call
-// (LuEthylene_qss, 4096 cells, 1e-5 s: 14 ms per Jacobian).
-template <class T, int G>
-__device__ __noinline__ void group_qss_jacobian(double* sh, double* J, const bool eform) {
-  using C = GroupChem<T, G>;
-  using Gr = Grp<G>;
+// The QSS mechanisms' Jacobian (TabMech::jacobian_qss) of one cell by WD lanes
+// (its group, or the wave): y in their LDS area, which is overwritten; J (n x n,
+// column major) in that area at J_AT or in the workspace, followed by X, the
+// derivatives of the balances by the concentrations (NQ x NS; then d x / d c), and
+// W, d wdot / d x (NQ x NS).  Reactions are split over the lanes, with atomic sums;
+// the QSS solves over the columns, and W X over its elements.
+// Out of line: it is rare (about one per cell and call) and must not weigh on the
+// registers of the steps.  What bounds it: the latency of the reactions' tables and
+// of the rounds of unlike reaction kinds.  By one lane per cell it was 90% of a call
+// (LuEthylene_qss, 4096 cells, 1e-5 s: 14 ms per Jacobian); with its sums in the
+// workspace, and W X as a loop over all QSS reactions in every column, 65 to 90% of
+// a call of up to 30 steps (figures at GroupLayout).
+template <class T, int G, int WD>
+__device__ __noinline__ void group_qss_jacobian(lds_double* area, double* Jws, const bool eform) {
+  using C = GroupChem<T, WD>;
+  using L = GroupLayout<T, G>;
+  using Gr = Grp<WD>;
   using TM = TabMech<PackTab<T>>;
   constexpr int NS = T::NS, n = T::NEQ, NX = T::NX, NQ = T::NQ, SPL = C::SPL, SPX = C::SPX, NROW = C::NROW;
-  constexpr int RPL = (NROW + G - 1) / G;
+  constexpr int RPL = (NROW + WD - 1) / WD;
   const typename T::Packed& pk = lds_pack<T>();
   const int g = Gr::lane();
-  double* const X = J + C::JSQ;
-  double* const qq = X + NQ * NS;
+  double* const sh = (double*)area;
+  double* const J = L::JLDS ? sh + L::J_AT : Jws;
+  double *const X = J + L::JSQ, *const W = X + NQ * NS;
+  const auto ld = [&](const double* p) { return L::JLDS ? *p : ws_load(p); };
+  const auto st = [&](double* p, double v) {
+    if (L::JLDS)
+      *p = v;
+    else
+      ws_store(p, v);
+  };
+  const auto add = [&](double* p, double v) {
+    if (L::JLDS)
+      __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else
+      unsafeAtomicAdd(p, v);
+  };
+  const auto jsync = [&]() {
+    if (!L::JLDS) __threadfence();
+    wave_sync();
+  };
   double y[C::EPL], w1[SPL], w0[SPL] = {}, hk[SPL], sce[SPX], rw[RPL];
   const double Tv = sh[NS];
 #pragma unroll
-  for (int e = 0; e < C::EPL; ++e) y[e] = e * G + g < n ? sh[e * G + g] : 0.0;
-#pragma unroll 1
-  for (int i = g; i < C::JSQ + NQ * NS; i += G) ws_store(J + i, 0.0);
+  for (int e = 0; e < C::EPL; ++e) y[e] = e * WD + g < n ? sh[e * WD + g] : 0.0;
   wave_sync();
   // the rates at T + 1e-2 K (temperature column), then at T
 #pragma unroll 1
@@ -706,9 +744,9 @@ __device__ __noinline__ void group_qss_jacobian(double* sh, double* J, const boo
     }
     C::production(pk, sh, g, Tq, 1.0 / Tq, y, 1.0, hk, w0, [&] {
 #pragma unroll
-      for (int e = 0; e < SPX; ++e) sce[e] = e * G + g < NX ? sh[C::S_CA + 2 * (e * G + g)] : 0.0;
+      for (int e = 0; e < SPX; ++e) sce[e] = e * WD + g < NX ? sh[C::S_CA + 2 * (e * WD + g)] : 0.0;
 #pragma unroll
-      for (int e = 0; e < RPL; ++e) rw[e] = e * G + g < NROW ? sh[C::S_B + e * G + g] : 0.0;
+      for (int e = 0; e < RPL; ++e) rw[e] = e * WD + g < NROW ? sh[C::S_B + e * WD + g] : 0.0;
       wave_sync();
     });
   }
@@ -720,7 +758,7 @@ __device__ __noinline__ void group_qss_jacobian(double* sh, double* J, const boo
   double msum = 0.0;
 #pragma unroll
   for (int e = 0; e < SPX; ++e) {
-    const int k = e * G + g;
+    const int k = e * WD + g;
     if (k < NX) {
       double p[7], imw;
       C::coefs(pk, k, Tv, p, imw);
@@ -743,74 +781,76 @@ __device__ __noinline__ void group_qss_jacobian(double* sh, double* J, const boo
   }
 #pragma unroll
   for (int e = 0; e < RPL; ++e)
-    if (e * G + g < NROW) rows[e * G + g] = rw[e];
+    if (e * WD + g < NROW) rows[e * WD + g] = rw[e];
+#pragma unroll 1
+  for (int i = g; i < L::JSTRIDE; i += WD) st(J + i, 0.0);
   const double mixture = Gr::sum(msum);
-  __threadfence();
-  wave_sync();
+  jsync();
   const double* const x = c + NS;
 #pragma unroll 1
-  for (int i = g; i < T::NQR; i += G) {
+  for (int i = g; i < T::NQR; i += WD) {
     double qf, qr;
     TabMech<T>::qss_balance_terms(i, c1, a, b1, x, mixture, Tv, invT, logT, refC, refCinv, qf, qr,
-                                  [&](int idx, double v) { unsafeAtomicAdd(X + idx, v); });
-    ws_store(qq + 2 * i, qf);
-    ws_store(qq + 2 * i + 1, qr);
+                                  [&](int idx, double v) { add(X + idx, v); });
+    const int j = T::qRx_(i);
+    int qR = -1, qP = -1;
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+      const int r = T::rxR_(3 * j + l), p = T::rxP_(3 * j + l);
+      if (r >= NS) qR = r - NS;
+      if (p >= NS) qP = p - NS;
+    }
+    if (T::rxFwdOff_(j)) qR = -1;
+    if (!T::rxRev_(j)) qP = -1;
+#pragma unroll 1
+    for (int l = 0; l < T::MAXNET; ++l) {
+      const int m = T::rxNet_(T::MAXNET * j + l);
+      if (m < 0) break;
+      const double nu = T::rxNu_(T::MAXNET * j + l);
+      if (qR >= 0) add(W + qR * NS + m, nu * qf);
+      if (qP >= 0) add(W + qP * NS + m, -nu * qr);
+    }
   }
 #pragma unroll 1
-  for (int j = g; j < T::NR; j += G)
+  for (int j = g; j < T::NR; j += WD)
     TM::template jac_reaction<0>(
         j, c, gk, hh, mixture, Tv, invT, invT2, logT, refC, refCinv,
         [&](int idx, double v) {
-          if (idx < NS * n) unsafeAtomicAdd(J + idx, v);
+          if (idx < NS * n) add(J + idx, v);
         },
         [&](int, double) {});
-  __threadfence();
-  wave_sync();
-  // d x / d c = -A^-1 d(balance)/d c and J += (d wdot / d x)(d x / d c), a column a lane
+  jsync();
+  // d x / d c = -A^-1 d(balance)/d c, a column a lane
 #pragma unroll 1
-  for (int k = g; k < NS; k += G) {
+  for (int k = g; k < NS; k += WD) {
     double A[T::NSLOT], col[NQ];
 #pragma unroll
     for (int i = 0; i < T::NSLOT; ++i) A[i] = rows[i];
 #pragma unroll
-    for (int i = 0; i < NQ; ++i) col[i] = -ws_load(X + i * NS + k);
+    for (int i = 0; i < NQ; ++i) col[i] = -ld(X + i * NS + k);
     T::qss_eliminate(A, col);
 #pragma unroll
-    for (int i = 0; i < NQ; ++i) ws_store(X + i * NS + k, col[i]);
-    double* const Jk = J + k * n;
-#pragma unroll 2
-    for (int i = 0; i < T::NQR; ++i) {
-      const int j = T::qRx_(i);
-      int qR = -1, qP = -1;
-#pragma unroll
-      for (int l = 0; l < 3; ++l) {
-        const int r = T::rxR_(3 * j + l), p = T::rxP_(3 * j + l);
-        if (r >= NS) qR = r - NS;
-        if (p >= NS) qP = p - NS;
-      }
-      if (T::rxFwdOff_(j)) qR = -1;
-      if (!T::rxRev_(j)) qP = -1;
-      double d = 0.0;
-      if (qR >= 0) d += ws_load(qq + 2 * i) * ws_load(X + qR * NS + k);
-      if (qP >= 0) d -= ws_load(qq + 2 * i + 1) * ws_load(X + qP * NS + k);
-#pragma unroll 1
-      for (int l = 0; l < T::MAXNET; ++l) {
-        const int m = T::rxNet_(T::MAXNET * j + l);
-        if (m < 0) break;
-        unsafeAtomicAdd(Jk + m, T::rxNu_(T::MAXNET * j + l) * d);
-      }
-    }
+    for (int i = 0; i < NQ; ++i) st(X + i * NS + k, col[i]);
   }
-  __threadfence();
-  wave_sync();
+  jsync();
+  // J += (d wdot / d x)(d x / d c)
+#pragma unroll 1
+  for (int t = g; t < NS * NS; t += WD) {
+    const int k = t / NS, m = t - k * NS;
+    double d = ld(J + k * n + m);
+#pragma unroll 5
+    for (int i = 0; i < NQ; ++i) d += ld(W + i * NS + m) * ld(X + i * NS + k);
+    st(J + k * n + m, d);
+  }
+  jsync();
   // temperature column and row
   double s_cm = 0.0, s_dcm = 0.0, s_eh = 0.0, s_deh = 0.0;
 #pragma unroll
   for (int e = 0; e < SPL; ++e) {
-    const int k = e * G + g;
+    const int k = e * WD + g;
     if (k < NS) {
       const double dT = (w1[e] - w0[e]) / 1.0e-2;
-      ws_store(J + NS * n + k, dT);
+      st(J + NS * n + k, dT);
       s_cm += cR[e] * sce[e];
       s_dcm += dcR[e] * sce[e];
       s_eh += eh[e] * w0[e];
@@ -822,17 +862,16 @@ __device__ __noinline__ void group_qss_jacobian(double* sh, double* J, const boo
   const double cmixinv = 1.0 / cmix;
   const double tmp1 = ehmix * cmixinv, tmp3 = cmixinv * Tv, tmp2 = tmp1 * tmp3;
 #pragma unroll 1
-  for (int k = g, e = 0; k < NS; k += G, ++e) {
+  for (int k = g, e = 0; k < NS; k += WD, ++e) {
     double d = 0.0, ck = 0.0;
 #pragma unroll 8
-    for (int m = 0; m < NS; ++m) d += (eform ? hh[m] - 1.0 : hh[m]) * ws_load(J + k * n + m);
+    for (int m = 0; m < NS; ++m) d += (eform ? hh[m] - 1.0 : hh[m]) * ld(J + k * n + m);
 #pragma unroll
     for (int u = 0; u < SPL; ++u) ck = u == e ? cR[u] : ck;
-    ws_store(J + k * n + NS, tmp2 * ck - tmp3 * d);
+    st(J + k * n + NS, tmp2 * ck - tmp3 * d);
   }
-  if (g == 0) ws_store(J + n * n - 1, -tmp1 + tmp2 * dcmixdT - tmp3 * dehmixdT);
-  __threadfence();
-  wave_sync();
+  if (g == 0) st(J + n * n - 1, -tmp1 + tmp2 * dcmixdT - tmp3 * dehmixdT);
+  jsync();
 }
 
 // ------------------------------------------- group Newton-matrix inverse --
@@ -1034,7 +1073,7 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
   LU_T* const prow = reinterpret_cast<LU_T*>(sw + NP);
   constexpr long long GROWS = (long long)EPL * n * G;
   constexpr long long GSTRIDE = (GROWS * (long long)sizeof(LU_T) + 15) / 16 * 16 / (long long)sizeof(LU_T);
-  double* const Jw = C::JLDS ? wa + C::J_AT : P.ws + wid * group_ws_doubles<T, G, LU_T>();
+  double* const Jw = C::JLDS && !C::JOWN ? wa + C::J_AT : P.ws + wid * group_ws_doubles<T, G, LU_T>();
   // the groups' Jacobian rows: element (e, j) of lane g at [(e * n + j) * G + g]
   LU_T* const rows = reinterpret_cast<LU_T*>(P.ws + wid * group_ws_doubles<T, G, LU_T>() + C::JSPACE);
   const LU_T* const jrow = rows + gi * GSTRIDE + g;
@@ -1183,27 +1222,20 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
   // the loop runs until every group of the wave has drained the queue: all 64
   // lanes take part in the Jacobians
   while (__ballot(active)) {
-    // ---- Jacobian requests, one cell at a time by the whole wave
+    // ---- Jacobian requests: every group its own cell's, or the whole wave one
+    // cell's after the other's (GroupLayout)
     unsigned long long jreq = __ballot(active && need_jac != 0 && g == 0);
-    if constexpr (T::NQ > 0) {
+    if constexpr (C::JOWN) {
       if (__builtin_expect(jreq != 0, 0)) {
-        const bool mine = active && need_jac != 0;
-        double* const Jq = Jw + (long long)gi * C::JSTRIDE;
-        if (mine) {
+        wave_sync();
+        if (active && need_jac != 0) {
+          double* const Jq = C::JLDS ? sh + C::J_AT : Jw + (long long)gi * C::JSTRIDE;
 #pragma unroll
           for (int e = 0; e < EPL; ++e)
             if (valid[e]) sh[e * G + g] = need_jac == 1 ? D[0][e] : ypred[e];
-        }
-        wave_sync();
-        if (mine) group_qss_jacobian<T, G>(sh, Jq, eform);
-        wave_sync();
-        if (mine) {
-          LU_T* const out = rows + gi * GSTRIDE;
-#pragma unroll 2
-          for (int t = g; t < n * n; t += G) {
-            const int j = t / n, i = t - j * n;
-            out[((i / G) * n + j) * G + i % G] = (LU_T)C::jac_elem(pk, Jq, i, j);
-          }
+          wave_sync();
+          C::template cell_jacobian<G>(pk, sh, Jq, eform);
+          C::template jac_rows<G>(pk, Jq, rows + gi * GSTRIDE);
           need_jac = 0;
           njac++;
         }
@@ -1212,7 +1244,7 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
         jreq = 0;
       }
     }
-    while (__builtin_expect(T::NQ == 0 && jreq != 0, 0)) {
+    while (__builtin_expect(!C::JOWN && jreq != 0, 0)) {
       const int lead = __ffsll((long long)jreq) - 1, s = lead / G;
       jreq &= jreq - 1;
       wave_sync();
@@ -1222,11 +1254,8 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
           if (valid[e]) wa[e * G + g] = need_jac == 1 ? D[0][e] : ypred[e];
       }
       wave_sync();
-      if (eform)
-        C::template jacobian<0, 64>(pk, wa, Jw);
-      else
-        C::template jacobian<1, 64>(pk, wa, Jw);
-      C::template jac_rows<LU_T>(pk, Jw, rows + s * GSTRIDE);
+      C::template cell_jacobian<64>(pk, wa, Jw, eform);
+      C::template jac_rows<64>(pk, Jw, rows + s * GSTRIDE);
       __threadfence_block();
       wave_sync();
       if (gi == s) {

@@ -101,11 +101,11 @@ group_rk64_kernel(ReactParamsDev P, GroupIO io, double dt, int ncells, CellStats
   using Gr = Grp<G>;
   using Cell = GroupCell<T, G, BOX>;
   constexpr int EPL = C::EPL, SPL = C::SPL, NG = 64 / G;
-  __shared__ __attribute__((aligned(16))) double lds[GROUP_WAVES * NG * C::AREA];
+  __shared__ __attribute__((aligned(16))) double lds[GROUP_WAVES * NG * C::L::AREA_RHS];
   const auto& pk = load_pack<T>();
   const int g = Gr::lane();
   const int gb = (int)threadIdx.x / G;  // group of the block
-  double* const sh = lds + gb * C::AREA;
+  double* const sh = lds + gb * C::L::AREA_RHS;
   const bool eform = P.reactor_type == E_REACTOR;
   const RK64ParamsDev& p = P.rk64;
   const double dt_min = dt / (double)p.nsub_max, dt_max = dt / (double)p.nsub_min;
@@ -403,7 +403,7 @@ struct RowSolve {
 template <class T>
 constexpr int group_fixed_area() {
   using L = GroupLayout<T, 16>;
-  return ((L::cmax(L::cmax(RowSolve<L::n, L::EPL>::SIZE, L::AREA), L::J_AT + L::n * L::n) + 3) / 8) * 8 + 4;
+  return L::padded(L::cmax(L::cmax(RowSolve<L::n, L::EPL>::SIZE, L::S_RAW), L::JLEN));
 }
 template <class M>
 constexpr bool group_fixed_fits() {
@@ -424,7 +424,7 @@ group_bdf_fixed_kernel(ReactParamsDev P, GroupIO io, double dt_react, int ncells
   constexpr int n = C::n, EPL = C::EPL, SPL = C::SPL;
   using RS = RowSolve<n, EPL>;
   constexpr int RSIZE = group_fixed_area<T>();
-  static_assert(C::JLDS, "the Jacobian of these mechanisms is in LDS");
+  static_assert(C::JLDS && C::NQ == 0, "the Jacobian of these mechanisms is in LDS");
   __shared__ __attribute__((aligned(16))) double lds[GROUP_WAVES * NG * RSIZE];
   const auto& pk = load_pack<T>();
   const int g = Gr::lane();

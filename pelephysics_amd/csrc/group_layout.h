@@ -31,29 +31,49 @@ struct GroupLayout {
   static constexpr int S_Q = (cmax(cmax(3 * (NX + 1), NCH), 2 * (NX + 1) + NROW) + 1) & ~1;
   static constexpr int NRATE = NQ > 0 ? 2 * NR + 1 : NR + 1;  // QSS: forward and reverse rates apart
   static constexpr int S_RAW = S_Q + cmax(NRATE, 3 * NP);
-  static constexpr int AREA = ((S_RAW + 3) / 8) * 8 + 4;
-  // The wave's Jacobian area overlays its groups' areas: 5 species vectors and,
-  // where n is small enough, the n x n accumulator.
-  // (QSS mechanisms: each group works on its own cell's Jacobian, in the
-  // workspace, with JVEC doubles of its area.)
-  static constexpr bool JLDS = n <= 32 && NQ == 0;
-  static constexpr int J_AT = (5 * NP + 1) & ~1;
-  static constexpr int JVEC = NQ > 0 ? 6 * NX + NROW : 0;
-  // Jacobian accumulators in the workspace (doubles): n x n (JSQ) of the wave,
-  // or of each group with the QSS terms after it (JSTRIDE); of a wave
+  static constexpr int padded(int a) { return ((a + 3) / 8) * 8 + 4; }
+  static constexpr int AREA_RHS = padded(S_RAW);  // of a kernel without Jacobians
+
+  // A Jacobian in LDS (doubles): its species vectors (QSS mechanisms: with the
+  // balances), then the n x n accumulator (JSQ), for QSS mechanisms with the
+  // derivatives of the balances and of the rates (NQ x NS each) after it.
+  static constexpr int JVEC = NQ > 0 ? 6 * NX + NROW : 5 * NP;
+  static constexpr int J_AT = (JVEC + 1) & ~1;
   static constexpr int JSQ = (n * n + 1) & ~1;
-  static constexpr int JSTRIDE = NQ > 0 ? (JSQ + NQ * NS + 2 * T::NQR + 1) & ~1 : JSQ;
-  static constexpr int JSPACE = NQ > 0 ? NG * JSTRIDE : JSTRIDE;
-  static constexpr int WAREA = (cmax(NG * AREA, J_AT + (JLDS ? n * n : 0)) + 3) & ~3;
+  static constexpr int JSTRIDE = (JSQ + 2 * NQ * NS + 1) & ~1;
+  static constexpr int JLEN = J_AT + JSTRIDE;
   // vectors of the step that stay in LDS (group_bdf_kernel), per wave
   static constexpr int LVEC = 4 * 64 * EPL;
+  static constexpr int own_area() { return padded(cmax(S_RAW, JLEN)); }
+  static constexpr int wave_area() { return (cmax(NG * AREA_RHS, JLEN) + 3) & ~3; }
+  static constexpr long long bytes(int area) {
+    return (long long)sizeof(typename T::Packed) + 8LL * GROUP_WAVES * (area + LVEC);
+  }
+  // Who works on the Jacobians of a wave's cells, and where.  Every group on its
+  // own cell's (JOWN), in its own area: the groups of a wave ask at the same time
+  // when their cells start, which is most of a call of few steps per cell.  Or the
+  // whole wave on one cell's after the other's, over all its groups' areas.  In LDS
+  // (JLDS) where two blocks fit a compute unit, i.e. two waves per SIMD; else in
+  // the workspace, by the groups for QSS mechanisms and by the wave for the others.
+  // Without QSS species a group's own takes NR / G rounds of reactions, the wave NG
+  // times NR / 64: its own where that is at most half.  Measured, calls of one step
+  // per cell: LiDryer 262144 cells, 8 lanes, one cell after the other 5.7 ms, each
+  // its own 1.6; CH4_lean_qss 262144 cells and LuEthylene_qss 65536, by the group in
+  // the workspace 34.3 and 37.6 ms, in LDS by the group and by the wave 5.4 and 6.3.
+  static constexpr bool two_blocks(int area) { return bytes(area) <= LDS_BYTES / 2; }
+  static constexpr bool own_fits() { return n <= 32 && two_blocks(NG * own_area()); }
+  static constexpr bool wave_fits() { return n <= 32 && (NQ == 0 || two_blocks(wave_area())); }
+  static constexpr bool JOWN = NQ > 0 ? own_fits() || !wave_fits()
+                                      : own_fits() && 2 * ((NR + G - 1) / G) <= NG * ((NR + 63) / 64);
+  static constexpr bool JLDS = JOWN ? own_fits() : wave_fits();
+  static constexpr int AREA = JOWN && JLDS ? own_area() : AREA_RHS;
+  static constexpr int WAREA = JOWN || !JLDS ? (cmax(NG * AREA, JOWN ? 0 : J_AT) + 3) & ~3 : wave_area();
+  // Jacobian accumulators in the workspace (doubles) of a wave
+  static constexpr int JSPACE = NQ > 0 ? NG * JSTRIDE : JSTRIDE;
 
   // LDS of a block of the largest group kernel with G lanes per cell (the
   // adaptive BDF's; ReactorRK64's has the tables and the areas only)
-  static constexpr long long lds_bytes() {
-    return (long long)sizeof(typename T::Packed) + 8LL * GROUP_WAVES * (WAREA + LVEC);
-  }
-  static constexpr bool fits() { return JVEC <= AREA && lds_bytes() <= LDS_BYTES; }
+  static constexpr bool fits() { return (!JOWN || JVEC <= AREA) && bytes(WAREA) <= LDS_BYTES; }
 };
 
 }  // namespace ppc

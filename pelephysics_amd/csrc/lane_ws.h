@@ -135,7 +135,7 @@ constexpr long long group_wave_doubles() {
   constexpr long long n = M::NEQ, acc = n * n + 1, groups = 64 / G;
   constexpr long long rows = groups * ((n + G - 1) / G * n * G + 1);
   if constexpr (has_qss<M>::value)
-    return groups * (acc + M::NQ * (n - 1) + 2 * M::NR + 1) + rows;
+    return groups * (acc + 2 * M::NQ * (n - 1) + 1) + rows;
   else
     return acc + rows;
 }
