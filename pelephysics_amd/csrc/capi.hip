@@ -416,15 +416,23 @@ constexpr long long kWsMaxBytes = 32LL << 30;
 
 // Cells per wave of the group kernels where the caller leaves the choice
 // (batched_cells_per_wave = 0): a lane per equation, rounded up to 8, 16, 32 or
-// 64 lanes per cell, while that fills the chip no more than kGroupRounds times
-// over; half as many lanes, two equations in each, above it.  A wide group ends
-// a cell's trip sooner, which is what a call of few cells waits for; a narrow
-// one has less of its lanes idle in the exchanges and reductions, which is what
-// a call of many cells waits for.  Measured (one call of 1e-5 s at rtol 1e-10,
-// cells in index order, 32 / 16 lanes): drm19 2898 cells 5.9 / 8.2 ms, 262144
-// cells 95 / 79 ms.  Above 32 equations the inverse's two rows per lane leave
-// one wave per SIMD (dodecane_lu, 10000 cells: 17.5 ms at 64 lanes, 27.3 at 32).
-constexpr long long kGroupRounds = 8;
+// 64 lanes per cell, up to kWideCells cells per compute unit; half as many lanes,
+// two equations in each, from there on.  A wide group ends a cell's trip sooner,
+// which is what a call of few cells waits for; a narrow one has less of its lanes
+// idle in the exchanges and reductions, which is what a call of many cells waits
+// for.  Measured (ms, wide / narrow; long: 1e-5 s at rtol 1e-10, short: 1e-8 s at
+// rtol 1e-6, one step per cell):
+//   drm19, 32 / 16 lanes: 8192 cells long 6.0 / 8.4, short 0.33 / 0.37;
+//     16384 6.2 / 8.9, 0.54 / 0.50; 32768 11.1 / 9.7, 0.98 / 0.86; 65536 22.6 / 16.8,
+//     1.83 / 1.58
+//   LiDryer, 16 / 8 lanes: 4096 cells long 2.36 / 3.05, short 0.100 / 0.106;
+//     16384 3.30 / 3.44, 0.182 / 0.149; 32768 6.14 / 4.53, 0.286 / 0.226; 65536
+//     11.8 / 8.6, 0.49 / 0.39; ReactorCvode, 1e-5 s (few cells take most of the
+//     steps), 32768 cells 1.69 / 2.12, 65536 3.26 / 2.79
+// The line lies where no measured call is slower on the narrow side.
+// Above 32 equations the inverse's two rows per lane leave one wave per SIMD
+// (dodecane_lu, 10000 cells: 17.5 ms at 64 lanes, 27.3 at 32).
+constexpr long long kWideCells = 256;
 
 int auto_cells_per_wave(const pp_chem* h, long long ncells) {
   const int n = h->L->ns + 1;
@@ -434,8 +442,7 @@ int auto_cells_per_wave(const pp_chem* h, long long ncells) {
   // (narrow groups of large tables do not fit the LDS: the next size there is)
   while (cpw > 1 && h->GL->group_ws_rows(cpw) <= 0) cpw /= 2;
   while (cpw < 8 && h->GL->group_ws_rows(cpw) <= 0) cpw *= 2;
-  const long long waves = 8LL * std::max(h->ncu, 1);
-  if (n <= 32 && h->GL->group_ws_rows(2 * cpw) > 0 && ncells >= kGroupRounds * waves * 2 * cpw) cpw *= 2;
+  if (n <= 32 && h->GL->group_ws_rows(2 * cpw) > 0 && ncells >= kWideCells * std::max(h->ncu, 1)) cpw *= 2;
   return cpw;
 }
 

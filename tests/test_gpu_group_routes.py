@@ -99,6 +99,26 @@ def test_rk64_on_both_sides_of_the_lane_kernel(models):
     _compare_y(m.n_species + 1, out[0][0], out[1][0])
 
 
+@pytest.mark.parametrize("mech", ["drm19", "LiDryer"])
+def test_adaptive_on_both_sides_of_the_narrow_group(models, oracles, mech):
+    """The largest call with a lane per equation and the next, with half as many
+    lanes: both meet the criterion, and every copy of a cell is alike in each."""
+    torch = _torch()
+    ncu = torch.cuda.get_device_properties(0).multi_processor_count
+    m, st, ysrc, esrc = _cells(models, mech, 64)
+    tol = dict(rtol=1e-12, atol=1e-18) if mech == "LiDryer" else dict(rtol=1e-10, atol=1e-16)
+    p = oracle.adapt_params(rtol=1e-13, atol=1e-20)
+    _, oy, _, _ = _oracle_1d(oracles[mech], "adaptive", st, ysrc, esrc, 1e-6, params=p)
+    for n in (256 * ncu - 1, 256 * ncu):
+        s = W.subsample(st, np.arange(n) % st.ncells)
+        _, y, _, R = _run_1d(torch, mech, "ReactorBDFAdaptiveMixed", s, np.zeros((n, m.n_species)), np.zeros(n), 1e-6,
+                             **tol)
+        assert R.stats()["nfailed"] == 0
+        y = y.reshape(n, -1)
+        assert (y == y[np.arange(n) % st.ncells]).all()
+        _compare_y(m.n_species + 1, y[:st.ncells].reshape(-1), oy)
+
+
 def test_statistics_and_cost_order_of_a_large_call(models):
     """More cells than the bookkeeping kernels have threads, an odd number of
     them: the statistics are those of the per-cell counts, and the second call,
