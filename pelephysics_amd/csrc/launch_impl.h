@@ -242,18 +242,20 @@ hipError_t launch_flatten(const FlatArgs& a, int unflatten, hipStream_t s) {
 // out[c*NR + j] = q_j (mol/m^3/s), written in place in the output array.
 //
 // One kernel per function: with the four in one, all took the Jacobian's 512
-// registers, one wave per SIMD (drm19 rates: 203, two).  The rates' flat arrays
-// pass through LDS in whole lines (a row is 65 cells: no bank conflicts either
-// way) where a wave's cells take little of it.  Bound by the FP64 vector issue:
-// drm19 is 7800 vector instructions per wave, 57 us at the full rate for 262144
-// cells; a call of them 99.1 -> 86.6 us.
-template <class M, int WHAT>
+// registers, one wave per SIMD (drm19 rates: 203, two).  WHOLE: the rates' flat
+// arrays pass through LDS in whole lines (a row is 65 cells: no bank conflicts
+// either way), for calls that give every SIMD a wave, where a wave's cells take
+// little LDS; below that a call waits for one wave's latency, and the way through
+// LDS is part of it.  Bound by the FP64 vector issue: drm19 is 7800 vector
+// instructions per wave, 57 us at the full rate for 262144 cells; a call of them
+// 99.1 -> 86.6 us (65536 cells 43.7 -> 43.3; 8192 cells 36.7 -> 39.2 through LDS).
+template <class M, int WHAT, bool WHOLE>
 __global__ void __launch_bounds__(64) mech_eval_kernel(const double* __restrict__ sc, const double* __restrict__ T,
                                                        int ncells, double* out) {
   constexpr int NS = M::NS;
   const int l = threadIdx.x, c0 = blockIdx.x * 64, nc = min(64, ncells - c0);
   double s[NS];
-  if constexpr (WHAT == 0 && NS <= 32) {
+  if constexpr (WHOLE) {
     __shared__ double row[NS * 65];
     const double* const from = sc + (long long)c0 * NS;
     for (int i = l; i < nc * NS; i += 64) row[i % NS * 65 + i / NS] = from[i];
@@ -288,10 +290,16 @@ template <class M>
 hipError_t launch_mech_eval(int what, const double* sc, const double* T, int ncells, double* out, hipStream_t s) {
   if (what < 0 || what > 3) return hipErrorInvalidValue;
   if (ncells <= 0) return hipSuccess;
-  auto k = what == 0   ? mech_eval_kernel<M, 0>
-           : what == 1 ? mech_eval_kernel<M, 1>
-           : what == 2 ? mech_eval_kernel<M, 2>
-                       : mech_eval_kernel<M, 3>;
+  int dev = 0, ncu = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  if (e != hipSuccess) return e;
+  auto k = what == 0   ? mech_eval_kernel<M, 0, false>
+           : what == 1 ? mech_eval_kernel<M, 1, false>
+           : what == 2 ? mech_eval_kernel<M, 2, false>
+                       : mech_eval_kernel<M, 3, false>;
+  if constexpr (M::NS <= 32)
+    if (what == 0 && ncells >= 256LL * ncu) k = mech_eval_kernel<M, 0, true>;
   hipLaunchKernelGGL(k, dim3((ncells + 63) / 64), dim3(64), 0, s, sc, T, ncells, out);
   return hipGetLastError();
 }

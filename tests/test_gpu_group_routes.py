@@ -163,3 +163,11 @@ def test_production_rate_counts(models, oracles, mech):
         assert np.abs(w[c].cpu().numpy() - wo).max() <= 1e-10 * np.abs(wo).max(), c
     for n in (1, 63, 64, 65, 129):
         assert torch.equal(R.production_rate(sc[:n].contiguous(), T[:n].contiguous()), w[:n]), n
+    # calls that fill the chip pass their arrays through LDS: every copy of a cell
+    # alike, and the rates above to the same tolerance
+    ncu = torch.cuda.get_device_properties(0).multi_processor_count
+    for n in (256 * ncu - 1, 256 * ncu, 256 * ncu + 1):
+        i = torch.arange(n, device="cuda") % 130
+        wn = R.production_rate(sc[i].contiguous(), T[i].contiguous())
+        assert torch.equal(wn, wn[:130][i]), n
+        assert ((wn[:130] - w).abs().amax(1) <= 1e-10 * w.abs().amax(1)).all(), n
