@@ -31,7 +31,7 @@ GRID = 64
 DT = 1e-5
 # Tolerances of the adaptive BDF: the config's rtol = 1e-8 with atol = 1e-10 on
 # rhoY leaves minor species above the 1e-6 relative error criterion; the
-# absolute tolerance is lowered until every cell meets it (see DESIGN.md).
+# absolute tolerance is lowered until every cell meets it.
 RTOL, ATOL = 1e-10, 1e-16
 P_FP64 = 78.6  # TFLOP/s, MI355X FP64 (vector and matrix)
 P_FP32 = 157.3  # TFLOP/s, MI355X FP32
@@ -41,8 +41,9 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-TUNABLES = ("batched_waves_per_cu", "batched_lu_batch", "batched_lu_wait", "batched_box_direct",
-            "batched_waves_per_simd", "batched_cells_per_wave")
+# launch parameters of a tuning entry
+TUNABLES = ("batched_waves_per_cu", "batched_lu_batch", "batched_lu_wait", "batched_waves_per_simd",
+            "batched_cells_per_wave")
 
 
 def run_gpu(ident, st, m, steps, warmup, rtol, atol, mech=MECH, launch=None, replay_steps=0):
@@ -135,7 +136,7 @@ def measured_traffic(ident, kernels, launch):
     except (OSError, ValueError):
         return None
     e = t.get(ident)
-    if e is None or e.get("kernels") != kernels or e.get("launch", {k: 0 for k in TUNABLES}) != launch:
+    if e is None or e.get("kernels") != kernels or e.get("launch", {}) != launch:
         return None
     return float(e["bytes_per_launch"])
 
@@ -320,10 +321,10 @@ def main():
             from pelephysics_amd.autotune import lookup
             e = lookup(MECH, integrator, "box")
             if e:
-                return (e["kernels"], {k: e.get(k, 0) for k in TUNABLES},
+                return (e["kernels"], {k: e[k] for k in TUNABLES if k in e},
                         {k: e[k] for k in e if k != "candidates"})
-            return MECH, {k: 0 for k in TUNABLES}, None
-        return {"unrolled": MECH, "table": MECH + "_table"}[kind], {k: 0 for k in TUNABLES}, None
+            return MECH, {}, None
+        return {"unrolled": MECH, "table": MECH + "_table"}[kind], {}, None
 
     kern, launch, tuning = choose(a.impl, ident)
     pkern, plaunch, ptuning = choose(a.plain_impl, "ReactorBDFAdaptive")

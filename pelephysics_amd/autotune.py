@@ -14,13 +14,14 @@ keeps the fastest:
   choice by mechanism and number of cells (0), or a group of 8, 16, 32 or 64
   lanes per cell (8, 4, 2, 1 cells per wave; the sizes a mechanism's kernels
   are built for);
-* batched_waves_per_cu (8, 6, 4 or 3 persistent waves per compute unit) and
-  batched_lu_batch / batched_lu_wait (how many waiting cells, or how many trips
-  of waiting, make a wave factor its cells' Newton matrices together): read
-  where batched_cells_per_wave names a size, as is the launch shape;
-* batched_waves_per_simd and batched_box_direct (batched forms): accepted, the
-  kernels have one build and one box route; candidates that differ in them
-  only, or in what is not read, time the same launch.
+* with a named size, batched_waves_per_cu (every resident wave, or 4 per
+  compute unit) and batched_lu_batch / batched_lu_wait (how many waiting cells,
+  or how many trips of waiting, make a wave factor its cells' Newton matrices
+  together);
+* batched_waves_per_simd (the plain adaptive BDF: the compiler's choice, or a
+  build held to 2 or 4 waves per SIMD).
+
+An entry holds the parameters that its launch reads, and no others.
 
 Each candidate runs `calls` calls on the same cells and arrays; its time is
 the kernel time of the last one (the queue in the cost order of the call
@@ -50,9 +51,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 # mechanisms compiled from their tables only, under their plain names
 TABLE_ONLY = ("dodecane_lu", "heptane_lu_88sk")
 BATCHED = ("ReactorBDFAdaptiveMixed", "ReactorBDFBatchedFP64")
-OCCUPANCY = ((2, 8), (2, 6), (2, 4), (1, 4), (1, 3))  # (waves per SIMD, waves per CU)
 PLAIN_OCCUPANCY = (0, 2, 4)  # plain adaptive BDF builds: compiler choice, 2 or 4 waves per SIMD
-LU_SERVICE = ((16, 4), (64, 8), (64, 32))
 GROUPS = (8, 4, 2, 1)  # cells per wave of the group kernel
 GROUP_WAVES = (0, 4)  # persistent waves per CU of the group kernel (0: every resident wave)
 GROUP_LU = ((1, 1), (64, 8), (64, 32))
@@ -90,20 +89,17 @@ def candidates(mech: str, integrator: str, form: str = "1d") -> list:
         from .mechgen.__main__ import load
         fits = load(mech).n_species + 1 <= 32
         occs = PLAIN_OCCUPANCY if integrator == "ReactorBDFAdaptive" and fits else (0,)
-        return [{"kernels": k, "batched_waves_per_simd": o, "batched_waves_per_cu": 0, "batched_lu_batch": 0,
-                 "batched_lu_wait": 0, "batched_box_direct": 0} for k in impls for o in occs]
-    routes = (0, 1) if form == "box" else (0,)
-    lane = [{"kernels": k, "batched_waves_per_simd": o, "batched_waves_per_cu": w, "batched_lu_batch": b,
-             "batched_lu_wait": t, "batched_box_direct": r, "batched_cells_per_wave": 0}
-            for k in impls for o, w in OCCUPANCY for b, t in LU_SERVICE for r in routes
-            if not (o == 1 and r == 1)]  # the box kernel is built at 2 waves per SIMD only
+        return [{"kernels": k, "batched_waves_per_simd": o} for k in impls for o in occs]
+    # the library's choice of the group size, with each implementation's own
+    # kernels around it
+    auto = [{"kernels": k, "batched_cells_per_wave": 0} for k in impls]
     # group kernels: table-driven implementations only (a size a mechanism is
     # not built for is rejected at init and skipped)
     tables = [k for k in impls if k.endswith("_table") or k in TABLE_ONLY]
-    group = [{"kernels": k, "batched_waves_per_simd": 0, "batched_waves_per_cu": w, "batched_lu_batch": b,
-              "batched_lu_wait": t, "batched_box_direct": 0, "batched_cells_per_wave": g}
+    group = [{"kernels": k, "batched_cells_per_wave": g, "batched_waves_per_cu": w, "batched_lu_batch": b,
+              "batched_lu_wait": t}
              for k in tables for g in GROUPS for w in GROUP_WAVES for b, t in GROUP_LU]
-    return lane + group
+    return auto + group
 
 
 def _time(cand: dict, integrator: str, form: str, st, m, dt: float, rtol: float, atol: float,

@@ -138,33 +138,24 @@ def test_workspace_smaller_than_grid(models, ident):
     assert np.array_equal(y_full, y_one) and np.array_equal(rX_full, rX_one)
 
 
+@pytest.mark.parametrize("cpw", [2, 1])
 @pytest.mark.parametrize("mech", ["dodecane_lu", "heptane_lu_88sk"])
-def test_large_one_wave_build_tuned_service(models, oracles, mech):
-    """The batched FP32-LU kernel built at 1 wave per SIMD with the tuned
-    Jacobian/LU service (64 lanes or 8 trips) against the oracle."""
+def test_large_lu_service_parameters_bitwise(models, oracles, mech, cpw):
+    """Groups of 32 and 64 lanes: the Jacobian/LU service parameters (every request
+    served at once; all groups or 8 trips; the default) and fewer resident waves
+    leave states and per-cell step counts bitwise unchanged, and the state meets the
+    criterion against the oracle."""
     torch = _torch()
     m, st, ysrc, esrc = _case(models, mech)
-    ret, y, rX, R = _run_1d(torch, mech, "ReactorBDFAdaptiveMixed", st, ysrc, esrc, 1e-5, rtol=1e-10,
-                            atol=1e-16, batched_waves_per_simd=1, batched_lu_batch=64, batched_lu_wait=8)
-    assert R.stats()["nfailed"] == 0
-    p = oracle.adapt_params(rtol=1e-13, atol=1e-20)
-    _, oy, orX, _ = _oracle_1d(oracles[mech], "adaptive", st, ysrc, esrc, 1e-5, params=p)
-    _compare_y(m.n_species + 1, y, oy)
-
-
-def test_large_lu_service_parameters_bitwise(models):
-    """With the matrices in the workspace too, the Jacobian/LU service
-    parameters (every request served at once; 16 lanes or 4 trips; the default
-    64 lanes or 32 trips) leave states and per-cell step counts bitwise
-    unchanged."""
-    torch = _torch()
-    mech = "dodecane_lu"
-    m, st, ysrc, esrc = _case(models, mech, ncells=128)
     runs = []
-    for b, t in ((1, 1), (16, 4), (0, 0)):
+    for b, t, w in ((1, 1, 0), (64, 8, 0), (0, 0, 0), (64, 1, 1)):
         _, y, rX, R = _run_1d(torch, mech, "ReactorBDFAdaptiveMixed", st, ysrc, esrc, 1e-5, rtol=1e-10,
-                              atol=1e-16, batched_lu_batch=b, batched_lu_wait=t)
+                              atol=1e-16, batched_cells_per_wave=cpw, batched_lu_batch=b, batched_lu_wait=t,
+                              batched_waves_per_cu=w)
         assert R.stats()["nfailed"] == 0
         runs.append((y, rX, R.cell_steps(st.ncells)))
     for y, rX, fc in runs[1:]:
         assert np.array_equal(y, runs[0][0]) and np.array_equal(rX, runs[0][1]) and np.array_equal(fc, runs[0][2])
+    p = oracle.adapt_params(rtol=1e-13, atol=1e-20)
+    _, oy, _, _ = _oracle_1d(oracles[mech], "adaptive", st, ysrc, esrc, 1e-5, params=p)
+    _compare_y(m.n_species + 1, runs[0][0], oy)

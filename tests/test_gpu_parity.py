@@ -461,9 +461,11 @@ def test_full_size_invariants_drm19_64cubed(models, ident):
 
 
 @pytest.mark.parametrize("ident", ["ReactorBDFAdaptiveMixed", "ReactorBDFBatchedFP64"])
-def test_batched_box_routes_agree(models, ident):
-    """The batched box call through flat state and the 1-D kernel (default)
-    and through the box kernel give the same rY, T, rE and FC, bit for bit."""
+def test_batched_box_is_the_flat_call(models, ident):
+    """A batched box call is the 1-D call on the box's flat state with the
+    temperature inversions of the box form around it: the same rhoY, energy and
+    per-cell steps bit for bit from a state whose temperature is at the inversion's
+    end already.  batched_box_direct (0 or 1) changes nothing."""
     torch = _torch()
     from pelephysics_amd.reactor import ReactorBase
     m = models["drm19"]
@@ -475,25 +477,41 @@ def test_batched_box_routes_agree(models, ident):
         return torch.from_numpy(np.ascontiguousarray(a.T.reshape(nc, n, n, n))).to(dev)
 
     rng = np.random.default_rng(3)
-    rYs = soa(1e-3 * rng.standard_normal(st.rY.shape) * st.rY, m.n_species)
-    rEs = soa((1e-3 * rng.standard_normal(st.ncells) * np.abs(st.rE))[:, None], 1)
+    ysrc = 1e-3 * rng.standard_normal(st.rY.shape) * st.rY
+    esrc = 1e-3 * rng.standard_normal(st.ncells) * np.abs(st.rE)
+    rYs, rEs = soa(ysrc, m.n_species), soa(esrc[:, None], 1)
+    # the box form's first inversion, by a call of no duration on the guess
+    T0 = soa(st.T[:, None] + 3.0, 1)
+    R = ReactorBase.create("ReactorRK64")
+    R.init(2, st.ncells, mechanism="drm19")
+    zero = torch.zeros_like(rYs), torch.zeros_like(rEs)
+    R.react(soa(st.rY, m.n_species), zero[0], T0, soa(st.rE[:, None], 1), zero[1], None, 0.0)
     out = []
     for direct in (0, 1):
         R = ReactorBase.create(ident)
         R.init(2, st.ncells, mechanism="drm19", rtol=1e-10, atol=1e-16, batched_box_direct=direct)
-        rY, T, rE = soa(st.rY, m.n_species), soa(st.T[:, None] + 3.0, 1), soa(st.rE[:, None], 1)
+        rY, T, rE = soa(st.rY, m.n_species), T0.clone(), soa(st.rE[:, None], 1)
         FC = torch.zeros_like(T)
         R.react(rY, rYs, T, rE, rEs, FC, 1e-5)
         out.append([x.cpu().numpy() for x in (rY, T, rE, FC)])
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+    y = np.concatenate([st.rY, T0.reshape(-1, 1).cpu().numpy()], axis=1)
+    ty = torch.from_numpy(y.reshape(-1).copy()).to(dev)
+    tx = torch.from_numpy(st.rE.copy()).to(dev)
+    R.react_1d(ty, torch.from_numpy(ysrc.reshape(-1).copy()).to(dev), tx, torch.from_numpy(esrc).to(dev), 1e-5)
+    got = ty.reshape(st.ncells, -1)[:, :-1].T.reshape(m.n_species, n, n, n).cpu().numpy()
+    assert np.array_equal(out[0][0], got)
+    assert np.array_equal(out[0][2].reshape(-1), tx.cpu().numpy())
+    assert np.array_equal(out[0][3].reshape(-1), R.cell_steps(st.ncells))
 
 
 @pytest.mark.parametrize("mech", ["drm19", "drm19_table"])
 @pytest.mark.parametrize("ident", ["ReactorBDFAdaptiveMixed", "ReactorBDFBatchedFP64"])
-def test_batched_one_wave_build(models, oracles, mech, ident):
-    """The batched kernels built at 1 wave per SIMD (batched_waves_per_simd = 1,
-    1-D kernel, also for box calls) against the tight FP64 oracle."""
+def test_batched_parameters_of_other_builds(models, oracles, mech, ident):
+    """batched_waves_per_simd, and without a group size the Jacobian/LU service, are
+    accepted and change nothing (the group kernels have one build); the combination
+    of one wave per SIMD with batched_box_direct stays refused."""
     torch = _torch()
     from pelephysics_amd.reactor import ReactorBase
     m = models["drm19"]
@@ -501,33 +519,37 @@ def test_batched_one_wave_build(models, oracles, mech, ident):
     ysrc, esrc = np.zeros((st.ncells, m.n_species)), np.zeros(st.ncells)
     p = oracle.adapt_params(rtol=1e-13, atol=1e-20)
     _, oy, _, _ = _oracle_1d(oracles["drm19"], "adaptive", st, ysrc, esrc, 1e-5, params=p)
-    ret, y, rX, R = _run_1d(torch, mech, ident, st, ysrc, esrc, 1e-5, rtol=1e-10, atol=1e-16,
-                            batched_waves_per_simd=1, batched_lu_batch=64, batched_lu_wait=8)
-    assert R.stats()["nfailed"] == 0
-    _compare_y(m.n_species + 1, y, oy)
+    runs = []
+    for ode in ({}, dict(batched_waves_per_simd=1, batched_lu_batch=64, batched_lu_wait=8),
+                dict(batched_waves_per_simd=2, batched_waves_per_cu=3)):
+        ret, y, rX, R = _run_1d(torch, mech, ident, st, ysrc, esrc, 1e-5, rtol=1e-10, atol=1e-16, **ode)
+        assert R.stats()["nfailed"] == 0
+        runs.append(y)
+    _compare_y(m.n_species + 1, runs[0], oy)
+    assert np.array_equal(runs[0], runs[1]) and np.array_equal(runs[0], runs[2])
     with pytest.raises(Exception):
         ReactorBase.create(ident).init(2, 4, mechanism=mech, batched_waves_per_simd=1, batched_box_direct=1)
 
 
+@pytest.mark.parametrize("cpw", [8, 4, 2])
 @pytest.mark.parametrize("ident", ["ReactorBDFAdaptiveMixed", "ReactorBDFBatchedFP64"])
-def test_lu_service_parameters_bitwise(models, ident):
-    """The wave-shared Jacobian/LU service only decides when a wave factors
-    its waiting lanes' matrices: every request served at once (lu_batch 1),
-    (16 lanes, 4 trips), (64, 8) and the default (64, 32) give the same
-    states, step counts and per-cell work, bit for bit, on 2-wave and 1-wave
-    builds."""
+def test_lu_service_parameters_bitwise(models, ident, cpw):
+    """The wave's LU service only decides when it factors its waiting groups'
+    matrices: every request served at once (lu_batch 1), 2 groups or 8 trips, all
+    groups or 32 trips, the kernel's default, and fewer resident waves give the same
+    states, step counts and per-cell work, bit for bit, for every group size."""
     torch = _torch()
     m = models["drm19"]
     st = W.subsample(W.drm19_grf(m, 64), np.arange(0, 64 ** 3, 97))
     ysrc, esrc = np.zeros((st.ncells, m.n_species)), np.zeros(st.ncells)
     runs = []
-    for occ in (2, 1):
-        for b, t in ((1, 1), (16, 4), (64, 8), (0, 0)):
-            _, y, rX, R = _run_1d(torch, "drm19", ident, st, ysrc, esrc, 1e-5, rtol=1e-10, atol=1e-16,
-                                  batched_waves_per_simd=occ, batched_lu_batch=b, batched_lu_wait=t)
-            s = R.stats()
-            assert s["nfailed"] == 0
-            runs.append((y, rX, R.cell_steps(st.ncells), [s[k] for k in ("nsteps", "nrhs", "njac", "nlu")]))
+    for b, t, w in ((1, 1, 0), (2, 8, 0), (64, 32, 0), (0, 0, 0), (64, 1, 1)):
+        _, y, rX, R = _run_1d(torch, "drm19_table", ident, st, ysrc, esrc, 1e-5, rtol=1e-10, atol=1e-16,
+                              batched_cells_per_wave=cpw, batched_lu_batch=b, batched_lu_wait=t,
+                              batched_waves_per_cu=w)
+        s = R.stats()
+        assert s["nfailed"] == 0
+        runs.append((y, rX, R.cell_steps(st.ncells), [s[k] for k in ("nsteps", "nrhs", "njac", "nlu")]))
     y0, rX0, fc0, w0 = runs[0]
     for y, rX, fc, w in runs[1:]:
         assert np.array_equal(y, y0) and np.array_equal(rX, rX0)
