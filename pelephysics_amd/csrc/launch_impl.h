@@ -290,16 +290,13 @@ template <class M>
 hipError_t launch_mech_eval(int what, const double* sc, const double* T, int ncells, double* out, hipStream_t s) {
   if (what < 0 || what > 3) return hipErrorInvalidValue;
   if (ncells <= 0) return hipSuccess;
-  int dev = 0, ncu = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-  if (e != hipSuccess) return e;
+  constexpr int fills = 64 * 4 * 256;  // a wave for each of the 4 SIMDs of 256 compute units
   auto k = what == 0   ? mech_eval_kernel<M, 0, false>
            : what == 1 ? mech_eval_kernel<M, 1, false>
            : what == 2 ? mech_eval_kernel<M, 2, false>
                        : mech_eval_kernel<M, 3, false>;
   if constexpr (M::NS <= 32)
-    if (what == 0 && ncells >= 256LL * ncu) k = mech_eval_kernel<M, 0, true>;
+    if (what == 0 && ncells >= fills) k = mech_eval_kernel<M, 0, true>;
   hipLaunchKernelGGL(k, dim3((ncells + 63) / 64), dim3(64), 0, s, sc, T, ncells, out);
   return hipGetLastError();
 }
