@@ -3,7 +3,10 @@
 //
 // * lane g of a group holds equations i = e*G + g for slots e < EPL =
 //   ceil(NEQ / G): its entries of the BDF difference array, the iterate, the
-//   error weights and rows i of the inverted Newton matrix, all in registers;
+//   error weights and rows i of the inverted Newton matrix, in registers as far
+//   as 256 go (four vectors in LDS; spilled with an FP32 inverse: drm19 74 at 32
+//   lanes and 132 at 16, LiDryer 64 at 8, LuEthylene_qss 194, dodecane_lu 287,
+//   heptane_lu_88sk 783, which has two rows of 89 in every lane);
 // * the mechanism's packed tables (tab/<name>.h, struct Packed) are copied to
 //   LDS once per block; the four waves of a block share them and never wait
 //   for each other afterwards;
@@ -14,26 +17,27 @@
 //   the species' stoichiometric rows are cut into are spread over the lanes
 //   again, and each lane adds up its species' chunks; mixture sums are group
 //   reductions;
-// * Jacobian (rare: about one per cell and call): all 64 lanes of the wave
-//   work on one group's cell at a time, accumulating with FP64 atomics into an
-//   n x n area (LDS when it fits, else the device workspace), then store the
-//   group's rows (molecular-weight scaling of ReactorBDF.cpp:67-82) in LU_T in
-//   the workspace for the Newton-matrix refreshes;
+// * Jacobian (about one per cell and call): all 64 lanes of the wave work on one
+//   group's cell at a time, or each group on its own (group_layout.h),
+//   accumulating with FP64 atomics into an n x n area (LDS when it fits, else the
+//   device workspace), then store the group's rows (molecular-weight scaling of
+//   ReactorBDF.cpp:67-82) in LU_T in the workspace for the Newton-matrix
+//   refreshes;
 // * Newton matrix: inverted in LU_T by row-per-lane Gauss-Jordan exchange
 //   steps with partial pivoting (the pivot row through LDS, rows never move,
 //   the columns rotate through the registers so that the step loop is not
 //   unrolled), so that each Newton iteration's solve is one dot product per
 //   row: no sequential triangular sweeps.
 //
-// What bounds it: the latency of a trip (one right-hand side and one Newton
-// iteration for every group of the wave) at 1 or 2 waves per SIMD: about 27000
-// cycles for drm19 at 32 lanes, a third of them the falloff reactions.  Tables
-// read from device memory by lane and unrolled factorisation steps made it
-// 105000.  Measured (one MI355X, box or 1-D call of 1e-5 s at rtol 1e-10, state
-// restored before each call), against one cell per lane: drm19 64^3 cells 222 ->
-// 70 ms, 2898 cells 95 -> 5.9 ms; dodecane_lu 10000 cells 1558 -> 13.6 ms;
-// heptane_lu_88sk 2048 cells, 1e-6 s at rtol 1e-8, 1169 -> 11.0 ms;
-// LuEthylene_qss 4096 cells 198 -> 7.4 ms.
+// What bounds it: calls that fill the chip, the FP64 vector issue of two waves
+// per SIMD (drm19 64^3 cells at 16 lanes: a vector instruction every 6.3 cycles of
+// a SIMD, of which it takes 4; a wave waits 44% of its cycles, for LDS, spills and
+// dependent results); others, the latency of the longest cells' trips (one
+// right-hand side and one Newton iteration for every group of the wave).  Measured
+// (one MI355X, box or 1-D call of 1e-5 s at rtol 1e-10, state restored before each
+// call), against one cell per lane: drm19 64^3 cells 222 -> 70 ms, 2898 cells 95 ->
+// 5.9 ms; dodecane_lu 10000 cells 1558 -> 13.6 ms; heptane_lu_88sk 2048 cells, 1e-6 s
+// at rtol 1e-8, 1169 -> 11.0 ms; LuEthylene_qss 4096 cells 198 -> 4.2 ms.
 //
 // Every group reduction returns the bitwise-identical value in all lanes of
 // the group (pairs are always added in commuted order on both partners), so
@@ -42,7 +46,8 @@
 // persistent loop evaluates one right-hand side for every group that is not
 // waiting for a factorisation, and the groups' LU requests are served together
 // once enough of them wait.  A cell's arithmetic does not depend on which
-// groups share its wave, so results do not depend on the queue's order.
+// groups share its wave, so results do not depend on the queue's order; it
+// depends on the group's width, which a call's number of cells can choose.
 //
 // The step / order / Newton logic is that of adaptive_cell (reactors.h), the
 // NDF family of SciPy's BDF integrator; every loop over a cell's work is
@@ -679,7 +684,7 @@ struct GroupChem {
   template <int WD, typename JT>
   PPC_DI static void jac_rows(const PK& pk, const double* J, JT* out) {
 #pragma unroll 4
-    for (int t = Grp<WD>::lane(); t < n * n; t += WD) {
+    for (int t = WD == 64 ? (int)__lane_id() : Grp<WD>::lane(); t < n * n; t += WD) {
       const int j = t / n, i = t - j * n;
       out[((i / G) * n + j) * G + i % G] = (JT)jac_elem(pk, J, i, j);
     }
@@ -1254,7 +1259,14 @@ group_bdf_kernel(ReactParamsDev P, IO1D io, double dt, QueueArgs q, CellStats st
           if (valid[e]) wa[e * G + g] = need_jac == 1 ? D[0][e] : ypred[e];
       }
       wave_sync();
-      C::template cell_jacobian<64>(pk, wa, Jw, eform);
+      // (without QSS species not through cell_jacobian, which made heptane_lu_88sk's
+      // registers spill more: 783 -> 820, 10.5 -> 11.0 ms)
+      if constexpr (T::NQ > 0)
+        C::template cell_jacobian<64>(pk, wa, Jw, eform);
+      else if (eform)
+        C::template jacobian<0, 64>(pk, wa, Jw);
+      else
+        C::template jacobian<1, 64>(pk, wa, Jw);
       C::template jac_rows<64>(pk, Jw, rows + s * GSTRIDE);
       __threadfence_block();
       wave_sync();
