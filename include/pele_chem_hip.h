@@ -39,7 +39,7 @@ enum {
   PP_CHEM_BDF_ADAPTIVE_MIXED = 3,  /* batched adaptive BDF: persistent work queue, FP32 Newton-matrix
                                       LU, FP64 residuals, rates and error control */
   PP_CHEM_BDF_BATCHED_FP64 = 4,    /* batched adaptive BDF with an FP64 LU */
-  PP_CHEM_CVODE = 5,               /* "ReactorCvode": the FP64 adaptive BDF (one lane per cell) with
+  PP_CHEM_CVODE = 5,               /* "ReactorCvode": the FP64 adaptive BDF (a group of lanes per cell) with
                                       ReactorCvode's options and defaults (rtol 1e-6, atol 1e-10 x the
                                       typical values, order <= cvode.max_order = 2, ode.max_nls_iters
                                       = 3 Newton iterations, Jacobian age <= 100 steps,
@@ -111,10 +111,11 @@ typedef struct {
   int batched_waves_per_simd;
   /* Batched forms, cells per 64-lane wavefront: 8, 4, 2 or 1 give each cell a
    * group of 8, 16, 32 or 64 lanes that share its equations, reactions and
-   * Newton-matrix rows, so its state stays in registers (table-driven
-   * mechanism kernels only; the values a mechanism supports depend on its
-   * size); 0 (default): the library chooses by the mechanism's size and the
-   * number of cells (the only choice for QSS mechanisms). */
+   * Newton-matrix rows (table-driven mechanism kernels only; the values a
+   * mechanism supports depend on its size); 0 (default): the library chooses by
+   * the mechanism's size and the number of cells (the only choice for QSS
+   * mechanisms), and a mechanism without group kernels runs the adaptive BDF one
+   * cell per lane. */
   int batched_cells_per_wave;
   /* PP_CHEM_BDF_ADAPTIVE and PP_CHEM_CVODE (0 elsewhere): order cap 1..5
    * (cvode.max_order; 0: 5), Newton iterations per step attempt

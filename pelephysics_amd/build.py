@@ -23,13 +23,14 @@ OBJ = os.path.join(HERE, "_build")
 LIBNAME = "libpele_chem_hip.so"
 LIB = os.path.join(HERE, LIBNAME)
 # QSS mechanisms (quasi-steady-state species eliminated in every rate
-# evaluation) are compiled table-driven, one lane per cell
+# evaluation) are compiled table-driven
 MECHS = ["LiDryer", "drm19", "dodecane_lu", "heptane_lu_88sk", "CH4_lean_qss", "LuEthylene_qss",
          "dodecane_lu_qss"]
 MODES = {"bdf": ("MODE", "MODE_BDF"), "rk64": ("MODE", "MODE_RK64"),
          "adaptive": ("MODE", "MODE_ADAPTIVE"), "erk": ("MODE", "MODE_ERK"),
          "bmixed": ("BATCHED", "MODE_BATCHED_MIXED"),
-         "bfp64": ("BATCHED", "MODE_BATCHED_FP64"), "cvode": ("BATCHED", "MODE_GROUP_CVODE"), "gfixed": ("GFIXED", "MODE_BDF"), "adjoint": ("ADJOINT", "MODE_BDF"),
+         "bfp64": ("BATCHED", "MODE_BATCHED_FP64"), "cvode": ("BATCHED", "MODE_GROUP_CVODE"),
+         "gfixed": ("GFIXED", "MODE_BDF"), "adjoint": ("ADJOINT", "MODE_BDF"),
          "flatten": ("FLATTEN", "MODE_BDF")}
 ARCH = "gfx950"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -457,16 +457,18 @@ int gmode(const pp_chem* h) { return h->cfg.mode == PP_CHEM_CVODE ? ppc::MODE_GR
 // (group_fixed.h); 0: one lane per cell.  The one-lane kernels take about the
 // same time for any call up to the 65536 cells that give every SIMD a wave, the
 // group kernels' time grows with the cells once these fill the chip, and their
-// right-hand side spends more instructions per cell, so large calls go to the
-// lane kernels.  Measured (kernel us, one lane / group, drm19 with the box's
-// dt = 1e-6 s): BDF 2048 cells 388 / 59, 32768 795 / 415, 131072 2418 / 1630;
-// RK64 2048 cells 7899 / 2190, 24576 8220 / 7212, 32768 8290 / 9056; LiDryer
-// RK64 8192 cells 910 / 764, 24576 1029 / 1443.  RK64's state is three vectors:
-// the narrowest group that still gives every SIMD two waves; the BDF's group is
-// always 16 lanes.  The smallest mechanisms' BDF stays on one lane: LiDryer's
-// hot cells amplify the last bit of the Jacobian (ReactorBDFsolver.H's residual
-// test below rounding) and the group's order of its sums gives other results
-// there than the reference's order.
+// right-hand side spends more instructions per cell, so RK64's large calls go to
+// the lane kernels.  Measured (kernel us, one lane / group, drm19 with the box's
+// dt = 1e-6 s): RK64 2048 cells 7899 / 2190, 24576 8220 / 7212, 32768 8290 / 9056;
+// LiDryer RK64 8192 cells 910 / 764, 24576 1029 / 1443.  The larger and the QSS
+// mechanisms' calls of up to 96 cells per CU are all faster on groups, so the line
+// holds for them too, though not where it would be for each.  RK64's state is three
+// vectors: the narrowest group that still gives every SIMD two waves.
+// The BDF's group is always 16 lanes, and the faster one at every size (drm19 2048
+// cells 388 / 59, 32768 795 / 415, 131072 2418 / 1630).  The smallest mechanisms' BDF
+// stays on one lane: LiDryer's hot cells amplify the last bit of the Jacobian
+// (ReactorBDFsolver.H's residual test below rounding), more than drm19's, and the
+// group's order of its sums gives other results there than the reference's order.
 int fixed_cells_per_wave(const pp_chem* h, long long ncells) {
   const int mode = h->cfg.mode;
   if (!h->GL || (mode != PP_CHEM_BDF && mode != PP_CHEM_RK64)) return 0;
@@ -491,9 +493,8 @@ int cells_per_wave(const pp_chem* h, long long ncells) {
 // 64-lane blocks of workspace a call of ncells cells can use, and its rows per
 // lane: the Jacobians of the group kernels (group_bdf.h), per wave, and
 // the per-lane matrices of mechanisms too large for private memory
-// (lane_ws.h), for at most the resident waves per CU of the kernel build (4
-// SIMDs x 2 waves, x 1 for the 1-wave build and the one-lane-per-cell kernels
-// of the other integrators) and (by the caller) at most the bytes there are.
+// (lane_ws.h), for at most 8 waves per CU of the group kernels and 4 of the
+// one-lane ones, and (by the caller) at most the bytes there are.
 long long workspace_blocks(const pp_chem* h, long long ncells, int cpw, long long& rows) {
   rows = cpw ? h->GL->group_ws_rows(cpw) : h->L->ws_rows(kmode(h->cfg.mode));
   if (rows == 0 || ncells == 0) return 0;

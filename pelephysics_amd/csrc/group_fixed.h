@@ -92,8 +92,8 @@ struct GroupCell {
 // ------------------------------------------------------------- RK64 --------
 // rk64_core (reactors.h) per group; every trip is one step of all six stages
 // for every group of the wave, and a group that ends its cell takes the next.
-// Bound by the latency of the right-hand sides; the group's state is three
-// vectors, so four waves per SIMD hide it.
+// Bound by the latency of the right-hand sides at two waves per SIMD (170 to 209
+// registers, nothing spilled).
 template <class T, int G, bool BOX>
 __global__ void __launch_bounds__(64 * GROUP_WAVES) __attribute__((amdgpu_waves_per_eu(2, 8)))
 group_rk64_kernel(ReactParamsDev P, GroupIO io, double dt, int ncells, CellStats st) {
@@ -170,10 +170,15 @@ group_rk64_kernel(ReactParamsDev P, GroupIO io, double dt, int ncells, CellStats
 //
 // GMRES stops at an absolute residual of 1e-10 in the equations' CGS units,
 // below the rounding of hot cells' rates, so on such cells the result depends
-// on how the sums round.  Every sum here therefore runs over the same terms in
-// the same order as in the one-lane form: rows of A and the sweeps by
-// construction, the dot products one per lane (lane i takes basis vector i)
-// over vectors in LDS, the norms in every lane.
+// on how the sums round.  GMRES' own sums run over the same terms in the same
+// order as in the one-lane form: rows of A and the sweeps by construction, the dot
+// products one per lane (lane i takes basis vector i) over vectors in LDS, the
+// norms in every lane.  The sums in the matrix and the right-hand side (Jacobian
+// entries, heat and mixture sums, production rates) are the group's; the result on
+// hot cells then lies within the spread of the one-lane form's own roundings
+// (tests/test_gpu_fixed_group.py).
+// One block per compute unit by its LDS (the Krylov bases of 16 cells), i.e. one
+// wave per SIMD on dependent chains.
 template <int J>
 PPC_DI double row_bcast(const double v) {
   return wave::dpp<0x150 + J>(v);

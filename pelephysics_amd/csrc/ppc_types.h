@@ -16,10 +16,10 @@ struct RK64ParamsDev {  // ReactorRK64 ode.* (Source/Reactions/ReactorRK64.H:131
 struct AdaptParamsDev {  // adaptive BDF tolerances
   double rtol, atol, first_step;
   int max_steps;
-  int lu_batch, lu_wait;  // batched forms: wave-shared Jacobian/LU service (0: defaults 64, 32)
-  int lane_occ;           // batched forms: kernel build held to 1 or 2 waves per SIMD (0: 2)
-  int group;              // batched forms: cells per wave of the group kernel (8, 4, 2, 1); 0: one cell per lane
-  // CVODE-style options of the plain FP64 form (0 / null: SciPy's behaviour)
+  int lu_batch, lu_wait;  // group kernels: the wave's LU service (0: half of its groups, as many trips)
+  int lane_occ;           // plain adaptive BDF: kernel build held to 2 or 4 waves per SIMD (0: the compiler's choice)
+  int group;              // cells per wave of the group kernel (8, 4, 2, 1); 0: one cell per lane
+  // CVODE-style options (0 / null: SciPy's behaviour)
   int max_order;          // order cap 1..5 (cvode.max_order)
   int newton_maxiter;     // Newton iterations per attempt (ode.max_nls_iters)
   int jac_age;            // re-evaluate the Jacobian after this many steps

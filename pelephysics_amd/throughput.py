@@ -11,7 +11,7 @@ the initial state, with --chained the calls continue from each other (as a
 flow solver's successive chemistry steps do).  Prints one JSON line: cells/s
 from the kernel time of each call (HIP events around the launch), the
 per-cell work counters (means, and the largest and 99th-percentile step
-count of a cell) and the matrix workspace per resident cell.
+count of a cell) and the matrix workspace per lane.
 """
 from __future__ import annotations
 
@@ -111,7 +111,7 @@ def main(argv=None) -> dict:
         "cells_per_s": st.ncells / (float(np.median(kms)) * 1e-3),
         "cells_per_s_wall": st.ncells * a.calls / wall,
         "kernel_ms": kms, "wall_s": wall, "per_cell": per_call,
-        "workspace_bytes_per_resident_cell": R.workspace_rows() * 8,
+        "workspace_bytes_per_lane": R.workspace_rows() * 8,
         "finite": bool(torch.isfinite(y).all().item()),
     }
     R.close()
