@@ -218,8 +218,9 @@ struct pp_chem {
   // per-cell counters (device), grown on demand
   int cap = 0;
   int* d_cnt = nullptr;  // 6 * cap ints
-  unsigned long long* d_red = nullptr;  // reduce_stats' accumulators, zero between calls
+  unsigned long long* d_red = nullptr;  // reduce_stats' accumulators
   unsigned long long* h_red = nullptr;  // its result (pinned host memory)
+  bool red_clear = false;  // the accumulators are zero: the last sum was handed over
   // work queue of the batched forms: counter, visiting order, cost bins and
   // the identity of the last call (its per-cell costs order the next call)
   int* d_queue = nullptr;  // [0] counter, [1..NBINS] bins, [NBINS+1..2NBINS] offsets
@@ -326,17 +327,13 @@ ppc::CellStats counters(pp_chem* h) {
   return st;
 }
 
-// Clears reduce_stats' accumulators, and waits: the calls run on streams that
-// the null stream does not order.
-hipError_t clear_stats(pp_chem* h) {
-  const hipError_t e = hipMemset(h->d_red, 0, sizeof(unsigned long long) * (NSTAT + 1));
-  return e == hipSuccess ? hipStreamSynchronize(nullptr) : e;
-}
-
 // Reduces the counters st of the call's kernels on stream s, waits for the
 // stream, takes the kernels' time from the events around them and returns
 // int(average steps) or an error.
 int finish(pp_chem* h, int ncells, hipStream_t s, const ppc::CellStats& st) {
+  if (!h->red_clear)  // on the call's own stream, which nothing else orders
+    hipLaunchKernelGGL(zero_ints, dim3(1), dim3(64), 0, s, reinterpret_cast<int*>(h->d_red), 2 * (NSTAT + 1));
+  h->red_clear = false;  // until a result is there
   h->h_red[NSTAT - 1] = NOT_DELIVERED;
   // a block per compute unit: its sums meet the others' on nine words
   const int blocks = std::max(1, std::min(std::max(h->ncu, 1), (ncells + 255) / 256));
@@ -347,10 +344,8 @@ int finish(pp_chem* h, int ncells, hipStream_t s, const ppc::CellStats& st) {
   float kernel_ms = 0.f;
   HIPCHK(h, hipEventElapsedTime(&kernel_ms, h->ev0, h->ev1));
   const unsigned long long* r = h->h_red;
-  if (r[NSTAT - 1] == NOT_DELIVERED) {
-    HIPCHK(h, clear_stats(h));
-    return fail(h, PP_CHEM_EHIP, "the call's statistics were not delivered");
-  }
+  if (r[NSTAT - 1] == NOT_DELIVERED) return fail(h, PP_CHEM_EHIP, "the call's statistics were not delivered");
+  h->red_clear = true;
   pp_chem_stats& S = h->stats;
   S.ncells = ncells;
   S.nsteps = (long long)r[0];
@@ -830,7 +825,6 @@ int pp_chem_create(const pp_chem_config* cfg, pp_chem** out) {
   // one allocation: the accumulators, the queue and the failure count
   constexpr size_t red_bytes = sizeof(unsigned long long) * (NSTAT + 1), queue_ints = 1 + 2 * NBINS;
   if (e == hipSuccess) e = hipMalloc(&h->d_red, red_bytes + sizeof(int) * (queue_ints + 1));
-  if (e == hipSuccess) e = clear_stats(h);
   if (e == hipSuccess) {
     h->d_queue = reinterpret_cast<int*>(h->d_red + NSTAT + 1);
     h->d_fail = h->d_queue + queue_ints;

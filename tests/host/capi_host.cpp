@@ -6,7 +6,8 @@
 //
 // Device memory is host memory from a pool in which a freed block is the next
 // one handed out (oldest first), as a device allocator may do.  Kernels do not
-// run; reduce_stats hands over a preset result unless `deliver` is off.
+// run but for zero_ints; reduce_stats hands over a preset result unless `deliver`
+// is off.
 #include "../../pelephysics_amd/csrc/capi.hip"
 
 #include <deque>
@@ -20,7 +21,7 @@ int captures = 0, replays = 0;
 bool deliver = true;
 unsigned long long result[NSTAT] = {};
 const void *acc = nullptr;           // reduce_stats' accumulators of the last call
-bool memset_pending = false;         // a hipMemset nothing has waited for
+bool acc_clear = false;              // and whether they were zero then
 char symbol[1024];                   // the device scratch's address (never dereferenced)
 // last integrator launch
 std::string launched;
@@ -93,11 +94,12 @@ hipError_t hipMalloc(void** p, size_t n) {
   if (fake::malloc_fails_in >= 0 && fake::malloc_fails_in-- == 0) return hipErrorOutOfMemory;
   if (n > fake::BLOCK) return hipErrorOutOfMemory;
   if (fake::freed.empty()) {
-    *p = std::calloc(1, fake::BLOCK);
+    *p = std::malloc(fake::BLOCK);
   } else {
     *p = fake::freed.front();
     fake::freed.pop_front();
   }
+  std::memset(*p, 0xab, fake::BLOCK);
   return hipSuccess;
 }
 hipError_t hipFree(void* p) {
@@ -106,18 +108,9 @@ hipError_t hipFree(void* p) {
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return (*p = std::calloc(1, n)) ? hipSuccess : hipErrorOutOfMemory; }
 hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
-hipError_t hipMemset(void* p, int v, size_t n) {
-  std::memset(p, v, n);
-  fake::memset_pending = true;
-  return hipSuccess;
-}
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { std::memcpy(d, s, n); return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t s) {
-  if (!s) fake::memset_pending = false;
-  return hipSuccess;
-}
-hipError_t hipDeviceSynchronize() { fake::memset_pending = false; return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 2; return hipSuccess; }
@@ -148,10 +141,15 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* m, hipStream_t* s
 }
 hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t) {
   if (f == (const void*)&reduce_stats) {
-    fake::acc = *(const void**)args[7];
+    const unsigned long long* acc = *(unsigned long long**)args[7];
+    fake::acc = acc;
+    fake::acc_clear = true;
+    for (int i = 0; i <= NSTAT; ++i) fake::acc_clear = fake::acc_clear && acc[i] == 0;
     unsigned long long* host = *(unsigned long long**)args[8];
     if (fake::deliver)
       for (int i = 0; i < NSTAT; ++i) host[i] = fake::result[i];
+  } else if (f == (const void*)&zero_ints) {
+    std::memset(*(int**)args[0], 0, sizeof(int) * (size_t)(*(int*)args[1]));
   }
   return hipSuccess;
 }
@@ -199,17 +197,13 @@ int call_box(pp_chem* h, int n) {
 // a call's statistics do not arrive: an error, and the next call is sound again
 void undelivered() {
   pp_chem* h = handle("drm19", PP_CHEM_RK64);
-  std::printf("memset_pending_after_create %d\n", (int)fake::memset_pending);
   fake::result[0] = 800;  // 8 steps a cell
-  std::printf("first %d\n", call_1d(h, 100));
+  std::printf("first %d\nclear_at_first %d\n", call_1d(h, 100), (int)fake::acc_clear);
   fake::deliver = false;
   h->d_red[0] = 5, h->d_red[NSTAT] = 3;  // what such a call leaves behind
   std::printf("undelivered %d\n", call_1d(h, 100));
   fake::deliver = true;
-  bool clear = true;
-  for (int i = 0; i <= NSTAT; ++i) clear = clear && h->d_red[i] == 0;
-  std::printf("accumulators_clear %d\n", (int)clear);
-  std::printf("next %d\n", call_1d(h, 100));
+  std::printf("next %d\nclear_at_next %d\n", call_1d(h, 100), (int)fake::acc_clear);
 }
 
 // two handles' calls without allocation share no accumulators

@@ -39,13 +39,13 @@ def host(tmp_path_factory):
 def test_undelivered_statistics_are_an_error(host):
     """The kernel that sums up a call hands its result to host memory.  A call
     whose result does not arrive must not return an earlier call's, and must
-    leave nothing behind that spoils the next."""
+    leave nothing behind that spoils the next; the accumulators, which are not
+    zero when they are allocated, are cleared on the call's own stream."""
     s = host("undelivered")
-    assert s["create"] == 0 and s["memset_pending_after_create"] == 0
-    assert s["first"] == 8
+    assert s["create"] == 0
+    assert s["first"] == 8 and s["clear_at_first"] == 1
     assert s["undelivered"] == -3  # EHIP
-    assert s["accumulators_clear"] == 1
-    assert s["next"] == 8
+    assert s["next"] == 8 and s["clear_at_next"] == 1
 
 
 def test_noalloc_calls_share_no_accumulators(host):
