@@ -681,9 +681,12 @@ struct GroupChem {
     return v;
   }
   // all of them by WD lanes, element (i, j) at out[(e*n + j)*G + g] for i = e*G + g
+  // (unrolled four times it made the FP64 dodecane_lu_qss kernel spill 714 registers
+  // in place of 463, ReactorCvode calls of 64 cells 3.1 -> 4.2 ms)
   template <int WD, typename JT>
   PPC_DI static void jac_rows(const PK& pk, const double* J, JT* out) {
-#pragma unroll 4
+    constexpr int U = NQ > 0 && !JLDS ? 2 : 4;
+#pragma unroll U
     for (int t = WD == 64 ? (int)__lane_id() : Grp<WD>::lane(); t < n * n; t += WD) {
       const int j = t / n, i = t - j * n;
       out[((i / G) * n + j) * G + i % G] = (JT)jac_elem(pk, J, i, j);
@@ -792,8 +795,10 @@ __device__ __noinline__ void group_qss_jacobian(lds_double* area, double* Jws, c
   const double mixture = Gr::sum(msum);
   jsync();
   const double* const x = c + NS;
+  // (both from the last reaction down: the unlike kinds, which the tables have
+  // last, share the first round)
 #pragma unroll 1
-  for (int i = g; i < T::NQR; i += WD) {
+  for (int i = T::NQR - 1 - g; i >= 0; i -= WD) {
     double qf, qr;
     TabMech<T>::qss_balance_terms(i, c1, a, b1, x, mixture, Tv, invT, logT, refC, refCinv, qf, qr,
                                   [&](int idx, double v) { add(X + idx, v); });
@@ -817,7 +822,7 @@ __device__ __noinline__ void group_qss_jacobian(lds_double* area, double* Jws, c
     }
   }
 #pragma unroll 1
-  for (int j = g; j < T::NR; j += WD)
+  for (int j = T::NR - 1 - g; j >= 0; j -= WD)
     TM::template jac_reaction<0>(
         j, c, gk, hh, mixture, Tv, invT, invT2, logT, refC, refCinv,
         [&](int idx, double v) {
@@ -838,13 +843,14 @@ __device__ __noinline__ void group_qss_jacobian(lds_double* area, double* Jws, c
     for (int i = 0; i < NQ; ++i) st(X + i * NS + k, col[i]);
   }
   jsync();
-  // J += (d wdot / d x)(d x / d c)
+  // J += (d wdot / d x)(d x / d c); plain loads, which the fence has ordered after
+  // the sums, and which the lanes of one round share in the cache
 #pragma unroll 1
   for (int t = g; t < NS * NS; t += WD) {
     const int k = t / NS, m = t - k * NS;
-    double d = ld(J + k * n + m);
-#pragma unroll 5
-    for (int i = 0; i < NQ; ++i) d += ld(W + i * NS + m) * ld(X + i * NS + k);
+    double d = J[k * n + m];
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) d += W[i * NS + m] * X[i * NS + k];
     st(J + k * n + m, d);
   }
   jsync();
