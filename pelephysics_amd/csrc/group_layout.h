@@ -58,8 +58,8 @@ struct GroupLayout {
   // Without QSS species a group's own takes NR / G rounds of reactions, the wave NG
   // times NR / 64: its own where that is at most half.  Measured, calls of one step
   // per cell: LiDryer 262144 cells, 8 lanes, one cell after the other 5.7 ms, each
-  // its own 1.6; CH4_lean_qss 262144 cells and LuEthylene_qss 65536, by the group in
-  // the workspace 34.3 and 37.6 ms, in LDS by the group and by the wave 5.4 and 6.3.
+  // its own 1.3; CH4_lean_qss 262144 cells and LuEthylene_qss 65536, by the group in
+  // the workspace 34.3 and 37.6 ms, in LDS by the group and by the wave 5.2 and 5.9.
   static constexpr bool two_blocks(int area) { return bytes(area) <= LDS_BYTES / 2; }
   static constexpr bool own_fits() { return n <= 32 && two_blocks(NG * own_area()); }
   static constexpr bool wave_fits() { return n <= 32 && (NQ == 0 || two_blocks(wave_area())); }
